@@ -538,14 +538,13 @@ dbd_status plan(dbd_ctx* c) {
   CHK(c->blk.ensure(8 * (size_t)(std::max(c->nb, (int64_t)kMaxCats) + 2)));
   CHK(c->err.ensure(64));  // error word, then a sink the numeric kernels write degenerate rows to
   CHK(c->bdesc_s.ensure(8 * (size_t)(c->A.nnz + 1)));
-  CHK(c->bdesc_l.ensure(4 * (size_t)(c->A.nnz + 1)));
+  // the lengths, then the row analysis' tile table
+  CHK(c->bdesc_l.ensure(4 * (size_t)(c->A.nnz + 1 + row_tiles(c->A.nnz) + 1)));
   c->A.bstart = c->bdesc_s.as<int64_t>();
   c->A.blen = c->bdesc_l.as<int32_t>();
   if (c->same) c->B = c->A;
-  launch_fill_i32(c->err.as<int32_t>(), 1, 0, s);
-
   launch_row_products(c->A, c->B, c->P.as<int64_t>(), c->nnz.as<int64_t>(), (int64_t*)c->A.bstart,
-                      (int32_t*)c->A.blen, s);
+                      (int32_t*)c->A.blen, c->bdesc_l.as<int32_t>() + c->A.nnz + 1, c->err.as<int>(), s);
   launch_exclusive_scan(c->P.as<int64_t>(), c->Pptr.as<int64_t>(), nr, c->tmp.as<int64_t>(), s);
   launch_gather_strided(c->Pptr.as<int64_t>(), nr, BR, c->nb, c->blk.as<int64_t>(), s);
   c->h_blk.assign((size_t)c->nb + 1, 0);
@@ -1321,8 +1320,8 @@ void dbd::enqueue_pipeline(const Work& w, const Tables& tb, Mat A, const Mat& B,
   const int64_t nr = w.nr;
   A.bstart = w.bstart;
   A.blen = w.blen;
-  launch_fill_i32(w.err, 1, 0, s);
-  launch_row_products(A, B, w.P, w.nnz, w.bstart, w.blen, s);
+  // the analysis' tile table lies in the cursors, which the row kernels only write later
+  launch_row_products(A, B, w.P, w.nnz, w.bstart, w.blen, (int32_t*)w.cursor, w.err, s);
   const CatTable& ct = tb.sym_ct;
   launch_bin_count(w.P, nr, B.ncols, ct, w.cnt, s);
   launch_exclusive_scan(w.cnt, w.offs_sym, (int64_t)ct.n * w.nwg, w.tmp, s);

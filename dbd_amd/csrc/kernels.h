@@ -86,10 +86,11 @@ void launch_band_index(const int32_t* slot_row, int64_t nslots, const int64_t* B
                        int32_t* band, hipStream_t s);
 
 // ---- planning ----
-// P[i] = sum_{k in A_i} len(B_k); nnz[i] = 0 where P[i] == 0; per A nonzero j with column k:
-// bstart[j] = B.ptr[k], blen[j] = len(B_k) (both nullable).
+// P[i] = sum_{k in A_i} len(B_k), nnz[i] = 0 and *err = 0; per A nonzero j with column k:
+// bstart[j] = B.ptr[k], blen[j] = len(B_k). tile_row: scratch of row_tiles(nnz(A)) + 1 entries.
+int64_t row_tiles(int64_t nnz);
 void launch_row_products(const Mat& A, const Mat& B, int64_t* P, int64_t* nnz, int64_t* bstart, int32_t* blen,
-                         hipStream_t s);
+                         int32_t* tile_row, int* err, hipStream_t s);
 // Stable counting sort of rows [0, n) by category of min(key[i], cap).
 // counts/offs have ncat * nwg (+1) int64 where nwg = bin_tiles(n).
 int64_t bin_tiles(int64_t n);

@@ -1,0 +1,59 @@
+"""The pipeline's kernels at the sizes where they can go wrong, against the oracle: edges of tiles,
+remainders, the smallest and largest of a branch's range. Structure exact; values within the
+bound of any summation order (helpers.compare)."""
+import numpy as np
+import pytest
+
+import dbd_amd
+import oracle
+from helpers import check_product, compare, reference
+
+pytestmark = pytest.mark.gpu
+
+
+def from_lengths(lens, ncols, seed, dtype=np.float64):
+    """CSR with the given row lengths, distinct random columns, normal values."""
+    rng = np.random.default_rng(seed)
+    lens = np.asarray(lens, np.int64)
+    ptr = np.concatenate([[0], np.cumsum(lens)])
+    idx = np.concatenate([np.sort(rng.choice(ncols, int(n), replace=False)) for n in lens if n] or [np.zeros(0)])
+    return dbd_amd.CSR(ptr, idx.astype(np.int32), rng.standard_normal(int(ptr[-1])).astype(dtype), (len(lens), ncols))
+
+
+# row analysis: rows that end at, before and after the edges of the 2048-nonzero tiles, rows over
+# several tiles, and tiles over thousands of empty rows (the bisecting branch)
+@pytest.mark.parametrize("lens", [
+    [1], [2047], [2048], [2049, 1], [2048] * 3, [1] * 2048 + [5], [2047, 2, 2047, 0, 4096],
+    [3] + [0] * 5000 + [7, 0, 2100] + [0] * 9000, [0] * 4095 + [1], [1] + [0] * 4100 + [1] * 20 + [0] * 4200 + [4500, 3],
+], ids=lambda v: f"{len(v)}rows{sum(v)}nnz")
+def test_row_analysis_tiles(gpu_ok, lens):
+    B = from_lengths(np.random.default_rng(5).integers(0, 9, 6000), 700, 6)
+    A = from_lengths(lens, 6000, 7)
+    with dbd_amd.Context() as ctx:
+        ctx.set_operands(A, B)
+        info = ctx.plan()
+        P = oracle.row_products(A.ptr, A.idx, B.ptr)
+        assert np.array_equal(ctx.row_products(A.shape[0]), P) and info["products"] == P.sum()
+    check_product(A, B)
+
+
+def test_device_view_of_a_run_of_rows(gpu_ok):
+    """A device view may be rows [r0, r1) of a larger matrix: its row pointer starts past 0 and ends
+    before the index array does."""
+    import torch
+    M = from_lengths(np.random.default_rng(8).integers(0, 40, 900), 500, 9)
+    B = dbd_amd.gen_er(500, 800, 6, seed=10)
+    r0, r1 = 211, 640
+    dM, dB = dbd_amd.DeviceCSR.from_host(M), dbd_amd.DeviceCSR.from_host(B)
+    V = dbd_amd.DeviceCSR(dM.ptr[r0:r1 + 1].clone(), dM.idx, dM.val, (r1 - r0, 500))
+    with dbd_amd.Context(stream=torch.cuda.current_stream()) as ctx:
+        ctx.set_operands(V, dB)
+        ctx.plan()
+        p = torch.empty(r1 - r0 + 1, dtype=torch.int64, device="cuda")
+        n = ctx.symbolic(p)
+        i, v = torch.empty(n, dtype=torch.int32, device="cuda"), torch.empty(n, dtype=torch.float64, device="cuda")
+        ctx.numeric(p, i, v)
+        C = dbd_amd.CSR(p.cpu().numpy(), i.cpu().numpy(), v.cpu().numpy(), (r1 - r0, 800))
+    e0, e1 = int(M.ptr[r0]), int(M.ptr[r1])
+    S = dbd_amd.CSR(M.ptr[r0:r1 + 1] - e0, M.idx[e0:e1], M.val[e0:e1], (r1 - r0, 500))
+    compare(C, reference(S, B), np.float64, "rows of a larger matrix")
