@@ -125,7 +125,7 @@ Tables dbd::default_tables(int g_small, int g_big, double load, int top, int64_t
   }
   t.num_ct.lim[n] = INT64_MAX;
   t.num_k[n++] = {0, 256, 16};  // long rows
-  t.num_ct.lim[n] = INT64_MAX;  // hub rows: long rows of more than kHubEntries A entries
+  t.num_ct.lim[n] = INT64_MAX;  // hub rows: the long rows hub_row picks
   t.num_k[n++] = {kHubShape, 1024, 0};
   t.num_ct.n = n;
   return t;
@@ -315,13 +315,12 @@ struct dbd_ctx {
   // band index of B's long rows (for the long-row window kernels), built once per operand set
   DevBuf band_hist, band_flag, band_tmp, band_slot, band_row, band;
   bool band_ready = false;
-  // workspace of the hub-row range kernels: banded-entry lists (per A nonzero), per-row counts,
-  // per-(row, range) short-product counts and column counts with their scans, short products
-  DevBuf hub_list, hub_cnt, hub_scnt, hub_rcnt, hub_tmp, hub_scol, hub_sval;
-  // hub slots of the symbolic long rows of more than kHubEntries entries (per row, -1: none) and
-  // their column counts per hub range, written by the symbolic long kernel
-  DevBuf hub_slot, hub_flag, hub_rng;
-  int64_t hub_n = 0;
+  // hub rows: slots (per row, -1: none), the scanned flags they come from, lists and counters
+  // (hub_meta), columns per (slot, range); per chunk the short-product and column counts per (row,
+  // range) with their scans, and the short products' buckets
+  DevBuf hub_slot, hub_flag, hub_meta, hub_rng, hub_scnt, hub_rcnt, hub_tmp, hub_scol, hub_sval;
+  HubWork hub;
+  bool hub_split = false;  // the entry records (in `cursor`) are those of the current plan
   int64_t band_minlen = 0, band_rows = 0, band_nb1 = 0;
   std::vector<int64_t> h_blk, h_blockP, h_blockC, h_offs_num, h_sym_tot;
   dbd_plan_info info{};
@@ -359,11 +358,13 @@ dbd_status ensure_events(dbd_ctx* c) {
   return DBD_OK;
 }
 
-dbd_status check_err(dbd_ctx* c, const char* phase) {
-  int e = 0;
-  HIPCHK(hipMemcpyAsync(&e, c->err.p, sizeof(int), hipMemcpyDeviceToHost, c->st));
+// `many`: the number of hub rows of many entries, which lies beside the error word.
+dbd_status check_err(dbd_ctx* c, const char* phase, int* many = nullptr) {
+  int e[2] = {0, 0};
+  HIPCHK(hipMemcpyAsync(e, c->err.p, sizeof(e), hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
-  if (e != 0) return set_error(DBD_ERR_INTERNAL, "%s: device consistency check failed (flags 0x%x)", phase, e);
+  if (many) *many = e[1];
+  if (e[0] != 0) return set_error(DBD_ERR_INTERNAL, "%s: device consistency check failed (flags 0x%x)", phase, e[0]);
   return DBD_OK;
 }
 
@@ -371,12 +372,16 @@ dbd_status check_err(dbd_ctx* c, const char* phase) {
 // keep one counter per column range in LDS.
 bool hub_ranges_ok(const dbd_ctx* c) { return c->B.band != nullptr && hub_ranges(c->B.ncols) <= kHubMaxRanges; }
 
-// Hub slots (after the symbolic binning and the band index): the symbolic long rows of more than
-// kHubEntries A entries, when the table sends hub rows to the range kernels for this width. The
-// symbolic long kernel then records their column counts per range, and the numeric binning puts
-// the ones that stay long into the hub category.
+// Hub slots (after the symbolic binning and the band index): the symbolic long rows that hub_row
+// picks, when the table sends hub rows to the range kernels for this width. The symbolic pass then
+// counts their columns per range, and the numeric binning puts the ones that stay long into the hub
+// category. Should the rule by products pick more (row, range) pairs than kHubMaxItems (1 GiB of
+// counts), only the rows of many entries take slots.
+constexpr int64_t kHubMaxItems = (int64_t)1 << 28;
+
 dbd_status assign_hub_slots(dbd_ctx* c) {
-  c->hub_n = 0;
+  c->hub = HubWork{};
+  c->hub_split = false;
   const CatTable& ct = c->tb.sym_ct;
   const int64_t p0 = c->h_sym_tot[(size_t)ct.n - 1], nlong = c->h_sym_tot[(size_t)ct.n] - p0;
   if (nlong <= 0 || !hub_enabled(c->tb, c->B.ncols) || !hub_ranges_ok(c)) return DBD_OK;
@@ -384,47 +389,81 @@ dbd_status assign_hub_slots(dbd_ctx* c) {
   const int nrng = hub_ranges(c->B.ncols);
   const int32_t* rows = c->rows_sym.as<int32_t>() + p0;
   CHK(c->hub_slot.ensure(4 * (size_t)c->nr));
-  CHK(c->hub_flag.ensure(16 * (size_t)(nlong + 1)));
+  CHK(c->hub_flag.ensure(8 * (size_t)(2 * nlong + 2)));
   CHK(c->hub_tmp.ensure(8 * (size_t)scan_tmp_elems(nlong + 1)));
   int64_t* flag = c->hub_flag.as<int64_t>();
   int64_t* pos = flag + nlong + 1;
-  launch_fill_i32(c->hub_slot.as<int32_t>(), c->nr, -1, s);
-  launch_hub_flags(rows, nlong, c->A.ptr, flag, s);
-  launch_exclusive_scan(flag, pos, nlong, c->hub_tmp.as<int64_t>(), s);
-  int64_t n = 0;
-  HIPCHK(hipMemcpyAsync(&n, pos + nlong, 8, hipMemcpyDeviceToHost, s));
-  HIPCHK(hipStreamSynchronize(s));
-  if (n <= 0 || n * (int64_t)nrng >= INT32_MAX) return DBD_OK;  // none, or too many to count per range
-  launch_hub_slots(rows, nlong, flag, pos, c->hub_slot.as<int32_t>(), s);
+  int64_t n = 0, nfine = 0;
+  for (int64_t per_range : {kHubPerRange, (int64_t)INT64_MAX}) {
+    launch_hub_flags(rows, nlong, c->A, c->B, c->P.as<int64_t>(), per_range, hub_wide(c->B.ncols, nlong), c->info.products, flag, s);
+    launch_exclusive_scan(flag, pos, nlong, c->hub_tmp.as<int64_t>(), s);
+    int64_t got = 0;
+    HIPCHK(hipMemcpyAsync(&got, pos + nlong, sizeof(got), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    n = got & (kHubFineOne - 1);
+    nfine = got >> kHubFineShift;
+    if (n == 0) return DBD_OK;
+    if (n * nrng <= kHubMaxItems) break;
+  }
+  if (n * nrng >= INT32_MAX || n > kHubSlotMask) return DBD_OK;  // too many to count per range
+  const int64_t n4 = (n + 3) & ~(int64_t)3;
+  CHK(c->hub_meta.ensure(8 * (size_t)(2 * (n + 1)) + 4 * (size_t)(6 * n4)));
   CHK(c->hub_rng.ensure(4 * (size_t)(n * nrng)));
-  launch_fill_i32(c->hub_rng.as<int32_t>(), n * nrng, 0, s);
-  c->hub_n = n;
+  CHK(c->hub_tmp.ensure(8 * (size_t)scan_tmp_elems(n + 1)));
+  HubWork& h = c->hub;
+  h.n = n;
+  h.nfine = nfine;
+  h.wide = hub_wide(c->B.ncols, nlong);
+  h.slot = c->hub_slot.as<int32_t>();
+  h.coff = c->hub_meta.as<int64_t>();
+  h.boff = h.coff + n + 1;
+  h.rows = (int32_t*)(h.boff + n + 1);
+  h.fine = h.rows + n4;
+  h.hcnt = h.fine + n4;
+  h.lcnt = h.hcnt + n4;
+  h.span = h.lcnt + n4;
+  h.rng_cnt = c->hub_rng.as<int32_t>();
+  h.tmp = c->hub_tmp.as<int64_t>();
+  launch_fill_i32(h.slot, c->nr, -1, s);
+  launch_hub_slots(rows, nlong, c->A, flag, pos, h, s);
   return DBD_OK;
 }
 
-// Hub rows rows_num[pos0, pos0 + n) of a chunk in column ranges: banded-entry lists and bucketed
-// short products, the symbolic pass's (row, range) column counts scanned into output offsets, the
-// numeric pass. hub_reserve sizes the workspace for n rows; hub_head lists the banded entries and
-// scans the short products' counts per (row, range); hub_tail fills the buckets (at most
-// `short_cap` products, else the capacity bit is set and nothing is written) and runs the ranges.
+// The hub rows' entry records lie in the cursor workspace; backward's cursors overwrite them.
+void hub_split(dbd_ctx* c, hipStream_t s) {
+  const CatTable& ct = c->tb.sym_ct;
+  c->hub.recs = c->cursor.p;
+  launch_hub_split(c->hub, c->A, c->B, c->P.as<int64_t>(), ct.n > 1 ? ct.lim[ct.n - 2] : 0, c->nnz.as<int64_t>(),
+                   c->err.as<int>() + 1, s);
+}
+
+void hub_symbolic(dbd_ctx* c, hipStream_t s) {
+  hub_split(c, s);
+  launch_hub_count(c->hub, c->A, c->B, c->nnz.as<int64_t>(), s);
+}
+
+// Hub rows rows_num[pos0, pos0 + n) of a chunk in column ranges: bucketed short products, the
+// symbolic pass's (row, range) column counts scanned into output offsets, the numeric pass.
+// hub_reserve sizes the workspace for n rows; hub_head scans the short products' counts per (row,
+// range); hub_tail fills the buckets (at most `short_cap` products, else the capacity bit is set and
+// nothing is written) and runs the ranges.
 dbd_status hub_reserve(dbd_ctx* c, int64_t n) {
   const int64_t items = n * hub_ranges(c->B.ncols);
-  CHK(c->hub_list.ensure(4 * (size_t)std::max<int64_t>(c->A.nnz, 1)));
-  CHK(c->hub_cnt.ensure(4 * (size_t)n));
-  CHK(c->hub_scnt.ensure(16 * (size_t)(items + 1)));  // counts, then their scan
-  CHK(c->hub_rcnt.ensure(16 * (size_t)(items + 1)));
+  if (hub_buckets_used(c->B.ncols)) CHK(c->hub_scnt.ensure(16 * (size_t)(items + 1)));  // counts, then their scan
+  CHK(c->hub_rcnt.ensure(16 * (size_t)(items + 1) + kHubRowBytes * (size_t)(n + 1)));  // counts, scan, rows
+  c->hub.info = (void*)(((uintptr_t)(c->hub_rcnt.as<int64_t>() + 2 * (items + 1)) + 31) & ~(uintptr_t)31);
   CHK(c->hub_tmp.ensure(8 * (size_t)scan_tmp_elems(items + 1)));
+  c->hub.tmp = c->hub_tmp.as<int64_t>();
   return DBD_OK;
 }
 
 // The number of short products lands at hub_scnt[2 * items + 1] (the end of their scan).
 void hub_head(dbd_ctx* c, int64_t pos0, int64_t n, hipStream_t s) {
-  const int nrng = hub_ranges(c->B.ncols);
-  const int64_t items = n * nrng;
+  if (!hub_buckets_used(c->B.ncols)) return;
+  const int64_t items = n * hub_ranges(c->B.ncols);
   int64_t* scnt = c->hub_scnt.as<int64_t>();
-  launch_hub_prepare(c->rows_num.as<int32_t>() + pos0, n, c->A, c->B, nrng, scnt, c->hub_list.as<int32_t>(),
-                     c->hub_cnt.as<int32_t>(), s);
-  launch_exclusive_scan(scnt, scnt + items + 1, items, c->hub_tmp.as<int64_t>(), s);
+  launch_hub_bucket_count(c->hub, c->rows_num.as<int32_t>() + pos0, n, c->A, c->B, scnt, s);
+  launch_exclusive_scan(scnt, scnt + items + 1, items, c->hub.tmp, s);
 }
 
 void hub_tail(dbd_ctx* c, int64_t pos0, int64_t n, int64_t short_cap, const int64_t* Cptr, int64_t cbase,
@@ -432,22 +471,28 @@ void hub_tail(dbd_ctx* c, int64_t pos0, int64_t n, int64_t short_cap, const int6
   const int nrng = hub_ranges(c->B.ncols);
   const int64_t items = n * nrng;
   const int32_t* rows = c->rows_num.as<int32_t>() + pos0;
-  const int64_t* soff = c->hub_scnt.as<int64_t>() + items + 1;
   int64_t* rcnt = c->hub_rcnt.as<int64_t>();
   int64_t* roff = rcnt + items + 1;
   int* err = c->err.as<int>();
-  launch_hub_guard(soff + items, short_cap, err, s);
-  launch_hub_scatter(c->o.dtype, rows, n, c->A, c->B, nrng, soff, c->hub_scol.as<int32_t>(), c->hub_sval.p, err, s);
-  launch_hub_gather_counts(rows, n, nrng, c->hub_slot.as<int32_t>(), c->hub_rng.as<int32_t>(), rcnt, s);
-  launch_exclusive_scan(rcnt, roff, items, c->hub_tmp.as<int64_t>(), s);
-  launch_hub_range(c->o.dtype, rows, n, nrng, c->A, c->B, c->hub_list.as<int32_t>(), c->hub_cnt.as<int32_t>(), soff,
-                   c->hub_scol.as<int32_t>(), c->hub_sval.p, roff, Cptr, cbase, Cidx, Cval, err, s);
+  const int64_t* soff = nullptr;
+  if (hub_buckets_used(c->B.ncols)) {
+    int64_t* scnt = c->hub_scnt.as<int64_t>();
+    soff = scnt + items + 1;
+    launch_hub_guard(soff + items, short_cap, err, s);
+    launch_hub_bucket_fill(c->o.dtype, c->hub, rows, n, c->A, c->B, scnt, soff, c->hub_scol.as<int32_t>(),
+                           c->hub_sval.p, err, s);
+  }
+  launch_hub_gather_counts(c->hub, rows, n, c->A, c->B, Cptr, cbase, rcnt, s);
+  launch_exclusive_scan(rcnt, roff, items, c->hub.tmp, s);
+  launch_hub_range(c->o.dtype, c->hub, n, c->A, c->B, soff, c->hub_scol.as<int32_t>(), c->hub_sval.p, roff, Cidx, Cval,
+                   err, s);
 }
 
 // Sizes the buckets: one host synchronisation for the number of short products.
 dbd_status hub_buckets(dbd_ctx* c, int64_t n, int64_t* nshort) {
-  const int64_t items = n * hub_ranges(c->B.ncols);
   *nshort = 0;
+  if (!hub_buckets_used(c->B.ncols)) return DBD_OK;
+  const int64_t items = n * hub_ranges(c->B.ncols);
   HIPCHK(hipMemcpyAsync(nshort, c->hub_scnt.as<int64_t>() + 2 * items + 1, 8, hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
   CHK(c->hub_scol.ensure(4 * (size_t)std::max<int64_t>(*nshort, 1)));
@@ -458,6 +503,10 @@ dbd_status hub_buckets(dbd_ctx* c, int64_t n, int64_t* nshort) {
 dbd_status hub_numeric(dbd_ctx* c, int64_t pos0, int64_t n, const int64_t* Cptr, int64_t cbase, int32_t* Cidx,
                        void* Cval) {
   CHK(hub_reserve(c, n));
+  if (!c->hub_split) {
+    hub_split(c, c->st);
+    c->hub_split = true;
+  }
   hub_head(c, pos0, n, c->st);
   int64_t nshort = 0;
   CHK(hub_buckets(c, n, &nshort));
@@ -600,15 +649,21 @@ dbd_status symbolic(dbd_ctx* c) {
   hipStream_t s = c->st;
   const CatTable& ct = c->tb.sym_ct;
   const int64_t* offs = c->offs_sym.as<int64_t>();
+  if (c->hub.n > 0) {
+    CHK(ensure_cursor(c));
+    hub_symbolic(c, s);
+    c->hub_split = true;
+  }
   for (int k = 1; k < ct.n; ++k) {
     const int64_t n = c->h_sym_tot[(size_t)k + 1] - c->h_sym_tot[(size_t)k];
     if (n <= 0) continue;
-    if (c->tb.sym_k[k].T == 0) CHK(ensure_cursor(c));
-    const bool hubs = c->hub_n > 0;
+    if (c->tb.sym_k[k].T == 0) {
+      if (n == c->hub.n) continue;  // every long row is a hub row
+      CHK(ensure_cursor(c));
+    }
     launch_symbolic(c->tb.sym_k[k], c->rows_sym.as<int32_t>(), offs + (int64_t)k * c->nwg,
                     offs + (int64_t)(k + 1) * c->nwg, n, 0, c->A, c->B, c->nnz.as<int64_t>(),
-                    c->cursor.as<int64_t>(), c->err.as<int>(), s, hubs ? c->hub_slot.as<int32_t>() : nullptr,
-                    hubs ? c->hub_rng.as<int32_t>() : nullptr, hubs ? hub_ranges(c->B.ncols) : 0);
+                    c->cursor.as<int64_t>(), c->err.as<int>(), s, c->hub.slot);
   }
   launch_exclusive_scan(c->nnz.as<int64_t>(), c->Cptr.as<int64_t>(), c->nr, c->tmp.as<int64_t>(), s);
   const int BR = c->o.block_rows;
@@ -618,19 +673,25 @@ dbd_status symbolic(dbd_ctx* c) {
   // numeric bins by exact nnz_i
   const CatTable& nt = c->tb.num_ct;
   const int64_t n_off = (int64_t)nt.n * c->nwg;
-  const int32_t* hub_rows = c->hub_n > 0 ? c->hub_slot.as<int32_t>() : nullptr;
-  launch_bin_count(c->nnz.as<int64_t>(), c->nr, INT64_MAX, nt, c->cnt.as<int64_t>(), s, hub_rows);
+  launch_bin_count(c->nnz.as<int64_t>(), c->nr, INT64_MAX, nt, c->cnt.as<int64_t>(), s, c->hub.slot,
+                   c->err.as<int>() + 1);
   launch_exclusive_scan(c->cnt.as<int64_t>(), c->offs_num.as<int64_t>(), n_off, c->tmp.as<int64_t>(), s);
   launch_bin_scatter(c->nnz.as<int64_t>(), c->nr, INT64_MAX, nt, c->offs_num.as<int64_t>(), c->rows_num.as<int32_t>(),
-                     s, hub_rows);
+                     s, c->hub.slot);
   c->h_offs_num.assign((size_t)n_off + 1, 0);
   HIPCHK(hipMemcpyAsync(c->h_offs_num.data(), c->offs_num.p, 8 * (size_t)(n_off + 1), hipMemcpyDeviceToHost, s));
-  CHK(check_err(c, "symbolic"));  // synchronises the stream
+  int many = 0;
+  CHK(check_err(c, "symbolic", &many));  // synchronises the stream
   c->h_blockC.assign((size_t)c->nb, 0);
   for (int64_t b = 0; b < c->nb; ++b) c->h_blockC[(size_t)b] = hb[(size_t)b + 1] - hb[(size_t)b];
   c->info.nnz = c->nb > 0 ? hb[(size_t)c->nb] : 0;
   for (int k = 0; k < nt.n; ++k)
     c->info.num_rows[k] = c->h_offs_num[(size_t)(k + 1) * c->nwg] - c->h_offs_num[(size_t)k * c->nwg];
+  if (c->hub.n > 0) {  // the report's hub category: rows of more than kHubEntries entries
+    const int64_t few = c->info.num_rows[nt.n - 1] - many;
+    c->info.num_rows[nt.n - 1] -= few;
+    c->info.num_rows[nt.n - 2] += few;
+  }
   c->symb = true;
   return DBD_OK;
 }
@@ -650,7 +711,7 @@ dbd_status numeric_blocks(dbd_ctx* c, int64_t b0, int64_t b1, const int64_t* Cpt
     const int64_t i0 = (int64_t)k * c->nwg + w0, i1 = (int64_t)k * c->nwg + w1;
     const int64_t n = c->h_offs_num[(size_t)i1] - c->h_offs_num[(size_t)i0];
     if (n <= 0) continue;
-    if (c->tb.num_k[k].T == kHubShape) {  // rows with hub slots (hub_n > 0): the range kernels apply
+    if (c->tb.num_k[k].T == kHubShape) {  // rows with hub slots: the range kernels apply
       CHK(hub_numeric(c, c->h_offs_num[(size_t)i0], n, Cptr, cbase, Cidx, Cval));
       continue;
     }
@@ -702,7 +763,7 @@ int64_t fixed_device_bytes(dbd_ctx* c) {
   s += (int64_t)c->cnt.bytes + c->offs_sym.bytes + c->offs_num.bytes + c->tmp.bytes + c->cursor.bytes;
   s += (int64_t)c->bdesc_s.bytes + c->bdesc_l.bytes;
   s += (int64_t)c->band_hist.bytes + c->band_flag.bytes + c->band_tmp.bytes + c->band_slot.bytes + c->band_row.bytes +
-       c->band.bytes + c->hub_list.bytes + c->hub_cnt.bytes + c->hub_scnt.bytes + c->hub_rcnt.bytes + c->hub_tmp.bytes +
+       c->band.bytes + c->hub_meta.bytes + c->hub_scnt.bytes + c->hub_rcnt.bytes + c->hub_tmp.bytes +
        c->hub_scol.bytes + c->hub_sval.bytes + c->hub_slot.bytes + c->hub_flag.bytes + c->hub_rng.bytes;
   return s;
 }
@@ -1084,8 +1145,8 @@ dbd_status dbd_destroy(dbd_ctx* c) {
   if (c->cst) (void)hipStreamSynchronize(c->cst);
   for (auto* b : {&c->P, &c->Pptr, &c->nnz, &c->Cptr, &c->rows_sym, &c->rows_num, &c->cnt, &c->offs_sym, &c->offs_num,
                   &c->tmp, &c->cursor, &c->blk, &c->err, &c->g_rng, &c->bdesc_s, &c->bdesc_l, &c->band_hist,
-                  &c->band_flag, &c->band_tmp, &c->band_slot, &c->band_row, &c->band, &c->hub_list, &c->hub_cnt,
-                  &c->hub_scnt, &c->hub_rcnt, &c->hub_tmp, &c->hub_scol, &c->hub_sval, &c->hub_slot, &c->hub_flag,
+                  &c->band_flag, &c->band_tmp, &c->band_slot, &c->band_row, &c->band, &c->hub_meta, &c->hub_scnt,
+                  &c->hub_rcnt, &c->hub_tmp, &c->hub_scol, &c->hub_sval, &c->hub_slot, &c->hub_flag,
                   &c->hub_rng})
     b->release();
   for (int i = 0; i < 3; ++i) {
@@ -1281,6 +1342,7 @@ dbd_status dbd_backward(dbd_ctx* c, const int64_t* d_Cptr, const int32_t* d_Cidx
   if (!c->symb) return set_error(DBD_ERR_STATE, "dbd_backward needs the forward plan (run dbd_symbolic first)");
   hipStream_t s = c->st;
   launch_fill_i32(c->err.as<int32_t>(), 1, 0, s);
+  c->hub_split = false;  // the long rows' cursors take the records' place
   if (d_dA) launch_fill_bytes0(d_dA, (int64_t)c->vsz * c->A.nnz, s);
   const CatTable& nt = c->tb.num_ct;
   const int64_t* offs = c->offs_num.as<int64_t>();
@@ -1326,13 +1388,13 @@ void dbd::enqueue_pipeline(const Work& w, const Tables& tb, Mat A, const Mat& B,
   launch_bin_count(w.P, nr, B.ncols, ct, w.cnt, s);
   launch_exclusive_scan(w.cnt, w.offs_sym, (int64_t)ct.n * w.nwg, w.tmp, s);
   launch_bin_scatter(w.P, nr, B.ncols, ct, w.offs_sym, w.rows_sym, s);
+  if (w.hub_sym_fn) w.hub_sym_fn(w.hub_arg, s);
   for (int k = 1; k < ct.n; ++k)
     launch_symbolic(tb.sym_k[k], w.rows_sym, w.offs_sym + (int64_t)k * w.nwg, w.offs_sym + (int64_t)(k + 1) * w.nwg, 0,
-                    persistent_grid(num_cu, tb.sym_k[k]), A, B, w.nnz, w.cursor, w.err, s, w.hub_slot, w.hub_rng,
-                    w.nrng);
+                    persistent_grid(num_cu, tb.sym_k[k]), A, B, w.nnz, w.cursor, w.err, s, w.hub_slot);
   launch_exclusive_scan(w.nnz, d_Cptr, nr, w.tmp, s);
   const CatTable& nt = tb.num_ct;
-  launch_bin_count(w.nnz, nr, INT64_MAX, nt, w.cnt, s, w.hub_slot);
+  launch_bin_count(w.nnz, nr, INT64_MAX, nt, w.cnt, s, w.hub_slot, w.err + 1);
   launch_exclusive_scan(w.cnt, w.offs_num, (int64_t)nt.n * w.nwg, w.tmp, s);
   launch_bin_scatter(w.nnz, nr, INT64_MAX, nt, w.offs_num, w.rows_num, s, w.hub_slot);
   launch_capacity_guard(d_Cptr + nr, cap, w.offs_num, (int64_t)nt.n * w.nwg + 1, w.err, s);
@@ -1363,13 +1425,13 @@ static dbd_status batch_enqueue(dbd_ctx* c, hipStream_t s, int64_t* d_Cptr, int3
   w.err = c->err.as<int>();
   w.nr = c->nr;
   w.nwg = c->nwg;
-  if (c->bh_n > 0) {
-    w.hub_slot = c->hub_slot.as<int32_t>();
-    w.hub_rng = c->hub_rng.as<int32_t>();
-    w.nrng = hub_ranges(c->B.ncols);
+  if (c->hub.n > 0) {
+    w.hub_slot = c->hub.slot;
     w.hub_arg = c;
+    w.hub_sym_fn = [](void* arg, hipStream_t st) { hub_symbolic(static_cast<dbd_ctx*>(arg), st); };
     w.hub_fn = [](void* arg, const int64_t* Cptr, int32_t* Cidx, void* Cval, hipStream_t st) {
       dbd_ctx* cc = static_cast<dbd_ctx*>(arg);
+      if (cc->bh_n == 0) return;
       hub_head(cc, cc->bh_pos0, cc->bh_n, st);
       hub_tail(cc, cc->bh_pos0, cc->bh_n, cc->bh_nshort, Cptr, 0, Cidx, Cval, st);
     };
@@ -1395,7 +1457,7 @@ dbd_status dbd_batch_prepare(dbd_ctx* c, const dbd_csr* A_cat, const dbd_csr* B_
   // their range kernels, buckets included, sized here so the graph neither allocates nor waits
   c->bh_n = c->bh_pos0 = c->bh_nshort = 0;
   const CatTable& nt = c->tb.num_ct;
-  if (c->hub_n > 0 && c->tb.num_k[nt.n - 1].T == kHubShape) {
+  if (c->hub.n > 0 && c->tb.num_k[nt.n - 1].T == kHubShape) {
     const int64_t p0 = c->h_offs_num[(size_t)(nt.n - 1) * c->nwg], p1 = c->h_offs_num[(size_t)nt.n * c->nwg];
     if (p1 > p0) {
       CHK(hub_reserve(c, p1 - p0));

@@ -42,15 +42,32 @@ struct KernelShape {
   int G;   // lanes cooperating on one A entry (B row)
 };
 constexpr int kHubShape = -1;
-// Rows with more A entries than this, among the rows of the long (last by key) category, form the
-// hub category: their output is computed in column ranges, one workgroup per (row, range).
+// Hub rows: long rows whose output is computed in column ranges of kHubRange columns, one workgroup
+// per (row, range). Of the rows of the long (last by key) category these are the ones with more
+// than kHubEntries A entries (the windows of the other kernel visit them all, window after window)
+// and the ones with at least per_range products for every range between their first and last
+// column (kHubPerRange, so a range's products outweigh its clears, its emission and its visits of
+// the entries).
 #ifndef DBD_HUB_ENTRIES
 #define DBD_HUB_ENTRIES 1024
 #endif
+#ifndef DBD_HUB_PER_RANGE
+#define DBD_HUB_PER_RANGE 2048
+#endif
 constexpr int64_t kHubEntries = DBD_HUB_ENTRIES;
-// Column ranges of the hub-row kernels (16384 columns); the symbolic long windows hold whole ranges.
-constexpr int kHubRangeShift = 14;
+constexpr int64_t kHubPerRange = DBD_HUB_PER_RANGE;
+constexpr int kHubRangeShift = 13;
 constexpr int kHubRange = 1 << kHubRangeShift;
+__host__ __device__ inline bool hub_row(int64_t nA, int64_t P, int nrng, int64_t per_range) {
+  return nA > kHubEntries || P / nrng >= per_range;
+}
+// A slot value carries kHubMany for the rows of more than kHubEntries entries (plan reports count
+// the others as long rows) and kHubFineBit for the rows counted range by range; a row's flag has a
+// 1 for a hub row and a kHubFineOne for a fine one, so one scan gives its place in both lists.
+constexpr int32_t kHubMany = 1 << 30, kHubFineBit = 1 << 29;
+constexpr int32_t kHubSlotMask = kHubFineBit - 1;
+constexpr int kHubFineShift = 40;
+constexpr int64_t kHubFineOne = (int64_t)1 << kHubFineShift;
 
 // ---- generic device utilities ----
 void launch_fill_i64(int64_t* p, int64_t n, int64_t v, hipStream_t s);
@@ -95,22 +112,19 @@ void launch_row_products(const Mat& A, const Mat& B, int64_t* P, int64_t* nnz, i
 // counts/offs have ncat * nwg (+1) int64 where nwg = bin_tiles(n).
 int64_t bin_tiles(int64_t n);
 // With hub_slot, rows of the category before the last (the long one by key) that have a hub slot
-// (>= 0) go to the last category (the hub category).
+// (>= 0) go to the last category (the hub category); *many counts those marked kHubMany.
 void launch_bin_count(const int64_t* key, int64_t n, int64_t cap, const CatTable& ct, int64_t* counts,
-                      hipStream_t s, const int32_t* hub_slot = nullptr);
+                      hipStream_t s, const int32_t* hub_slot = nullptr, int* many = nullptr);
 void launch_bin_scatter(const int64_t* key, int64_t n, int64_t cap, const CatTable& ct, const int64_t* offs,
                         int32_t* rows, hipStream_t s, const int32_t* hub_slot = nullptr);
 
 // ---- symbolic / numeric / backward per category ----
 // grid == 0 -> exact grid from nrows_hint; else a persistent grid of that many workgroups.
 int symbolic_groups_per_wg(const KernelShape& k);
-// With hub_slot, the long-row kernel gives rows of slot hs >= 0 windows aligned to whole hub ranges
-// and writes their columns per range into rng_cnt[hs * nrng + range] (ranges with no column are
-// left as they are: zero them first).
+// With hub_slot, the long-row kernel leaves out the rows that have a slot (>= 0): launch_hub_count's.
 void launch_symbolic(const KernelShape& k, const int32_t* rows, const int64_t* pbeg, const int64_t* pend,
                      int64_t nrows_hint, int grid, const Mat& A, const Mat& B, int64_t* nnz, int64_t* cursor,
-                     int* err, hipStream_t s, const int32_t* hub_slot = nullptr, int32_t* rng_cnt = nullptr,
-                     int nrng = 0);
+                     int* err, hipStream_t s, const int32_t* hub_slot = nullptr);
 // distinct: most products of the problem are distinct columns of their row (nnzC close to the
 // product count); the one-wave shapes then take rows whose products are all distinct through a
 // register path instead of the hash table.
@@ -118,33 +132,57 @@ void launch_numeric(int dtype, const KernelShape& k, const int32_t* rows, const 
                     const int64_t* pend, int64_t nrows_hint, int grid, const Mat& A, const Mat& B,
                     const int64_t* Cptr, int64_t cbase, int32_t* Cidx, void* Cval, int64_t* cursor, int* err,
                     hipStream_t s, bool distinct = false);
-// Hub rows rows[0, nh) in column ranges of 16384 (hub_ranges(ncols) of them; B's band index
-// required). prepare: per (row, range) count of the short entries' products into scnt[nh *
-// nrng], each row's banded entries (offsets in the row) into hlist at the row's A positions and
-// their number into hcount. scatter: those products, (column, value), into buckets at soff (the
-// exclusive scan of scnt). range(count): distinct columns per (row, range) into rcnt;
-// range(!count): values, emitted at Cptr[row] - cbase + roff[item] - roff[row's first item].
-constexpr int kHubMaxRanges = 4096;
+// ---- hub rows ----
+constexpr int kHubMaxRanges = 8192;
 int hub_ranges(int64_t ncols);
-// Hub slots: flag[j] = 1 for rows[j] with more than kHubEntries A entries; with pos the exclusive
-// scan of flag, hub_slot[rows[j]] = pos[j] for the flagged rows (hub_slot filled with -1 first).
-void launch_hub_flags(const int32_t* rows, int64_t n, const int64_t* Aptr, int64_t* flag, hipStream_t s);
-void launch_hub_slots(const int32_t* rows, int64_t n, const int64_t* flag, const int64_t* pos, int32_t* hub_slot,
-                      hipStream_t s);
-// rcnt[j * nrng + r] = rng_cnt[hub_slot[rows[j]] * nrng + r] (the symbolic pass's range counts).
-void launch_hub_gather_counts(const int32_t* rows, int64_t n, int nrng, const int32_t* hub_slot,
-                              const int32_t* rng_cnt, int64_t* rcnt, hipStream_t s);
-void launch_hub_prepare(const int32_t* rows, int64_t nh, const Mat& A, const Mat& B, int nrng, int64_t* scnt,
-                        int32_t* hlist, int32_t* hcount, hipStream_t s);
-void launch_hub_scatter(int dtype, const int32_t* rows, int64_t nh, const Mat& A, const Mat& B, int nrng,
-                        const int64_t* soff, int32_t* scol, void* sval, const int* err, hipStream_t s);
-// Sets the capacity bit in err when *total (the hub rows' short products) exceeds cap: the hub
-// scatter and range kernels then write nothing.
+// Ranges per window of the hub rows' symbolic count, for B of this width and so many long rows.
+int hub_wide(int64_t ncols, int64_t nlong);
+// Whether the short entries' products are bucketed per (row, range) for B of this width.
+bool hub_buckets_used(int64_t ncols);
+// Device workspace of the hub rows: their list (slot -> row) and slots (row -> slot, -1: none), the
+// slots of the fine rows (counted range by range), chunk offsets of the split and the buckets
+// (n + 1), scan partials, the entry records (16 bytes per A nonzero), per slot the number of banded
+// and short entries and the column span (2), the columns per (slot, range), and what the range
+// workgroups read of their row.
+struct HubWork {
+  int64_t n = 0, nfine = 0;
+  int wide = 16;  // ranges per count window (hub_wide)
+  int32_t *rows = nullptr, *slot = nullptr, *fine = nullptr, *hcnt = nullptr, *lcnt = nullptr, *span = nullptr,
+          *rng_cnt = nullptr;
+  int64_t *coff = nullptr, *boff = nullptr, *tmp = nullptr;
+  void *recs = nullptr, *info = nullptr;
+};
+constexpr size_t kHubRowBytes = 32;  // of info, per row of a chunk
+// flag[j] of rows[j] by hub_row; with pos the exclusive scan of flag: h's slots (filled with -1
+// first), list and fine list.
+void launch_hub_flags(const int32_t* rows, int64_t n, const Mat& A, const Mat& B, const int64_t* P, int64_t per_range,
+                      int wide, int64_t products, int64_t* flag, hipStream_t s);
+void launch_hub_slots(const int32_t* rows, int64_t n, const Mat& A, const int64_t* flag, const int64_t* pos,
+                      const HubWork& h, hipStream_t s);
+// The rows' entries by kind into h.recs (hcnt, lcnt, span), nnz of the rows and *many cleared. Rows that are
+// not long by their products (min(P, ncols) <= key_lim) are left empty.
+void launch_hub_split(const HubWork& h, const Mat& A, const Mat& B, const int64_t* P, int64_t key_lim, int64_t* nnz,
+                      int* many, hipStream_t s);
+// Columns per (slot, range) into h.rng_cnt, their sums added to nnz (after launch_hub_split).
+void launch_hub_count(const HubWork& h, const Mat& A, const Mat& B, int64_t* nnz, hipStream_t s);
+// For the hub rows rows[0, n) of a chunk. gather: rcnt[j * nrng + r] = the row's columns per range,
+// and h.info. bucket_count: short entries' products per (row, range) into scnt[n * nrng];
+// bucket_fill: those products, (column, value), at soff (the exclusive scan of scnt; scnt is used
+// up). guard: sets the capacity bit in err when *total short products exceed cap, on which
+// bucket_fill and range write nothing. range: the values, emitted at Cptr[row] - cbase + roff[item]
+// - roff[row's first item]; soff null: no buckets, the short entries are read from B.
+void launch_hub_gather_counts(const HubWork& h, const int32_t* rows, int64_t n, const Mat& A, const Mat& B,
+                              const int64_t* Cptr, int64_t cbase, int64_t* rcnt, hipStream_t s);
+void launch_hub_bucket_count(const HubWork& h, const int32_t* rows, int64_t n, const Mat& A, const Mat& B,
+                             int64_t* scnt, hipStream_t s);
+void launch_hub_bucket_fill(int dtype, const HubWork& h, const int32_t* rows, int64_t n, const Mat& A, const Mat& B,
+                            int64_t* scnt, const int64_t* soff, int32_t* scol, void* sval, const int* err,
+                            hipStream_t s);
 void launch_hub_guard(const int64_t* total, int64_t cap, int* err, hipStream_t s);
-void launch_hub_range(int dtype, const int32_t* rows, int64_t nh, int nrng, const Mat& A, const Mat& B,
-                      const int32_t* hlist, const int32_t* hcount, const int64_t* soff, const int32_t* scol,
-                      const void* sval, const int64_t* roff, const int64_t* Cptr, int64_t cbase, int32_t* Cidx,
-                      void* Cval, int* err, hipStream_t s);
+void launch_hub_range(int dtype, const HubWork& h, int64_t nh, const Mat& A, const Mat& B, const int64_t* soff,
+                      const int32_t* scol, const void* sval, const int64_t* roff, int32_t* Cidx, void* Cval, int* err,
+                      hipStream_t s);
+
 void launch_backward(int dtype, const KernelShape& k, const int32_t* rows, const int64_t* pbeg,
                      const int64_t* pend, int64_t nrows_hint, int grid, const Mat& A, const Mat& B,
                      const int64_t* Cptr, const int32_t* Cidx, const void* dC, void* dA, void* dB, int64_t* cursor,

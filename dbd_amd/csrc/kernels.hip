@@ -974,8 +974,8 @@ __device__ __forceinline__ int category_of(int64_t k, const CatTable& ct) {
 
 // Category of row i: by key. Numeric tables end with the long category (limit INT64_MAX, so no
 // key goes past it) and the hub category; with hub_slot, a long row that has a hub slot (a
-// symbolic long row of more than kHubEntries A entries, whose range counts the symbolic pass
-// wrote) is a hub row. Without hub_slot the hub category stays empty.
+// symbolic long row that hub_row picks, whose columns per range the symbolic pass counted) is a
+// hub row. Without hub_slot the hub category stays empty.
 __device__ __forceinline__ int row_category(int64_t k, const CatTable& ct, const int32_t* __restrict__ hub_slot,
                                             int64_t i) {
   const int c = category_of(k, ct);
@@ -985,7 +985,8 @@ __device__ __forceinline__ int row_category(int64_t k, const CatTable& ct, const
 
 __global__ __launch_bounds__(kBinTile) void k_bin_count(const int64_t* __restrict__ key, int64_t n, int64_t cap,
                                                         CatTable ct, int64_t* __restrict__ counts, int64_t nwg,
-                                                        const int32_t* __restrict__ hub_slot) {
+                                                        const int32_t* __restrict__ hub_slot,
+                                                        int* __restrict__ many) {
   __shared__ int hist[kMaxCats];
   if (threadIdx.x < kMaxCats) hist[threadIdx.x] = 0;
   __syncthreads();
@@ -993,7 +994,9 @@ __global__ __launch_bounds__(kBinTile) void k_bin_count(const int64_t* __restric
   if (i < n) {
     int64_t k = key[i];
     if (k > cap) k = cap;
-    atomicAdd(&hist[row_category(k, ct, hub_slot, i)], 1);
+    const int c = row_category(k, ct, hub_slot, i);
+    atomicAdd(&hist[c], 1);
+    if (hub_slot && c == ct.n - 1 && (hub_slot[i] & kHubMany)) atomicAdd(many, 1);
   }
   __syncthreads();
   if ((int)threadIdx.x < ct.n) counts[(int64_t)threadIdx.x * nwg + blockIdx.x] = hist[threadIdx.x];
@@ -1027,10 +1030,11 @@ __global__ __launch_bounds__(kBinTile) void k_bin_scatter(const int64_t* __restr
 }
 
 void launch_bin_count(const int64_t* key, int64_t n, int64_t cap, const CatTable& ct, int64_t* counts,
-                      hipStream_t s, const int32_t* hub_slot) {
+                      hipStream_t s, const int32_t* hub_slot, int* many) {
   const int64_t nwg = bin_tiles(n);
   if (nwg == 0) return;
-  hipLaunchKernelGGL(k_bin_count, dim3((unsigned)nwg), dim3(kBinTile), 0, s, key, n, cap, ct, counts, nwg, hub_slot);
+  hipLaunchKernelGGL(k_bin_count, dim3((unsigned)nwg), dim3(kBinTile), 0, s, key, n, cap, ct, counts, nwg, hub_slot,
+                     many);
 }
 void launch_bin_scatter(const int64_t* key, int64_t n, int64_t cap, const CatTable& ct, const int64_t* offs,
                         int32_t* rows, hipStream_t s, const int32_t* hub_slot) {
@@ -1158,7 +1162,7 @@ constexpr int kSpanCap = 64;
 constexpr int kSymSpanEntries = 64;  // symbolic span walks: rows of up to one wave of entries
 
 // Rows too long for an LDS table: sweep the row's columns in windows of W bits.
-// With B's band index, rows of up to kSymSpanEntries entries (no hub slot) walk
+// With B's band index, rows of up to kSymSpanEntries entries walk
 // element-parallel: every active entry's element span in the window (banded B rows: up to the
 // band boundary at or past the window end; other B rows: at most kSpanCap elements, the
 // window then ending before the first element left out) is flattened by a scan in wave 0, each
@@ -1166,7 +1170,8 @@ constexpr int kSymSpanEntries = 64;  // symbolic span walks: rows of up to one w
 // length, elements consumed, next column, band slot) lives in LDS. (A workgroup-wide version for
 // rows of up to NT entries measured slower than the cursor walks below: its scans cost more
 // barriers per window than the walks' chains.)
-// Otherwise one cursor per A entry (cursor[] is indexed like A's nonzeros) walks its sorted B
+// Otherwise one cursor per A entry (16 bytes per A nonzero, so a row's workspace lies beside its
+// entries for every kernel that uses it) walks its sorted B
 // row, whose extent comes from the row analysis' descriptors; an entry with more elements in the
 // window than one step of G continues UL steps at a time, their loads issued together.
 template <int NT, int W, int G>
@@ -1174,20 +1179,16 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_
     const int32_t* __restrict__ rows, const int64_t* __restrict__ pbeg, const int64_t* __restrict__ pend,
     const int64_t* __restrict__ Aptr, const int64_t* __restrict__ bstart, const int32_t* __restrict__ blen,
     const int32_t* __restrict__ Bidx, int64_t* __restrict__ nnz, int64_t* __restrict__ cursor,
-    int* __restrict__ err, const int32_t* __restrict__ hub_slot, int32_t* __restrict__ rng_cnt, int nrng,
-    const int32_t* __restrict__ Aidx, const int32_t* __restrict__ hslot, const int32_t* __restrict__ band,
+    int* __restrict__ err, const int32_t* __restrict__ hub_slot, const int32_t* __restrict__ Aidx, const int32_t* __restrict__ hslot, const int32_t* __restrict__ band,
     int64_t nb1) {
   constexpr int NWORD = W / 32;
   constexpr int WPT = NWORD / NT;
   constexpr int UL = 8;
   constexpr int U = 4;
-  constexpr int RPW = W >> kHubRangeShift;          // hub ranges per window
-  constexpr int RWORD = NWORD / RPW;                // bitmap words per hub range
-  static_assert(NWORD % NT == 0 && W % kHubRange == 0 && NT % 64 == 0, "shape");
+  static_assert(NWORD % NT == 0 && NT % 64 == 0, "shape");
   __shared__ uint32_t bm[NWORD];
   __shared__ int sc[NT / 64 > 0 ? NT / 64 : 1];
   __shared__ long long scl[NT / 64 > 0 ? NT / 64 : 1];
-  __shared__ int rc[RPW];
   // span-walk entry state and window tables (entry e in slot e)
   __shared__ int64_t eB0[kSymSpanEntries];
   __shared__ int eL[kSymSpanEntries], eP[kSymSpanEntries], eNC[kSymSpanEntries], eSL[kSymSpanEntries];
@@ -1198,13 +1199,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_
   const int64_t beg = *pbeg, end = *pend;
   for (int64_t slot = beg + blockIdx.x; slot < end; slot += gridDim.x) {
     const int row = rows[slot];
+    if (hub_slot && hub_slot[row] >= 0) continue;  // uniform: k_hub_count counts the hub rows
     const int64_t a0 = Aptr[row], a1 = Aptr[row + 1];
-    // rows with a hub slot take windows aligned to W and record their columns per hub range
-    const int hs = hub_slot ? hub_slot[row] : -1;
 #pragma unroll
     for (int q = 0; q < WPT; ++q) bm[t + q * NT] = 0u;
     const int nA = (int)min(a1 - a0, (int64_t)kSymSpanEntries + 1);
-    if (band != nullptr && hs < 0 && nA <= kSymSpanEntries) {  // uniform
+    if (band != nullptr && nA <= kSymSpanEntries) {  // uniform
       // ================= span walks (entries in slots 0 .. nA - 1, wave 0) =================
       long long prow_l = 0;
       if (t < nA) {
@@ -1325,7 +1325,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_
     long long prow_l = 0;
     for (int64_t ka = a0 + t; ka < a1; ka += NT) {
       const int64_t b0 = bstart[ka];
-      cursor[ka] = b0;
+      cursor[2 * ka] = b0;
       prow_l += blen[ka];
       if (blen[ka] > 0) lo_l = min(lo_l, Bidx[b0]);
     }
@@ -1336,10 +1336,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_
     long long count = 0;
     long long windows = 0;
     while (lo != INT_MAX) {
-      if (hs >= 0) lo &= ~(W - 1);  // uniform
       const int64_t hi = min((int64_t)lo + W, (int64_t)INT_MAX);  // INT_MAX: past the B row
       for (int64_t ka = a0 + t / G; ka < a1; ka += NT / G) {
-        int64_t p = cursor[ka];
+        int64_t p = cursor[2 * ka];
         const int64_t b1 = bstart[ka] + blen[ka];
         int nin;
         {
@@ -1376,27 +1375,20 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_
             }
           }
         }
-        if (lg == 0) cursor[ka] = p;
+        if (lg == 0) cursor[2 * ka] = p;
       }
-      if (hs >= 0 && t < RPW) rc[t] = 0;
       __syncthreads();
       long long pc = 0;
 #pragma unroll
       for (int q = 0; q < WPT; ++q) {
         const int wq = __popc(bm[t + q * NT]);
         pc += wq;
-        if (hs >= 0 && wq) atomicAdd(&rc[(t + q * NT) / RWORD], wq);
         bm[t + q * NT] = 0u;
       }
       count += pc;
-      if (hs >= 0) {  // uniform
-        __syncthreads();
-        const int r0 = lo >> kHubRangeShift;
-        if (t < RPW && r0 + t < nrng) rng_cnt[(int64_t)hs * nrng + r0 + t] = rc[t];
-      }
       int nl = INT_MAX;
       for (int64_t ka = a0 + t; ka < a1; ka += NT) {
-        const int64_t p = cursor[ka];
+        const int64_t p = cursor[2 * ka];
         if (p < bstart[ka] + blen[ka]) nl = min(nl, Bidx[p]);
       }
       lo = Group<NT>::reduce(nl, OpMin(), sc);
@@ -1412,215 +1404,508 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(8))) void k_
 }
 
 // ------------------------------------------------------------------------------------
-// hub rows: rows with more A entries than the window kernels hold (kHubEntries)
+// hub rows: long rows computed in column ranges
 // ------------------------------------------------------------------------------------
-// A numeric window kernel visits every A entry of its row in every dense window of 4096 columns
-// it sweeps, so a row's cost grows as nA * ncols / 4096 beside its products: over a few million
-// columns a row of thousands of entries spends more on those visits than on its products, and
-// the whole row is one workgroup's work. Hub rows are cut into ranges of kHubRange columns
-// instead, one workgroup per (row, range), each accumulating its range in LDS (a presence bitmap
-// and, for the numeric pass, dense values), so a heavy row spreads over the GPU and no product
-// needs a global atomic:
-//   - entries whose B row is in the band index (long B rows) read their range's element span
-//     from two index entries; `k_hub_prepare` lists them per row (in A's order) and counts the
-//     products of the other (short) entries per range; `k_hub_scatter` writes those products,
-//     (column, a_ik * b_kj), into per-(row, range) buckets;
-//   - the symbolic long kernel counts each range's columns (hub rows' windows are aligned to
-//     whole ranges), a scan turns the counts into output offsets, and `k_hub_range` accumulates
-//     the range and emits it in column order at its offset.
-// Within a bucket the products' order follows LDS atomics, so sums of a column may associate
-// differently from run to run (within the usual rounding bound).
+// A window kernel sweeps its row with one workgroup, window after window, and visits the row's A
+// entries in every window: one round trip to memory after another, on one CU, however many are
+// idle. Hub rows are cut into ranges of kHubRange columns instead, a workgroup per (row, range)
+// that accumulates in LDS, so a heavy row spreads over the GPU and no product needs a global
+// atomic:
+//   - k_hub_split lists each row's entries by kind, 16 bytes each beside the row's A entries: those
+//     whose B row is in the band index (a range's element span is two index entries) from the
+//     front, the others (short B rows) from the back; and the row's first and last column;
+//   - k_hub_count counts the columns of every range (bitmap windows of one or several ranges), for
+//     nnz_i and, scanned, the ranges' output offsets;
+//   - over more than kHubWhole ranges the short B rows' products, (column, a_ik * b_kj), are
+//     bucketed per (row, range) by k_hub_bucket; over fewer each range reads the short rows whole
+//     and keeps its part (a short row's few cache lines cost less than writing and reading 12
+//     bytes per product);
+//   - k_hub_range accumulates a range and emits it in column order at its offset.
+// Which rows: hub_row (kernels.h). Sums of a column may associate differently from run to run (the
+// order of LDS atomics), within the usual rounding bound.
 constexpr int kHubRangeBands = kHubRange >> kBandShift;
+constexpr int kHubSplitNT = 256;
+constexpr int kHubSplitPer = 4;
+constexpr int kHubChunk = kHubSplitNT * kHubSplitPer;  // entries of a row per k_hub_split workgroup
+constexpr int kHubBucketChunk = 512;                   // short entries of a row per k_hub_bucket workgroup
+constexpr int kHubWhole = 8;
 
-template <int NT>
-__global__ __launch_bounds__(NT) void k_hub_prepare(const int32_t* __restrict__ rows, const int64_t* __restrict__ Aptr,
-                                                    const int32_t* __restrict__ Aidx,
-                                                    const int64_t* __restrict__ bstart,
-                                                    const int32_t* __restrict__ blen, const int32_t* __restrict__ Bidx,
-                                                    const int32_t* __restrict__ hslot, int nrng,
-                                                    int64_t* __restrict__ scnt, int32_t* __restrict__ hlist,
-                                                    int32_t* __restrict__ hcount) {
-  extern __shared__ int lcnt[];  // nrng counters
-  __shared__ int sc[NT / 64];
-  const int t = threadIdx.x;
-  const int64_t j = blockIdx.x;
-  const int row = rows[j];
-  const int64_t a0 = Aptr[row], nA = Aptr[row + 1] - a0;
-  for (int r = t; r < nrng; r += NT) lcnt[r] = 0;
+// The kinds of entries as k_hub_split lists them: start of the B row, its band slot or (short) its
+// length, index in the A row.
+struct HubRec {
+  int64_t b0;
+  int32_t s;
+  int32_t e;
+};
+static_assert(sizeof(HubRec) == 16, "records share the 16-byte workspace slots");
+
+// Per hub row: workgroups that split it (none for a row that is not long: only after a captured
+// pipeline's operands changed structure), and its counters and column span cleared; also the
+// number of rows of many entries that the numeric binning counts.
+__global__ void k_hub_chunks(const int32_t* __restrict__ hub_rows, int64_t n, const int64_t* __restrict__ Aptr,
+                             const int64_t* __restrict__ P, int64_t ncols, int64_t key_lim, int64_t* __restrict__ cnt,
+                             int32_t* __restrict__ hcnt, int32_t* __restrict__ lcnt, int32_t* __restrict__ span,
+                             int64_t* __restrict__ nnz, int* __restrict__ many) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *many = 0;
+  for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (int64_t)gridDim.x * blockDim.x) {
+    const int r = hub_rows[j];
+    const bool is_long = min(P[r], ncols) > key_lim;
+    cnt[j] = is_long ? (Aptr[r + 1] - Aptr[r] + kHubChunk - 1) / kHubChunk : 0;
+    if (is_long) nnz[r] = 0;  // k_hub_count adds the ranges' columns up
+    hcnt[j] = lcnt[j] = 0;
+    span[2 * j] = INT_MAX;
+    span[2 * j + 1] = -1;
+  }
+}
+
+// The list entry whose chunks hold chunk q (off: exclusive scan of the chunk counts, n + 1 entries).
+__device__ __forceinline__ int64_t chunk_owner(const int64_t* __restrict__ off, int64_t n, int64_t q) {
+  int64_t lo = 0, hi = n - 1;
+  while (lo < hi) {
+    const int64_t m = (lo + hi + 1) >> 1;
+    if (off[m] <= q) lo = m;
+    else hi = m - 1;
+  }
+  return lo;
+}
+
+__global__ __launch_bounds__(kHubSplitNT) void k_hub_split(
+    const int32_t* __restrict__ hub_rows, int64_t n, const int64_t* __restrict__ coff, const int64_t* __restrict__ Aptr,
+    const int32_t* __restrict__ Aidx, const int64_t* __restrict__ bstart, const int32_t* __restrict__ blen,
+    const int32_t* __restrict__ Bidx, const int32_t* __restrict__ hslot, HubRec* __restrict__ recs,
+    int32_t* __restrict__ hcnt, int32_t* __restrict__ lcnt, int32_t* __restrict__ span) {
+  __shared__ int s_n[2], s_base[2];
+  const int64_t q = blockIdx.x;
+  if (q >= coff[n]) return;  // the grid is a bound
+  const int64_t j = chunk_owner(coff, n, q);
+  const int row = hub_rows[j];
+  const int64_t a0 = Aptr[row], nA = Aptr[row + 1] - a0, e0 = (q - coff[j]) * kHubChunk;
+  const int t = threadIdx.x, lane = t & 63;
+  if (t < 2) s_n[t] = 0;
   __syncthreads();
-  int nH = 0;  // banded entries listed so far (uniform)
-  for (int64_t e0 = 0; e0 < nA; e0 += NT) {  // uniform
-    const int64_t e = e0 + t;
-    int banded = 0;
+  HubRec rec[kHubSplitPer];
+  int kind[kHubSplitPer], pos[kHubSplitPer];  // 0: banded, 1: short, -1: no product
+  int cmin = INT_MAX, cmax = -1;
+#pragma unroll
+  for (int i = 0; i < kHubSplitPer; ++i) {
+    const int64_t e = e0 + t + i * kHubSplitNT;
+    kind[i] = -1;
     if (e < nA) {
       const int64_t ka = a0 + e;
-      if (hslot[Aidx[ka]] >= 0) {
-        banded = 1;
-      } else {
-        const int64_t b0 = bstart[ka];
-        const int L = blen[ka];
-        for (int q = 0; q < L; ++q) atomicAdd(&lcnt[Bidx[b0 + q] >> kHubRangeShift], 1);
+      const int L = blen[ka];
+      const int sl = hslot[Aidx[ka]];
+      if (L > 0) {
+        kind[i] = sl >= 0 ? 0 : 1;
+        rec[i] = HubRec{bstart[ka], sl >= 0 ? sl : L, (int)e};
+        cmin = min(cmin, Bidx[rec[i].b0]);
+        cmax = max(cmax, Bidx[rec[i].b0 + L - 1]);
       }
     }
-    int tot;
-    const int pre = Group<NT>::exscan(banded, tot, sc);
-    if (banded) hlist[a0 + nH + pre] = (int32_t)e;
-    nH += tot;
+  }
+#pragma unroll
+  for (int i = 0; i < kHubSplitPer; ++i) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const uint64_t b = __builtin_amdgcn_ballot_w64(kind[i] == k);
+      int at = 0;
+      if (lane == 0) at = atomicAdd(&s_n[k], (int)__popcll(b));
+      at = __builtin_amdgcn_readfirstlane(at);
+      if (kind[i] == k) pos[i] = at + __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0));
+    }
   }
   __syncthreads();
-  for (int r = t; r < nrng; r += NT) scnt[j * nrng + r] = lcnt[r];
-  if (t == 0) hcount[j] = nH;
-}
-
-template <typename V, int NT>
-__global__ __launch_bounds__(NT) void k_hub_scatter(const int32_t* __restrict__ rows, const int64_t* __restrict__ Aptr,
-                                                    const int32_t* __restrict__ Aidx,
-                                                    const int64_t* __restrict__ bstart,
-                                                    const int32_t* __restrict__ blen, const V* __restrict__ Aval,
-                                                    const int32_t* __restrict__ Bidx, const V* __restrict__ Bval,
-                                                    const int32_t* __restrict__ hslot, int nrng,
-                                                    const int64_t* __restrict__ soff, int32_t* __restrict__ scol,
-                                                    V* __restrict__ sval, const int* __restrict__ err) {
-  extern __shared__ unsigned long long lcur[];  // nrng write positions
-  if (*err & kErrCapacity) return;  // the buckets (or C) are smaller than this structure needs
-  const int t = threadIdx.x;
-  const int64_t j = blockIdx.x;
-  const int row = rows[j];
-  const int64_t a0 = Aptr[row], nA = Aptr[row + 1] - a0;
-  for (int r = t; r < nrng; r += NT) lcur[r] = (unsigned long long)soff[j * nrng + r];
+  if (t == 0) s_base[0] = atomicAdd(&hcnt[j], s_n[0]);
+  if (t == 1) s_base[1] = atomicAdd(&lcnt[j], s_n[1]);
   __syncthreads();
-  for (int64_t e = t; e < nA; e += NT) {
-    const int64_t ka = a0 + e;
-    if (hslot[Aidx[ka]] >= 0) continue;
-    const int64_t b0 = bstart[ka];
-    const int L = blen[ka];
-    const V av = Aval[ka];
-    for (int q = 0; q < L; ++q) {
-      const int col = Bidx[b0 + q];
-      const int64_t pos = (int64_t)atomicAdd(&lcur[col >> kHubRangeShift], 1ull);
-      scol[pos] = col;
-      sval[pos] = av * Bval[b0 + q];
-    }
+#pragma unroll
+  for (int i = 0; i < kHubSplitPer; ++i) {
+    if (kind[i] == 0) recs[a0 + s_base[0] + pos[i]] = rec[i];
+    if (kind[i] == 1) recs[a0 + nA - 1 - (s_base[1] + pos[i])] = rec[i];
+  }
+  cmin = wave_reduce_dpp(cmin, OpMin());
+  cmax = wave_reduce_dpp(cmax, OpMax());
+  if (lane == 0 && cmax >= 0) {
+    atomicMin(&span[2 * j], cmin);
+    atomicMax(&span[2 * j + 1], cmax);
   }
 }
 
-// One (row, range) item per workgroup: the range's values, emitted at Cptr[row] - cbase +
-// roff[item] - roff[first item of the row], with roff[item + 1] - roff[item] columns expected.
-template <typename V, int NT>
-__global__ __launch_bounds__(NT) void k_hub_range(
-    const int32_t* __restrict__ rows, int nrng, const int64_t* __restrict__ Aptr, const int32_t* __restrict__ Aidx,
-    const int64_t* __restrict__ bstart, const V* __restrict__ Aval, const int32_t* __restrict__ Bidx,
-    const V* __restrict__ Bval, const int32_t* __restrict__ hslot, const int32_t* __restrict__ band, int64_t nb1,
-    const int32_t* __restrict__ hlist, const int32_t* __restrict__ hcount, const int64_t* __restrict__ soff,
-    const int32_t* __restrict__ scol, const V* __restrict__ sval,
-    const int64_t* __restrict__ roff, const int64_t* __restrict__ Cptr, int64_t cbase, int32_t* __restrict__ Cidx,
-    V* __restrict__ Cval, int* __restrict__ err) {
-  constexpr int NWORD = kHubRange / 32;
-  constexpr int NW = NT / 64;
-  constexpr int U = 4;
-  static_assert(NWORD <= NT, "one bitmap word per thread at most");
-  __shared__ uint32_t bm[NWORD];
-  __shared__ V dv[kHubRange];
-  __shared__ int64_t hb0[NT];
-  __shared__ V hva[NT];
-  __shared__ int hS[NT];
-  __shared__ int sc[NW];
-  if (*err & kErrCapacity) return;  // the buckets or C are smaller than this structure needs
-  const int t = threadIdx.x, lane = t & 63;
-  const int64_t item = blockIdx.x;
-  // a range without columns (by the symbolic count) holds no product: nothing to add or emit
-  if (roff[item + 1] == roff[item]) return;
-  const int64_t j = item / nrng;
-  const int r = (int)(item - j * nrng);
-  const int row = rows[j];
-  const int64_t a0 = Aptr[row];
-  const int nH = hcount[j];
-  const int64_t c0 = (int64_t)r << kHubRangeShift;
-  const int64_t w0 = c0 >> kBandShift;
-  const int64_t w1 = min(w0 + kHubRangeBands, nb1 - 1);
-  for (int q = t; q < NWORD; q += NT) bm[q] = 0u;
-  for (int q = t; q < kHubRange; q += NT) dv[q] = V(0);
-  __syncthreads();
-  // products of the banded entries in this range: chunks of NT entries, each wave taking 64 of
-  // them (strided, so the heaviest entries, which lie together in A's order, spread over the
-  // waves) and gathering its entries' spans element-parallel on its own: a wave scan flattens
-  // them and an element's owner is searched among 64 entries, with no workgroup barrier
-  const int wv = t >> 6;
-  int* whS = hS + (t & ~63);
-  const int64_t* whb0 = hb0 + (t & ~63);
-  const V* whva = hva + (t & ~63);
-  for (int e0 = 0; e0 < nH; e0 += NT) {  // uniform
-    const int e = e0 + wv + (NT / 64) * lane;
-    int len = 0;
-    if (e < nH) {
-      const int64_t ka = a0 + hlist[a0 + e];
-      const int32_t* bd = band + (int64_t)hslot[Aidx[ka]] * nb1;
-      const int s0 = bd[w0];
-      len = bd[w1] - s0;
-      hb0[t] = bstart[ka] + s0;
-      hva[t] = Aval[ka];
-    }
-    const int incl = wave_incl_scan_dpp(len);
-    hS[t] = incl - len;  // lanes past the row's entries hold the wave total: never an owner
-    const int T = __builtin_amdgcn_readlane(incl, 63);
+// Element-parallel walk of one wave over the spans of up to 64 entries, one per lane (`len`
+// elements at `start`): extra(rank) stores what else the elements need of this lane's entry, at its
+// rank among the entries with elements, and body(at, j) takes U elements per lane, element u of
+// them at position at[u], of the entry of rank j[u] (at[u] < 0: none). The owner of a flattened
+// element is not searched: the entries set a bit where their elements begin (word 64-wide, bit
+// S - 1 for the entry that starts at S >= 1), and an element's owner is the number of bits before
+// it, one mbcnt on a mask that readlane makes wave-uniform (a bisection over 64 starts costs 6
+// dependent LDS reads per element). tb and wm: 64 entries of LDS of this wave's own.
+template <int U, typename X, typename F>
+__device__ __forceinline__ void walk_spans(int lane, int len, int64_t start, int64_t* tb, unsigned long long* wm,
+                                           X&& extra, F&& body) {
+  const uint64_t live = __builtin_amdgcn_ballot_w64(len > 0);
+  if (!live) return;
+  const int incl = wave_incl_scan_dpp(len);
+  const int S = incl - len;
+  const int T = __builtin_amdgcn_readlane(incl, 63);
+  if (len > 0) {
+    const int r = __builtin_amdgcn_mbcnt_hi((uint32_t)(live >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)live, 0));
+    tb[r] = start - S;
+    extra(r);
+  }
+  for (int g0 = 0; g0 < T; g0 += 4096) {  // wave-uniform: 64 words of 64 elements
+    wm[lane] = 0ull;
     wave_sync();
-    for (int f0 = 0; f0 < T; f0 += 64 * U) {  // wave-uniform
-      int col[U];
-      V bv[U], va[U];
+    const int b = S - 1 - g0;
+    if (len > 0 && S > 0 && b >= 0 && b < 4096) atomicOr(&wm[b >> 6], 1ull << (b & 63));
+    wave_sync();
+    const unsigned long long m = wm[lane];
+    const int pc = __popcll(m);
+    const int before = __popcll(__builtin_amdgcn_ballot_w64(len > 0 && S > 0 && b < 0));
+    const int ex = before + wave_incl_scan_dpp(pc) - pc;
+    const int words = min(64, (T - g0 + 63) >> 6);
+    for (int w = 0; w < words; w += U) {
+      int64_t at[U];
+      int j[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int f = f0 + u * 64 + lane;
-        int jj = 0;  // largest jj with whS[jj] <= f
-#pragma unroll
-        for (int step = 32; step >= 1; step >>= 1)
-          if (whS[jj + step] <= f) jj += step;  // jj + step <= 63
-        const int64_t at = f < T ? whb0[jj] + (f - whS[jj]) : 0;  // lanes past T: unused read of B's first entry
-        col[u] = Bidx[at];
-        bv[u] = Bval[at];
-        va[u] = whva[jj];
+        const int wu = min(w + u, 63);
+        const uint64_t mw = (uint64_t)readlane64((int64_t)m, wu);
+        const int f = g0 + 64 * (w + u) + lane;
+        const bool ok = w + u < words && f < T;
+        const int o = __builtin_amdgcn_readlane(ex, wu) +
+                      __builtin_amdgcn_mbcnt_hi((uint32_t)(mw >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mw, 0));
+        j[u] = ok ? o : 0;
+        at[u] = ok ? tb[j[u]] + f : -1;
       }
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (f0 + u * 64 + lane < T) {
-          const int o = (int)(col[u] - c0);
-          atomicOr(&bm[o >> 5], 1u << (o & 31));
-          lds_add(&dv[o], va[u] * bv[u]);
-        }
+      body(at, j);
     }
-    wave_sync();  // this wave's tables are rewritten by its next chunk
   }
-  // products of the short entries, from the range's bucket
-  const int64_t q0 = soff[item], q1 = soff[item + 1];
-  for (int64_t q = q0 + t; q < q1; q += NT) {
-    const int o = (int)(scol[q] - c0);
-    atomicOr(&bm[o >> 5], 1u << (o & 31));
-    lds_add(&dv[o], sval[q]);
+  wave_sync();  // the tables are rewritten by the wave's next entries
+}
+
+// A row whose windows of `wide` ranges would hold more than 1/kHubFine of all products each: it is
+// counted range by range.
+constexpr int kHubFine = 1024;
+__device__ __forceinline__ bool hub_fine(int64_t P, int nrng, int wide, int64_t products) {
+  return P / ((nrng + wide - 1) / wide) > products / kHubFine;
+}
+
+// Columns per range of the hub rows: a workgroup per (row, window of SW ranges), presence bits in
+// LDS. rng_cnt[slot * nrng + range] receives the counts (0 beforehand), nnz[row] their sum. The wide
+// instance (fewer visits of the entries) leaves out the fine rows, the FINE one takes them from
+// their list: with windows of 131,072 columns alone the heaviest row of an R-MAT 20 sample would be
+// 8 workgroups' work while the other rows of the launch are long done. Windows of 16 ranges (16 KB
+// of bits) keep four workgroups on a CU; over many ranges and rows (hub_wide) the visits of the
+// entries and of the short rows, once per window, cost more than that, and 64 ranges are taken
+// (R-MAT 22: 0.84 s of symbolic pass with 16, 0.73 s with 64).
+template <int NT, int SW, bool FINE>
+__global__ __launch_bounds__(NT) void k_hub_count(
+    const int32_t* __restrict__ hub_rows, const int32_t* __restrict__ fine, int nwin, int nrng,
+    const int64_t* __restrict__ Aptr,
+    const int32_t* __restrict__ Bidx, const HubRec* __restrict__ recs, const int32_t* __restrict__ hcnt,
+    const int32_t* __restrict__ lcnt, const int32_t* __restrict__ span, const int32_t* __restrict__ band, int64_t nb1,
+    const int32_t* __restrict__ hub_slot, int32_t* __restrict__ rng_cnt, int64_t* __restrict__ nnz) {
+  constexpr int W = SW * kHubRange;
+  constexpr int NWORD = W / 32;
+  constexpr int WPT = NWORD > NT ? NWORD / NT : 1;  // bitmap words per thread, in one range
+  constexpr int RT = kHubRange / 32 / WPT;          // threads that count one range
+  constexpr int U = 4;
+  constexpr int RL = RT < 32 ? RT : 32;             // of them, lanes that add up before the LDS add
+  static_assert(NT % 64 == 0 && (NWORD % NT == 0 || NT % NWORD == 0) && RT >= 1, "a thread's words lie in one range");
+  __shared__ __align__(16) uint32_t bm[NWORD];
+  __shared__ int64_t tb[NT];
+  __shared__ unsigned long long wm[NT];
+  __shared__ int rc[SW];
+  const int t = threadIdx.x, lane = t & 63;
+  const int64_t i = blockIdx.x / nwin;
+  const int w = (int)(blockIdx.x - i * nwin);
+  const int64_t j = FINE ? fine[i] : i;
+  const int row = hub_rows[j];
+  const int64_t lo = (int64_t)w * W, hi = lo + W;
+  if (span[2 * j + 1] < lo || span[2 * j] >= hi) return;
+  if (!FINE && (hub_slot[row] & kHubFineBit)) return;
+  const int64_t a0 = Aptr[row], a1 = Aptr[row + 1];
+  const int nH = hcnt[j], nL = lcnt[j];
+  for (int q = t; q < NWORD; q += NT) bm[q] = 0u;
+  if (t < SW) rc[t] = 0;
+  __syncthreads();
+  const int64_t w0 = lo >> kBandShift, w1 = min(hi >> kBandShift, nb1 - 1);
+  for (int e0 = 0; e0 < nH; e0 += NT) {  // uniform; strided, so heavy neighbours spread over the waves
+    const int e = e0 + (t >> 6) + (NT / 64) * lane;
+    int len = 0;
+    int64_t start = 0;
+    if (e < nH) {
+      const HubRec r = recs[a0 + e];
+      const int32_t* bd = band + (int64_t)r.s * nb1;
+      const int s0 = bd[w0];
+      len = bd[w1] - s0;
+      start = r.b0 + s0;
+    }
+    walk_spans<U>(lane, len, start, tb + (t & ~63), wm + (t & ~63), [](int) {},
+                  [&](const int64_t (&at)[U], const int (&)[U]) {
+                    int c[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) c[u] = Bidx[at[u] < 0 ? 0 : at[u]];
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                      if (at[u] >= 0) {
+                        const int o = (int)(c[u] - lo);
+                        atomicOr(&bm[o >> 5], 1u << (o & 31));
+                      }
+                  });
+  }
+  for (int e0 = 0; e0 < nL; e0 += NT) {  // short rows whole
+    const int e = e0 + t;
+    const HubRec r = e < nL ? recs[a1 - 1 - e] : HubRec{0, 0, 0};
+    walk_spans<U>(lane, r.s, r.b0, tb + (t & ~63), wm + (t & ~63), [](int) {},
+                  [&](const int64_t (&at)[U], const int (&)[U]) {
+                    int c[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) c[u] = Bidx[at[u] < 0 ? 0 : at[u]];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                      const int64_t o = c[u] - lo;
+                      if (at[u] >= 0 && o >= 0 && o < W) atomicOr(&bm[o >> 5], 1u << (o & 31));
+                    }
+                  });
   }
   __syncthreads();
-  const uint32_t w = t < NWORD ? bm[t] : 0u;
-  const int pc = __popc(w);
-  int tot;
-  const int pre = Group<NT>::exscan(pc, tot, sc);
-  const int64_t base = roff[item] - roff[j * nrng];
-  const int64_t out = Cptr[row] - cbase + base;
-  const int64_t c1 = Cptr[row + 1] - cbase;
-  int flags = (roff[item + 1] - roff[item] != tot) ? kErrWindow : 0;
-  uint32_t bits = w;
-  int64_t pos = out + pre;
-  while (bits) {
-    const int b = __ffs(bits) - 1;
-    bits &= bits - 1u;
-    const int o = 32 * t + b;
-    if (pos < c1) {
-      Cidx[pos] = (int)(c0 + o);
-      Cval[pos] = dv[o];
-    } else {
-      flags |= kErrWindow;
+  int pc = 0;
+#pragma unroll
+  for (int q = 0; q < WPT; ++q) pc += t * WPT < NWORD ? __popc(bm[t * WPT + q]) : 0;
+#pragma unroll
+  for (int o = RL / 2; o > 0; o >>= 1) pc += __shfl_xor(pc, o);
+  if ((lane & (RL - 1)) == 0 && pc) atomicAdd(&rc[t / RT], pc);
+  __syncthreads();
+  if (t < SW) {
+    const int r = w * SW + t;
+    if (r < nrng && rc[t]) {
+      rng_cnt[j * nrng + r] = rc[t];
+      atomicAdd((unsigned long long*)&nnz[row], (unsigned long long)rc[t]);
     }
-    ++pos;
   }
-  flags = wave_reduce_dpp(flags, OpOr());
-  if ((t & 63) == 0 && flags) atomicOr(err, flags);
+}
+
+// Workgroups per listed row for its short entries.
+__global__ void k_hub_bucket_chunks(const int32_t* __restrict__ rows, int64_t n, const int32_t* __restrict__ hub_slot,
+                                    const int32_t* __restrict__ lcnt, int64_t* __restrict__ cnt) {
+  for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (int64_t)gridDim.x * blockDim.x) {
+    const int hs = hub_slot[rows[j]];
+    cnt[j] = hs >= 0 ? (lcnt[hs & kHubSlotMask] + kHubBucketChunk - 1) / kHubBucketChunk : 0;
+  }
+}
+
+// Products of the short entries per (row, range). WRITE = false adds their counts to scnt (0
+// beforehand). WRITE = true puts them into the buckets at soff, the scan of scnt: a workgroup
+// counts its own, takes its places off scnt (which runs down to 0), and writes.
+template <typename V, bool WRITE>
+__global__ __launch_bounds__(256) void k_hub_bucket(
+    const int32_t* __restrict__ rows, int64_t n, const int64_t* __restrict__ coff, const int64_t* __restrict__ Aptr,
+    const V* __restrict__ Aval, const int32_t* __restrict__ Bidx, const V* __restrict__ Bval,
+    const HubRec* __restrict__ recs, const int32_t* __restrict__ hub_slot, const int32_t* __restrict__ lcnt, int nrng,
+    int64_t* __restrict__ scnt, const int64_t* __restrict__ soff, int32_t* __restrict__ scol, V* __restrict__ sval,
+    const int* __restrict__ err) {
+  constexpr int NT = 256, U = 4;
+  extern __shared__ unsigned long long lc[];  // nrng counts, then places
+  __shared__ int64_t tb[NT];
+  __shared__ V tva[NT];
+  __shared__ unsigned long long wm[NT];
+  if (WRITE && (*err & kErrCapacity)) return;  // the buckets (or C) are smaller than this structure needs
+  const int64_t q = blockIdx.x;
+  if (q >= coff[n]) return;  // the grid is a bound
+  const int64_t j = chunk_owner(coff, n, q);
+  const int row = rows[j], hs = hub_slot[row] & kHubSlotMask;
+  const int t = threadIdx.x, lane = t & 63;
+  const int64_t a0 = Aptr[row], a1 = Aptr[row + 1];
+  const int l0 = (int)(q - coff[j]) * kHubBucketChunk, l1 = min(l0 + kHubBucketChunk, lcnt[hs]);
+  for (int r = t; r < nrng; r += NT) lc[r] = 0ull;
+  __syncthreads();
+  for (int e0 = l0; e0 < l1; e0 += NT) {
+    const HubRec r = e0 + t < l1 ? recs[a1 - 1 - (e0 + t)] : HubRec{0, 0, 0};
+    walk_spans<U>(lane, r.s, r.b0, tb + (t & ~63), wm + (t & ~63), [](int) {},
+                  [&](const int64_t (&at)[U], const int (&)[U]) {
+                    int c[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) c[u] = Bidx[at[u] < 0 ? 0 : at[u]];
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                      if (at[u] >= 0) atomicAdd(&lc[c[u] >> kHubRangeShift], 1ull);
+                  });
+  }
+  __syncthreads();
+  for (int r = t; r < nrng; r += NT) {
+    const unsigned long long c = lc[r];
+    if (!c) continue;
+    unsigned long long* g = (unsigned long long*)&scnt[j * nrng + r];
+    if (WRITE) lc[r] = (unsigned long long)soff[j * nrng + r] + atomicAdd(g, 0ull - c) - c;
+    else atomicAdd(g, c);
+  }
+  if (!WRITE) return;
+  __syncthreads();
+  V* wva = tva + (t & ~63);
+  for (int e0 = l0; e0 < l1; e0 += NT) {
+    const HubRec r = e0 + t < l1 ? recs[a1 - 1 - (e0 + t)] : HubRec{0, 0, 0};
+    const V va = e0 + t < l1 ? Aval[a0 + r.e] : V(0);
+    walk_spans<U>(lane, r.s, r.b0, tb + (t & ~63), wm + (t & ~63), [&](int k) { wva[k] = va; },
+                  [&](const int64_t (&at)[U], const int (&jj)[U]) {
+                    int c[U];
+                    V p[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                      const int64_t x = at[u] < 0 ? 0 : at[u];
+                      c[u] = Bidx[x];
+                      p[u] = wva[jj[u]] * Bval[x];
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                      if (at[u] >= 0) {
+                        const int64_t pos = (int64_t)atomicAdd(&lc[c[u] >> kHubRangeShift], 1ull);
+                        scol[pos] = c[u];
+                        sval[pos] = p[u];
+                      }
+                  });
+  }
+}
+
+// What a range workgroup needs to know of its row, in one 32-byte load: A entries [a0, a1), where the
+// row's output starts, banded and short entries.
+struct HubRow {
+  int64_t a0, a1, out;
+  int32_t nH, nL;
+};
+static_assert(sizeof(HubRow) == 32, "one load");
+
+// One (row, range) item per workgroup: the range's values, emitted from info.out + roff[item] -
+// roff[first item of the row] on, with roff[item + 1] - roff[item] columns expected. soff null: no
+// buckets, the short rows are read here.
+//
+// Bound by the latency of an item's chain (row, records, band ends, gathers, stores), so two
+// workgroups share a CU (77 KB of LDS each) and nothing else is kept in LDS: a column is present
+// when its sum is no longer -0.0, the initial value, which no sum reaches (products of -0.0 are
+// made +0.0 first), so there is no bitmap to OR (127 clocks a wave for 64 neighbouring columns) and
+// a thread emits the sums it reads. The sums are FP64 for FP32 operands too: ds_add_f32 takes 194
+// clocks a wave, ds_add_f64 9 to 21 (and the rounding is better).
+template <typename V, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_hub_range(
+    const HubRow* __restrict__ info, int nrng, const V* __restrict__ Aval, const int32_t* __restrict__ Bidx,
+    const V* __restrict__ Bval, const int32_t* __restrict__ band, int64_t nb1, const HubRec* __restrict__ recs,
+    const int64_t* __restrict__ soff, const int32_t* __restrict__ scol, const V* __restrict__ sval,
+    const int64_t* __restrict__ roff, int32_t* __restrict__ Cidx, V* __restrict__ Cval, int* __restrict__ err) {
+  constexpr int NW = NT / 64;
+  constexpr int U = 4;
+  constexpr int PT = kHubRange / NT;  // columns per thread
+  static_assert(NT % 64 == 0 && kHubRange % NT == 0 && PT * NW <= 128, "shape");
+  __shared__ __align__(16) double dv[kHubRange];
+  __shared__ int64_t tb[NT];
+  __shared__ double tva[NT];
+  __shared__ unsigned long long wm[NT];
+  __shared__ int wcnt[128];
+  const int64_t item = blockIdx.x;
+  const int64_t j = item / nrng;
+  const int64_t r0 = roff[item], nexp = roff[item + 1] - r0, rfirst = roff[j * nrng];
+  const HubRow row = info[j];
+  // a range without columns (by the symbolic count) holds no product: nothing to add or emit
+  if (nexp == 0) return;
+  if (*err & kErrCapacity) return;  // the buckets or C are smaller than this structure needs
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int64_t c0 = (item - j * nrng) << kHubRangeShift;
+  const int64_t w0 = c0 >> kBandShift;
+  const int64_t w1 = min(w0 + kHubRangeBands, nb1 - 1);
+  int64_t* wtb = tb + (t & ~63);
+  double* wva = tva + (t & ~63);
+  unsigned long long* wwm = wm + (t & ~63);
+#pragma unroll
+  for (int q = 0; q < PT / 2; ++q) reinterpret_cast<double2*>(dv)[t + q * NT] = make_double2(-0.0, -0.0);
+  __syncthreads();
+  auto add = [&](int o, double p) { lds_add(&dv[o], p + 0.0); };  // -0.0 + 0.0 is +0.0
+  // products of the banded entries in this range: chunks of NT entries, each wave taking 64 of
+  // them, strided, so the heaviest (which lie together) spread over the waves
+  for (int e0 = 0; e0 < row.nH; e0 += NT) {  // uniform
+    const int e = e0 + wv + NW * lane;
+    int len = 0;
+    int64_t start = 0;
+    double va = 0.0;
+    if (e < row.nH) {
+      const HubRec q = recs[row.a0 + e];
+      const int32_t* bd = band + (int64_t)q.s * nb1;
+      const int s0 = bd[w0];
+      len = bd[w1] - s0;
+      start = q.b0 + s0;
+      va = (double)Aval[row.a0 + q.e];
+    }
+    walk_spans<U>(lane, len, start, wtb, wwm, [&](int k) { wva[k] = va; },
+                  [&](const int64_t (&at)[U], const int (&jj)[U]) {
+                    int c[U];
+                    V b[U];
+                    double av[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                      const int64_t p = at[u] < 0 ? 0 : at[u];
+                      c[u] = Bidx[p];
+                      b[u] = Bval[p];
+                      av[u] = wva[jj[u]];
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                      if (at[u] >= 0) add((int)(c[u] - c0), av[u] * (double)b[u]);
+                  });
+  }
+  // products of the short entries: the range's bucket, or its part of the rows themselves
+  if (soff) {
+    const int64_t q1 = soff[item + 1];
+    for (int64_t q = soff[item] + t; q < q1; q += NT) add((int)(scol[q] - c0), (double)sval[q]);
+  } else {
+    for (int e0 = 0; e0 < row.nL; e0 += NT) {  // uniform
+      const int e = e0 + wv + NW * lane;
+      const HubRec q = e < row.nL ? recs[row.a1 - 1 - e] : HubRec{0, 0, 0};
+      const double va = e < row.nL ? (double)Aval[row.a0 + q.e] : 0.0;
+      walk_spans<U>(lane, q.s, q.b0, wtb, wwm, [&](int k) { wva[k] = va; },
+                    [&](const int64_t (&at)[U], const int (&jj)[U]) {
+                      int c[U];
+                      V b[U];
+                      double av[U];
+#pragma unroll
+                      for (int u = 0; u < U; ++u) {
+                        const int64_t p = at[u] < 0 ? 0 : at[u];
+                        c[u] = Bidx[p];
+                        b[u] = Bval[p];
+                        av[u] = wva[jj[u]];
+                      }
+#pragma unroll
+                      for (int u = 0; u < U; ++u) {
+                        const int64_t o = c[u] - c0;
+                        if (at[u] >= 0 && o >= 0 && o < kHubRange) add((int)o, av[u] * (double)b[u]);
+                      }
+                    });
+    }
+  }
+  __syncthreads();
+  // emission, a lane per column: a wave's stores lie side by side
+  double v[PT];
+  uint64_t m[PT];
+#pragma unroll
+  for (int q = 0; q < PT; ++q) {
+    v[q] = dv[t + q * NT];
+    m[q] = __builtin_amdgcn_ballot_w64(__double_as_longlong(v[q]) != (long long)0x8000000000000000ull);
+    if (lane == 0) wcnt[q * NW + wv] = __popcll(m[q]);
+  }
+  __syncthreads();
+  if (wv == 0) {  // exclusive scan of the 128 counts in place; the total goes to flags
+    const int x0 = 2 * lane < PT * NW ? wcnt[2 * lane] : 0, x1 = 2 * lane + 1 < PT * NW ? wcnt[2 * lane + 1] : 0;
+    const int incl = wave_incl_scan_dpp(x0 + x1);
+    wcnt[2 * lane] = incl - x0 - x1;
+    wcnt[2 * lane + 1] = incl - x1;
+    if (lane == 63 && (int64_t)incl != nexp) atomicOr(err, kErrWindow);
+  }
+  __syncthreads();
+  const int64_t out = row.out + r0 - rfirst;
+#pragma unroll
+  for (int q = 0; q < PT; ++q) {
+    const int k = wcnt[q * NW + wv] + __builtin_amdgcn_mbcnt_hi((uint32_t)(m[q] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m[q], 0));
+    if ((m[q] >> lane & 1ull) && k < nexp) {
+      Cidx[out + k] = (int)(c0 + t + q * NT);
+      Cval[out + k] = (V)v[q];
+    }
+  }
 }
 
 // ------------------------------------------------------------------------------------
@@ -3183,13 +3468,12 @@ int symbolic_groups_per_wg(const KernelShape& k) {
 
 void launch_symbolic(const KernelShape& k, const int32_t* rows, const int64_t* pbeg, const int64_t* pend,
                      int64_t nrows_hint, int grid, const Mat& A, const Mat& B, int64_t* nnz, int64_t* cursor,
-                     int* err, hipStream_t s, const int32_t* hub_slot, int32_t* rng_cnt, int nrng) {
+                     int* err, hipStream_t s, const int32_t* hub_slot) {
   const int gpb = symbolic_groups_per_wg(k);
-  if (k.T == 0 || k.T == kHubShape) {  // the symbolic pass counts hub rows with the long-row windows
+  if (k.T == 0) {
     const dim3 gr(grid_for(nrows_hint, gpb, grid));
     hipLaunchKernelGGL((k_symbolic_long<1024, kSymLongW, kLongG>), gr, dim3(1024), 0, s, rows, pbeg, pend, A.ptr,
-                       A.bstart, A.blen, B.idx, nnz, cursor, err, hub_slot, rng_cnt, nrng, A.idx, B.hslot, B.band,
-                       B.nb1);
+                       A.bstart, A.blen, B.idx, nnz, cursor, err, hub_slot, A.idx, B.hslot, B.band, B.nb1);
     return;
   }
 #define X(T_, NT_, G_)                                                                                         \
@@ -3260,73 +3544,139 @@ void launch_numeric(int dtype, const KernelShape& k, const int32_t* rows, const 
 }
 
 int hub_ranges(int64_t ncols) { return (int)((ncols + kHubRange - 1) >> kHubRangeShift); }
+bool hub_buckets_used(int64_t ncols) { return hub_ranges(ncols) > kHubWhole; }
 
-__global__ void k_hub_flags(const int32_t* __restrict__ rows, int64_t n, const int64_t* __restrict__ Aptr,
-                            int64_t* __restrict__ flag) {
-  for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (int64_t)gridDim.x * blockDim.x) {
+// A wave per long row. The rule counts the ranges between the row's first and last column, over at
+// most kHubEntries of its entries (rows of more are hub rows anyway).
+__global__ __launch_bounds__(256) void k_hub_flags(const int32_t* __restrict__ rows, int64_t n,
+                                                   const int64_t* __restrict__ Aptr, const int64_t* __restrict__ P,
+                                                   const int64_t* __restrict__ bstart, const int32_t* __restrict__ blen,
+                                                   const int32_t* __restrict__ Bidx, int64_t per_range, int wide,
+                                                   int64_t products, int64_t* __restrict__ flag) {
+  const int lane = threadIdx.x & 63;
+  for (int64_t j = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); j < n; j += (int64_t)gridDim.x * 4) {
     const int r = rows[j];
-    flag[j] = Aptr[r + 1] - Aptr[r] > kHubEntries ? 1 : 0;
+    const int64_t a0 = Aptr[r], nA = Aptr[r + 1] - a0, p = P[r];
+    const int m = (int)min(nA, kHubEntries);
+    int cmin = INT_MAX, cmax = -1;
+    for (int e = lane; e < m; e += 64) {
+      const int64_t ka = a0 + e * nA / m;
+      const int L = blen[ka];
+      if (L <= 0) continue;
+      cmin = min(cmin, Bidx[bstart[ka]]);
+      cmax = max(cmax, Bidx[bstart[ka] + L - 1]);
+    }
+    cmin = wave_reduce_dpp(cmin, OpMin());
+    cmax = wave_reduce_dpp(cmax, OpMax());
+    if (lane == 0) {
+      const int nrng = cmax >= cmin ? (cmax >> kHubRangeShift) - (cmin >> kHubRangeShift) + 1 : 1;
+      const bool hub = hub_row(nA, p, nrng, per_range);
+      const bool fine = hub && hub_fine(p, nrng, wide, products);
+      flag[j] = (hub ? 1 : 0) + (fine ? kHubFineOne : 0);
+    }
   }
 }
 
 __global__ void k_hub_slots(const int32_t* __restrict__ rows, int64_t n, const int64_t* __restrict__ flag,
-                            const int64_t* __restrict__ pos, int32_t* __restrict__ hub_slot) {
-  for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (int64_t)gridDim.x * blockDim.x)
-    if (flag[j]) hub_slot[rows[j]] = (int32_t)pos[j];
+                            const int64_t* __restrict__ pos, const int64_t* __restrict__ Aptr,
+                            int32_t* __restrict__ hub_slot, int32_t* __restrict__ hub_rows, int32_t* __restrict__ fine) {
+  for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (int64_t)gridDim.x * blockDim.x) {
+    if (!flag[j]) continue;
+    const int r = rows[j];
+    const int32_t sl = (int32_t)(pos[j] & (kHubFineOne - 1));
+    const bool is_fine = flag[j] >= kHubFineOne;
+    hub_slot[r] = sl | (Aptr[r + 1] - Aptr[r] > kHubEntries ? kHubMany : 0) | (is_fine ? kHubFineBit : 0);
+    hub_rows[sl] = r;
+    if (is_fine) fine[pos[j] >> kHubFineShift] = sl;
+  }
 }
 
 __global__ void k_hub_gather_counts(const int32_t* __restrict__ rows, int64_t n, int nrng,
-                                    const int32_t* __restrict__ hub_slot, const int32_t* __restrict__ rng_cnt,
-                                    int64_t* __restrict__ rcnt) {
+                                    const int32_t* __restrict__ hub_slot, const int32_t* __restrict__ hcnt,
+                                    const int32_t* __restrict__ lcnt, const int32_t* __restrict__ rng_cnt,
+                                    const int64_t* __restrict__ Aptr, const int64_t* __restrict__ Cptr, int64_t cbase,
+                                    int64_t* __restrict__ rcnt, HubRow* __restrict__ info) {
   const int64_t items = n * nrng;
   for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < items; q += (int64_t)gridDim.x * blockDim.x) {
     const int64_t j = q / nrng;
     const int r = (int)(q - j * nrng);
+    const int row = rows[j], hs = hub_slot[row];
     // a row without a slot (only if a captured pipeline's operands changed structure) has none
-    const int hs = hub_slot[rows[j]];
-    rcnt[q] = hs >= 0 ? rng_cnt[(int64_t)hs * nrng + r] : 0;
+    rcnt[q] = hs >= 0 ? rng_cnt[(int64_t)(hs & kHubSlotMask) * nrng + r] : 0;
+    if (r == 0)
+      info[j] = HubRow{Aptr[row], Aptr[row + 1], Cptr[row] - cbase, hs >= 0 ? hcnt[hs & kHubSlotMask] : 0,
+                       hs >= 0 ? lcnt[hs & kHubSlotMask] : 0};
   }
 }
 
-void launch_hub_flags(const int32_t* rows, int64_t n, const int64_t* Aptr, int64_t* flag, hipStream_t s) {
+void launch_hub_flags(const int32_t* rows, int64_t n, const Mat& A, const Mat& B, const int64_t* P, int64_t per_range,
+                      int wide, int64_t products, int64_t* flag, hipStream_t s) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_hub_flags, dim3(fill_grid(n)), dim3(256), 0, s, rows, n, Aptr, flag);
+  hipLaunchKernelGGL(k_hub_flags, dim3(fill_grid(64 * n)), dim3(256), 0, s, rows, n, A.ptr, P, A.bstart, A.blen, B.idx,
+                     per_range, wide, products, flag);
 }
-void launch_hub_slots(const int32_t* rows, int64_t n, const int64_t* flag, const int64_t* pos, int32_t* hub_slot,
-                      hipStream_t s) {
+void launch_hub_slots(const int32_t* rows, int64_t n, const Mat& A, const int64_t* flag, const int64_t* pos,
+                      const HubWork& h, hipStream_t s) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_hub_slots, dim3(fill_grid(n)), dim3(256), 0, s, rows, n, flag, pos, hub_slot);
+  hipLaunchKernelGGL(k_hub_slots, dim3(fill_grid(n)), dim3(256), 0, s, rows, n, flag, pos, A.ptr, h.slot, h.rows, h.fine);
 }
-void launch_hub_gather_counts(const int32_t* rows, int64_t n, int nrng, const int32_t* hub_slot,
-                              const int32_t* rng_cnt, int64_t* rcnt, hipStream_t s) {
+void launch_hub_gather_counts(const HubWork& h, const int32_t* rows, int64_t n, const Mat& A, const Mat& B,
+                              const int64_t* Cptr, int64_t cbase, int64_t* rcnt, hipStream_t s) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_hub_gather_counts, dim3(fill_grid(n * nrng)), dim3(256), 0, s, rows, n, nrng, hub_slot, rng_cnt,
-                     rcnt);
+  const int nrng = hub_ranges(B.ncols);
+  hipLaunchKernelGGL(k_hub_gather_counts, dim3(fill_grid(n * nrng)), dim3(256), 0, s, rows, n, nrng, h.slot, h.hcnt,
+                     h.lcnt, h.rng_cnt, A.ptr, Cptr, cbase, rcnt, (HubRow*)h.info);
 }
 
-void launch_hub_prepare(const int32_t* rows, int64_t nh, const Mat& A, const Mat& B, int nrng, int64_t* scnt,
-                        int32_t* hlist, int32_t* hcount, hipStream_t s) {
-  if (nh <= 0) return;
-  hipLaunchKernelGGL(k_hub_prepare<256>, dim3((unsigned)nh), dim3(256), (size_t)nrng * sizeof(int), s, rows, A.ptr,
-                     A.idx, A.bstart, A.blen, B.idx, B.hslot, nrng, scnt, hlist, hcount);
+void launch_hub_split(const HubWork& h, const Mat& A, const Mat& B, const int64_t* P, int64_t key_lim, int64_t* nnz,
+                      int* many, hipStream_t s) {
+  if (h.n <= 0) return;
+  hipLaunchKernelGGL(k_hub_chunks, dim3(fill_grid(h.n)), dim3(256), 0, s, h.rows, h.n, A.ptr, P, B.ncols, key_lim,
+                     h.coff, h.hcnt, h.lcnt, h.span, nnz, many);
+  launch_exclusive_scan(h.coff, h.coff, h.n, h.tmp, s);
+  // every row has at most one partly filled chunk
+  hipLaunchKernelGGL(k_hub_split, dim3((unsigned)(A.nnz / kHubChunk + h.n)), dim3(kHubSplitNT), 0, s, h.rows, h.n,
+                     h.coff, A.ptr, A.idx, A.bstart, A.blen, B.idx, B.hslot, (HubRec*)h.recs, h.hcnt, h.lcnt, h.span);
 }
 
-void launch_hub_scatter(int dtype, const int32_t* rows, int64_t nh, const Mat& A, const Mat& B, int nrng,
-                        const int64_t* soff, int32_t* scol, void* sval, const int* err, hipStream_t s) {
-  if (nh <= 0) return;
-  const size_t lds = (size_t)nrng * sizeof(unsigned long long);
-  if (dtype == 1)
-    hipLaunchKernelGGL((k_hub_scatter<double, 256>), dim3((unsigned)nh), dim3(256), lds, s, rows, A.ptr, A.idx,
-                       A.bstart, A.blen, (const double*)A.val, B.idx, (const double*)B.val, B.hslot, nrng, soff, scol,
-                       (double*)sval, err);
-  else
-    hipLaunchKernelGGL((k_hub_scatter<float, 256>), dim3((unsigned)nh), dim3(256), lds, s, rows, A.ptr, A.idx,
-                       A.bstart, A.blen, (const float*)A.val, B.idx, (const float*)B.val, B.hslot, nrng, soff, scol,
-                       (float*)sval, err);
+// Launches of n rows x nwin windows in groups of fewer than 2^32 work-items: go(first row, rows).
+template <typename F>
+static void row_groups(int64_t n, int nwin, int nt, F&& go) {
+  const int64_t per = std::max<int64_t>(1, (((int64_t)1 << 32) / nt - 1) / nwin);
+  for (int64_t j0 = 0; j0 < n; j0 += per) go(j0, std::min(per, n - j0));
+}
+
+int hub_wide(int64_t ncols, int64_t nlong) { return hub_ranges(ncols) > 64 && nlong >= 8192 ? 64 : 16; }
+
+template <int SW>
+static void launch_hub_count_wide(const HubWork& h, const Mat& A, const Mat& B, int64_t* nnz, hipStream_t s) {
+  constexpr int NT = 512;
+  const int nrng = hub_ranges(B.ncols), nwin = (nrng + SW - 1) / SW;
+  row_groups(h.n, nwin, NT, [&](int64_t j0, int64_t nj) {
+    hipLaunchKernelGGL((k_hub_count<NT, SW, false>), dim3((unsigned)(nj * nwin)), dim3(NT), 0, s, h.rows + j0, nullptr,
+                       nwin, nrng, A.ptr, B.idx, (const HubRec*)h.recs, h.hcnt + j0, h.lcnt + j0, h.span + 2 * j0,
+                       B.band, B.nb1, h.slot, h.rng_cnt + j0 * nrng, nnz);
+  });
+}
+
+void launch_hub_count(const HubWork& h, const Mat& A, const Mat& B, int64_t* nnz, hipStream_t s) {
+  if (h.n <= 0) return;
+  constexpr int NTF = 1024;
+  const int nrng = hub_ranges(B.ncols);
+  launch_fill_i32(h.rng_cnt, h.n * nrng, 0, s);
+  if (h.nfine < h.n) {
+    if (h.wide == 64) launch_hub_count_wide<64>(h, A, B, nnz, s);
+    else launch_hub_count_wide<16>(h, A, B, nnz, s);
+  }
+  row_groups(h.nfine, nrng, NTF, [&](int64_t j0, int64_t nj) {
+    hipLaunchKernelGGL((k_hub_count<NTF, 1, true>), dim3((unsigned)(nj * nrng)), dim3(NTF), 0, s, h.rows, h.fine + j0,
+                       nrng, nrng, A.ptr, B.idx, (const HubRec*)h.recs, h.hcnt, h.lcnt, h.span, B.band, B.nb1, h.slot,
+                       h.rng_cnt, nnz);
+  });
 }
 
 // Bucket capacity check of the hub path inside a captured pipeline: more short products than the
-// buckets hold flags the capacity bit, on which the scatter and range kernels write nothing.
+// buckets hold flags the capacity bit, on which the bucket and range kernels write nothing.
 __global__ void k_hub_guard(const int64_t* __restrict__ total, int64_t cap, int* __restrict__ err) {
   if (*total > cap) atomicOr(err, kErrCapacity);
 }
@@ -3335,35 +3685,65 @@ void launch_hub_guard(const int64_t* total, int64_t cap, int* err, hipStream_t s
   hipLaunchKernelGGL(k_hub_guard, dim3(1), dim3(1), 0, s, total, cap, err);
 }
 
-// One workgroup per (row, range) item; a launch holds fewer than 2^32 work-items, so rows go in
-// groups of at most (2^32 / 1024 - 1) / nrng, each launch with its rows' slices of the per-row
-// and per-item arrays.
 template <typename V>
-static void launch_hub_range_t(const int32_t* rows, int64_t nh, int nrng, const Mat& A, const Mat& B,
-                               const int32_t* hlist, const int32_t* hcount, const int64_t* soff, const int32_t* scol,
-                               const V* sval, const int64_t* roff, const int64_t* Cptr, int64_t cbase, int32_t* Cidx,
-                               V* Cval, int* err, hipStream_t s) {
-  constexpr int64_t kMaxItems = ((int64_t)1 << 32) / 1024 - 1;
-  const int64_t per = std::max<int64_t>(1, kMaxItems / nrng);
-  for (int64_t j0 = 0; j0 < nh; j0 += per) {
-    const int64_t nj = std::min(per, nh - j0), i0 = j0 * nrng;
-    hipLaunchKernelGGL((k_hub_range<V, 1024>), dim3((unsigned)(nj * nrng)), dim3(1024), 0, s, rows + j0, nrng, A.ptr,
-                       A.idx, A.bstart, (const V*)A.val, B.idx, (const V*)B.val, B.hslot, B.band, B.nb1, hlist,
-                       hcount + j0, soff + i0, scol, sval, roff + i0, Cptr, cbase, Cidx, Cval, err);
-  }
+static void launch_hub_bucket_t(bool write, const HubWork& h, const int32_t* rows, int64_t n, const Mat& A, const Mat& B,
+                                int64_t* scnt, const int64_t* soff, int32_t* scol, V* sval, const int* err,
+                                hipStream_t s) {
+  const int nrng = hub_ranges(B.ncols);
+  const size_t lds = (size_t)nrng * sizeof(unsigned long long);
+  const dim3 gr((unsigned)(A.nnz / kHubBucketChunk + n));  // a row has at most one partly filled chunk
+  const V *Av = (const V*)A.val, *Bv = (const V*)B.val;
+  if (write)
+    hipLaunchKernelGGL((k_hub_bucket<V, true>), gr, dim3(256), lds, s, rows, n, h.boff, A.ptr, Av, B.idx, Bv,
+                       (const HubRec*)h.recs, h.slot, h.lcnt, nrng, scnt, soff, scol, sval, err);
+  else
+    hipLaunchKernelGGL((k_hub_bucket<V, false>), gr, dim3(256), lds, s, rows, n, h.boff, A.ptr, Av, B.idx, Bv,
+                       (const HubRec*)h.recs, h.slot, h.lcnt, nrng, scnt, soff, scol, sval, err);
 }
 
-void launch_hub_range(int dtype, const int32_t* rows, int64_t nh, int nrng, const Mat& A, const Mat& B,
-                      const int32_t* hlist, const int32_t* hcount, const int64_t* soff, const int32_t* scol,
-                      const void* sval, const int64_t* roff, const int64_t* Cptr, int64_t cbase, int32_t* Cidx,
-                      void* Cval, int* err, hipStream_t s) {
+void launch_hub_bucket_count(const HubWork& h, const int32_t* rows, int64_t n, const Mat& A, const Mat& B,
+                             int64_t* scnt, hipStream_t s) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_hub_bucket_chunks, dim3(fill_grid(n)), dim3(256), 0, s, rows, n, h.slot, h.lcnt, h.boff);
+  launch_exclusive_scan(h.boff, h.boff, n, h.tmp, s);
+  launch_fill_i64(scnt, n * hub_ranges(B.ncols), 0, s);
+  launch_hub_bucket_t<float>(false, h, rows, n, A, B, scnt, nullptr, nullptr, nullptr, nullptr, s);
+}
+
+void launch_hub_bucket_fill(int dtype, const HubWork& h, const int32_t* rows, int64_t n, const Mat& A, const Mat& B,
+                            int64_t* scnt, const int64_t* soff, int32_t* scol, void* sval, const int* err,
+                            hipStream_t s) {
+  if (n <= 0) return;
+  if (dtype == 1)
+    launch_hub_bucket_t<double>(true, h, rows, n, A, B, scnt, soff, scol, (double*)sval, err, s);
+  else
+    launch_hub_bucket_t<float>(true, h, rows, n, A, B, scnt, soff, scol, (float*)sval, err, s);
+}
+
+// One workgroup per (row, range) item, rows in groups with their slices of the per-row and per-item
+// arrays.
+template <typename V>
+static void launch_hub_range_t(const HubWork& h, int64_t nh, const Mat& A, const Mat& B, const int64_t* soff,
+                               const int32_t* scol, const V* sval, const int64_t* roff, int32_t* Cidx, V* Cval, int* err,
+                               hipStream_t s) {
+  constexpr int NT = 512;
+  const int nrng = hub_ranges(B.ncols);
+  row_groups(nh, nrng, NT, [&](int64_t j0, int64_t nj) {
+    const int64_t i0 = j0 * nrng;
+    hipLaunchKernelGGL((k_hub_range<V, NT>), dim3((unsigned)(nj * nrng)), dim3(NT), 0, s, (const HubRow*)h.info + j0,
+                       nrng, (const V*)A.val, B.idx, (const V*)B.val, B.band, B.nb1, (const HubRec*)h.recs,
+                       soff ? soff + i0 : nullptr, scol, sval, roff + i0, Cidx, Cval, err);
+  });
+}
+
+void launch_hub_range(int dtype, const HubWork& h, int64_t nh, const Mat& A, const Mat& B, const int64_t* soff,
+                      const int32_t* scol, const void* sval, const int64_t* roff, int32_t* Cidx, void* Cval, int* err,
+                      hipStream_t s) {
   if (nh <= 0) return;
   if (dtype == 1)
-    launch_hub_range_t<double>(rows, nh, nrng, A, B, hlist, hcount, soff, scol, (const double*)sval, roff, Cptr, cbase,
-                               Cidx, (double*)Cval, err, s);
+    launch_hub_range_t<double>(h, nh, A, B, soff, scol, (const double*)sval, roff, Cidx, (double*)Cval, err, s);
   else
-    launch_hub_range_t<float>(rows, nh, nrng, A, B, hlist, hcount, soff, scol, (const float*)sval, roff, Cptr, cbase,
-                              Cidx, (float*)Cval, err, s);
+    launch_hub_range_t<float>(h, nh, A, B, soff, scol, (const float*)sval, roff, Cidx, (float*)Cval, err, s);
 }
 
 template <typename V>

@@ -45,7 +45,7 @@ struct Tables {
 // least hub_min_cols columns.
 Tables default_tables(int g_small, int g_big, double load, int top = 8192, int64_t hub_min_cols = 0);
 
-// Whether the numeric binning routes hub rows (long rows of more than kHubEntries A entries) to
+// Whether the numeric binning routes hub rows (the long rows that hub_row picks) to
 // the hub category for a problem of ncols columns.
 inline bool hub_enabled(const Tables& t, int64_t ncols) { return ncols >= t.hub_min_cols; }
 
@@ -57,11 +57,10 @@ struct Work {
   int32_t *rows_sym, *rows_num, *blen;
   int* err;
   int64_t nr, nwg;
-  // hub rows (all null / 0: none): their slots and per-range column counts for the symbolic pass
-  // and the numeric binning, and the enqueue of their range kernels after the numeric categories
+  // hub rows (all null: none): their slots for the symbolic pass and the numeric binning, the
+  // enqueue of their symbolic kernels, and of their range kernels after the numeric categories
   const int32_t* hub_slot = nullptr;
-  int32_t* hub_rng = nullptr;
-  int nrng = 0;
+  void (*hub_sym_fn)(void* arg, hipStream_t s) = nullptr;
   void (*hub_fn)(void* arg, const int64_t* Cptr, int32_t* Cidx, void* Cval, hipStream_t s) = nullptr;
   void* hub_arg = nullptr;
 };

@@ -57,3 +57,40 @@ def test_device_view_of_a_run_of_rows(gpu_ok):
     e0, e1 = int(M.ptr[r0]), int(M.ptr[r1])
     S = dbd_amd.CSR(M.ptr[r0:r1 + 1] - e0, M.idx[e0:e1], M.val[e0:e1], (r1 - r0, 500))
     compare(C, reference(S, B), np.float64, "rows of a larger matrix")
+
+
+# hub rows (long rows in column ranges of 8192): widths at the edges of a range, of the 131072-column
+# count window and of the bucketed form (more than 8 ranges); rows of many entries (over several
+# split chunks of 1024), rows of few entries with many products, and long rows that stay in the windows
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("ncols", [8191, 8192, 8193, 40000, 65536, 65537, 131072, 131073, 300001])
+def test_hub_rows_in_ranges(gpu_ok, ncols, dtype):
+    rng = np.random.default_rng(ncols)
+    blen = np.concatenate([rng.integers(0, 64, 2400), rng.integers(64, 600, 500), [min(ncols, 9000)] * 8, [63, 64, 65]])
+    B = from_lengths(rng.permutation(blen), ncols, 11, dtype)
+    A = from_lengths([1, 2900, 1025, 1024, 700, 300, 0, 60, 12, 2049], B.shape[0], 12, dtype)
+    _, _, info = check_product(A, B, what=f"{ncols} columns")
+    # rows of many entries are hub rows (a row of at most 8192 columns fits a hash table)
+    assert info["num_rows"][-1] >= 3 if ncols > 8192 else info["num_rows"][-1] == 0
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("ncols", [20000, 100000])
+def test_hub_sums_of_special_values(gpu_ok, ncols, dtype):
+    """Entries whose sum is zero, -0.0, denormal, infinite or NaN are entries of C like any other.
+    The values are small multiples of one number, so every order of summation gives the same sum."""
+    rng = np.random.default_rng(13)
+    B = from_lengths(rng.permutation([10, 40, 63, 64, 900, 2500] * 60), ncols, 14, dtype)
+    A = from_lengths([360, 200, 2, 360], B.shape[0], 15, dtype)
+    A.val[:] = rng.choice([1.0, -1.0, 0.0, -0.0], A.nnz)
+    tiny = np.finfo(dtype).smallest_subnormal
+    for what, vals in (("zeros", [0.0, -0.0]), ("signs", [1.0, -1.0, 0.0, -0.0]), ("subnormal", [tiny, -tiny, 0.0, -0.0]),
+                       ("infinite", [1.0, np.inf, 2.0, 0.0]), ("nan", [1.0, np.nan, -0.0, 3.0])):
+        B.val[:] = rng.choice(np.array(vals, dtype), B.nnz)
+        Cptr, Cidx, Cval, _ = reference(A, B)
+        with dbd_amd.Context(dtype=dtype) as ctx:
+            ctx.set_operands(A, B)
+            ctx.run("compute")
+            C = ctx.result()
+        assert np.array_equal(C.ptr, Cptr) and np.array_equal(C.idx, Cidx), what
+        assert np.array_equal(C.val, Cval.astype(dtype), equal_nan=True), what
