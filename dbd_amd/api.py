@@ -326,8 +326,8 @@ class Context:
 
     @staticmethod
     def table_knobs(table_id: int) -> dict:
-        """Knobs of candidate table `table_id` (table 0 is the default): lanes per B row in small /
-        large hash tables, the load limit, the largest numeric LDS table, and the column count from
+        """Knobs of candidate table `table_id` (table 0 is the default): lanes per B row in one-wave /
+        workgroup hash tables, the load limit, the largest numeric LDS table, and the column count from
         which hub rows take the numeric hub kernels."""
         d = dbd_table_desc()
         check(lib.dbd_table_knobs(table_id, C.byref(d)))

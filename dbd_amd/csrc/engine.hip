@@ -121,7 +121,7 @@ Tables dbd::default_tables(int g_small, int g_big, double load, int top, int64_t
   t.num_k[n++] = {0, 0, 0};
   for (int i = 0; i < 8 && Ts[i] <= top; ++i) {
     t.num_ct.lim[n] = (int64_t)(Ts[i] * load);
-    t.num_k[n++] = {Ts[i], NTs[i], Ts[i] <= 1024 ? g_small : g_big};
+    t.num_k[n++] = {Ts[i], NTs[i], NTs[i] <= 64 ? g_small : g_big};
   }
   t.num_ct.lim[n] = INT64_MAX;
   t.num_k[n++] = {0, 256, 16};  // long rows

@@ -314,6 +314,64 @@ __device__ __forceinline__ void clear_table(int t, int* K, V* H) {
   }
 }
 
+// Element-parallel walk over the spans of up to 64 entries, one per lane of a wave (`len` elements at
+// `start`): extra(rank) stores what else the elements need of this lane's entry, at its rank among
+// the entries with elements, and body(at, j) takes U elements per lane, element u of them at
+// position at[u], of the entry of rank j[u] (at[u] < 0: none). The owner of a flattened element is
+// not searched: the entries set a bit where their elements begin (bit S - 1 for the entry that
+// starts at S >= 1, in words of 64 elements), and an element's owner is the number of bits before it,
+// one mbcnt on a mask that readlane makes wave-uniform (a bisection over 64 starts costs 6
+// dependent LDS reads per element). l: LDS of this wave's own. With w0 and wstep several waves that
+// hold the same entries share the elements, U words at a time.
+constexpr int kSpanWords = 32;
+struct SpanLds {
+  int64_t tb[64];
+  unsigned long long wm[kSpanWords];
+};
+template <int U, typename X, typename F>
+__device__ __forceinline__ void walk_spans(int lane, int len, int64_t start, SpanLds& l, X&& extra, F&& body, int w0 = 0,
+                                           int wstep = U) {
+  const uint64_t live = __builtin_amdgcn_ballot_w64(len > 0);
+  if (!live) return;
+  const int incl = wave_incl_scan_dpp(len);
+  const int S = incl - len;
+  const int T = __builtin_amdgcn_readlane(incl, 63);
+  if (len > 0) {
+    const int r = __builtin_amdgcn_mbcnt_hi((uint32_t)(live >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)live, 0));
+    l.tb[r] = start - S;
+    extra(r);
+  }
+  for (int g0 = 0; g0 < T; g0 += 64 * kSpanWords) {  // wave-uniform
+    if (lane < kSpanWords) l.wm[lane] = 0ull;
+    wave_sync();
+    const int b = S - 1 - g0;
+    if (len > 0 && S > 0 && b >= 0 && b < 64 * kSpanWords) atomicOr(&l.wm[b >> 6], 1ull << (b & 63));
+    wave_sync();
+    const unsigned long long m = lane < kSpanWords ? l.wm[lane] : 0ull;
+    const int pc = __popcll(m);
+    const int before = __popcll(__builtin_amdgcn_ballot_w64(len > 0 && S > 0 && b < 0));
+    const int ex = before + wave_incl_scan_dpp(pc) - pc;
+    const int words = min(kSpanWords, (T - g0 + 63) >> 6);
+    for (int w = w0; w < words; w += wstep) {
+      int64_t at[U];
+      int j[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int wu = min(w + u, 63);
+        const uint64_t mw = (uint64_t)readlane64((int64_t)m, wu);
+        const int f = g0 + 64 * (w + u) + lane;
+        const bool ok = w + u < words && f < T;
+        const int o = __builtin_amdgcn_readlane(ex, wu) +
+                      __builtin_amdgcn_mbcnt_hi((uint32_t)(mw >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mw, 0));
+        j[u] = ok ? o : 0;
+        at[u] = ok ? l.tb[j[u]] + f : -1;
+      }
+      body(at, j);
+    }
+  }
+  wave_sync();  // the tables are rewritten by the wave's next entries
+}
+
 // Descriptor of the A entry a lane holds: start and length of the selected B row, A's value.
 template <typename V>
 struct ADesc {
@@ -424,40 +482,69 @@ __device__ __forceinline__ void gather_step(Step<U, V>& st, int lane, int e0, in
   });
 }
 
-// Hand a gathered step to the sink: f.batch(c[U], v[U]) for the first G entries of each B row
-// (c < 0 marks no product), f.one(c, v) for the tails of B rows longer than G; v = A_ik * B_kj.
+// Hand a gathered step to the sink: f.batch(c[U], v[U]) for the first G entries of each B row (c < 0
+// marks no product), v = A_ik * B_kj. What B rows longer than G have left is walk_tails'.
 template <int G, int U, bool WITHV, typename V, typename F, int S = 0>
-__device__ __forceinline__ void consume_step(const Step<U, V>& st, int lane, int e0, int cnt, const ADesc<V>& d,
-                                             const int32_t* __restrict__ Bidx, const V* __restrict__ Bval, F& f) {
+__device__ __forceinline__ void consume_step(const Step<U, V>& st, int lane, int e0, int cnt, const ADesc<V>& d, F& f) {
   const int sg = lane / G, lg = lane % G;
-  int pl[U], c[U];
-  V v[U], pv[U];
-  bool tail = false;
+  int c[U];
+  V v[U];
   static_for<U>([&](auto uc) {
     constexpr int u = decltype(uc)::value;
     const int e = step_entry<G, S>(e0, u, sg);
     const int er = min(e0 + u, 63);
     const int lv = ebcast<G, 4 * S + (u & 3)>(d.len, er);
-    if constexpr (WITHV) pv[u] = ebcastv<G, 4 * S + (u & 3)>(d.va, er);
-    else pv[u] = V(0);
-    pl[u] = e < cnt ? lv : 0;
-    const bool has = lg < pl[u];
+    V pv = V(0);
+    if constexpr (WITHV) pv = ebcastv<G, 4 * S + (u & 3)>(d.va, er);
+    const bool has = e < cnt && lg < lv;
     c[u] = has ? st.c[u] : -1;
-    v[u] = (WITHV && has) ? pv[u] * st.bv[u] : V(0);
-    tail |= pl[u] > G;
+    v[u] = (WITHV && has) ? pv * st.bv[u] : V(0);
   });
   f.template batch<U>(c, v);
-  if (__builtin_amdgcn_ballot_w64(tail)) {  // B rows longer than G: the rest of them, one by one
-    static_for<U>([&](auto uc) {
-      constexpr int u = decltype(uc)::value;
-      const int64_t pb = ebcast64<G, 4 * S + (u & 3)>(d.b0, min(e0 + u, 63));
-      for (int q = G + lg; q < pl[u]; q += G) {
-        const int64_t p = pb + q;
-        f.one(Bidx[p], WITHV ? pv[u] * Bval[p] : V(0));
-      }
-    });
-    wait_vmem();
-  }
+}
+
+// LDS of one wave for walk_flat: the spans' tables and A's values by rank.
+template <typename V, bool WITHV>
+struct FlatLds {
+  SpanLds sp;
+  V va[WITHV ? 64 : 1];
+};
+
+// The products of one entry per lane (`len` elements of its B row from `start` on, A's value va),
+// element-parallel over the wave.
+template <int U, bool WITHV, typename V, typename F>
+__device__ __forceinline__ void walk_flat(int lane, int len, int64_t start, V va, const int32_t* __restrict__ Bidx,
+                                          const V* __restrict__ Bval, FlatLds<V, WITHV>& l, F& f, int w0 = 0,
+                                          int wstep = U) {
+  walk_spans<U>(lane, len, start, l.sp,
+                [&](int r) {
+                  if (WITHV) l.va[r] = va;
+                },
+                [&](const int64_t (&at)[U], const int (&j)[U]) {
+                  int c[U];
+                  V v[U];
+#pragma unroll
+                  for (int u = 0; u < U; ++u) {
+                    const int64_t p = at[u] < 0 ? 0 : at[u];
+                    c[u] = Bidx[p];
+                    v[u] = WITHV ? l.va[WITHV ? j[u] : 0] * Bval[p] : V(0);
+                  }
+#pragma unroll
+                  for (int u = 0; u < U; ++u) c[u] = at[u] < 0 ? -1 : c[u];
+                  f.template batch<U>(c, v);
+                },
+                w0, wstep);
+}
+
+// The rest of the B rows longer than G of one chunk's entries. One by one, G lanes each, they were a
+// chain of dependent loads: half of the time of rows whose B rows average 33 entries.
+template <int G, int U, bool WITHV, typename V, typename F>
+__device__ __forceinline__ void walk_tails(int lane, int cnt, const ADesc<V>& d, const int32_t* __restrict__ Bidx,
+                                           const V* __restrict__ Bval, FlatLds<V, WITHV>& l, F& f) {
+  const int len = desc_slot<G>(lane) < cnt ? max(d.len - G, 0) : 0;
+  if (!__builtin_amdgcn_ballot_w64(len > 0)) return;
+  walk_flat<U, WITHV>(lane, len, d.b0 + G, d.va, Bidx, Bval, l, f);
+  wait_vmem();
 }
 
 template <int G, int U, bool WITHV, typename V, typename F, int S>
@@ -465,7 +552,7 @@ __device__ __forceinline__ void walk_step(int lane, int e0, int cnt, const ADesc
                                           const int32_t* __restrict__ Bidx, const V* __restrict__ Bval, F& f) {
   Step<U, V> st;
   gather_step<G, U, WITHV, V, S>(st, lane, e0, cnt, d, Bidx, Bval);
-  consume_step<G, U, WITHV, V, F, S>(st, lane, e0, cnt, d, Bidx, Bval, f);
+  consume_step<G, U, WITHV, V, F, S>(st, lane, e0, cnt, d, f);
 }
 
 // All products of `cnt` (<= 64) A entries of one chunk, from entry `from` on (a multiple of a
@@ -491,7 +578,7 @@ __device__ __forceinline__ void for_row_products_pre(int t, int64_t a0, int64_t 
                                                      const int64_t* __restrict__ bstart,
                                                      const int32_t* __restrict__ blen, const V* __restrict__ Aval,
                                                      const int32_t* __restrict__ Bidx, const V* __restrict__ Bval,
-                                                     F& f, const Step<U, V>* step0 = nullptr) {
+                                                     FlatLds<V, WITHV>& l, F& f, const Step<U, V>* step0 = nullptr) {
   static_assert(NT >= 64, "wave-level walk");
   constexpr int STEP = G == 16 ? 16 : U;  // entries per step
   const int lane = t & 63, wv = t >> 6;
@@ -500,29 +587,55 @@ __device__ __forceinline__ void for_row_products_pre(int t, int64_t a0, int64_t 
     const int cnt = (int)min((int64_t)64, a1 - base);
     int from = 0;
     if (step0) {  // the caller already issued the first step's gathers
-      consume_step<G, U, WITHV, V, F, 0>(*step0, lane, 0, cnt, first, Bidx, Bval, f);
+      consume_step<G, U, WITHV, V, F, 0>(*step0, lane, 0, cnt, first, f);
       from = STEP;
     }
     if (from < cnt) {
       walk_chunk<G, U, WITHV, V>(lane, cnt, first, Bidx, Bval, f, from);
       if (step0) wait_vmem();
     }
+    walk_tails<G, U, WITHV>(lane, cnt, first, Bidx, Bval, l, f);
   }
   if (base + NT < a1) {
     for (base += NT; base < a1; base += NT) {
       const ADesc<V> d = load_desc<G, WITHV, V>(base, a1, lane, bstart, blen, Aval);
-      walk_chunk<G, U, WITHV, V>(lane, (int)min((int64_t)64, a1 - base), d, Bidx, Bval, f);
+      const int cnt = (int)min((int64_t)64, a1 - base);
+      walk_chunk<G, U, WITHV, V>(lane, cnt, d, Bidx, Bval, f);
+      walk_tails<G, U, WITHV>(lane, cnt, d, Bidx, Bval, l, f);
     }
     if (step0) wait_vmem();
   }
 }
 
+// All products of one row for a workgroup of NT > 64 threads. G = 16: 16 lanes per B row, 64 entries
+// per wave. G = 64: element-parallel; a row of up to 64 entries is every wave's, which share its
+// elements (dealt 64 entries per wave such a row was one wave's work), a row of more is dealt entry
+// by entry over the waves.
 template <int NT, int G, int U, bool WITHV, typename V, typename F>
 __device__ __forceinline__ void for_row_products(int t, int64_t a0, int64_t a1, const int64_t* __restrict__ bstart,
                                                  const int32_t* __restrict__ blen, const V* __restrict__ Aval,
-                                                 const int32_t* __restrict__ Bidx, const V* __restrict__ Bval, F& f) {
-  const ADesc<V> first = load_desc<G, WITHV, V>(a0 + 64 * (t >> 6), a1, t & 63, bstart, blen, Aval);
-  for_row_products_pre<NT, G, U, WITHV, V>(t, a0, a1, first, bstart, blen, Aval, Bidx, Bval, f);
+                                                 const int32_t* __restrict__ Bidx, const V* __restrict__ Bval,
+                                                 FlatLds<V, WITHV>& l, F& f) {
+  if constexpr (G == 64) {
+    constexpr int NW = NT / 64;
+    const int lane = t & 63, wv = t >> 6;
+    const bool shared = a1 - a0 <= 64;  // uniform
+    for (int64_t base = a0; base < a1; base += NT) {
+      const int64_t ka = base + (shared ? lane : wv + NW * lane);
+      int len = 0;
+      int64_t start = 0;
+      V va = V(0);
+      if (ka < a1) {
+        len = blen[ka];
+        start = bstart[ka];
+        va = WITHV ? Aval[ka] : V(0);
+      }
+      walk_flat<U, WITHV>(lane, len, start, va, Bidx, Bval, l, f, shared ? wv * U : 0, shared ? NW * U : U);
+    }
+  } else {
+    const ADesc<V> first = load_desc<G, WITHV, V>(a0 + 64 * (t >> 6), a1, t & 63, bstart, blen, Aval);
+    for_row_products_pre<NT, G, U, WITHV, V>(t, a0, a1, first, bstart, blen, Aval, Bidx, Bval, l, f);
+  }
 }
 
 // Workgroups are dispatched round-robin over the 8 XCDs (each with its own L2). When the grid
@@ -1050,8 +1163,10 @@ void launch_bin_scatter(const int64_t* key, int64_t n, int64_t cap, const CatTab
 template <int NT>
 constexpr int wg_of() { return NT <= 64 ? 256 : NT; }
 
+// One-wave rows: 7 waves per SIMD (72 VGPRs); a seventh of the waves fewer is 6 % of the pass on
+// 2,000,000 rows of 256 products.
 template <int T, int NT, int G>
-__global__ __launch_bounds__(wg_of<NT>()) void k_symbolic_hash(
+__global__ __launch_bounds__(wg_of<NT>()) __attribute__((amdgpu_waves_per_eu(NT == 64 ? 7 : 1))) void k_symbolic_hash(
     const int32_t* __restrict__ rows, const int64_t* __restrict__ pbeg, const int64_t* __restrict__ pend,
     const int64_t* __restrict__ Aptr, const int64_t* __restrict__ bstart, const int32_t* __restrict__ blen,
     const int32_t* __restrict__ Bidx, int64_t* __restrict__ nnz, int* __restrict__ err) {
@@ -1060,8 +1175,10 @@ __global__ __launch_bounds__(wg_of<NT>()) void k_symbolic_hash(
   static_assert(NT % G == 0 && T % NT == 0, "shape");
   __shared__ int hk[GPB][T];
   __shared__ int sc[GPB][NT > 64 ? NT / 64 : 1];
+  __shared__ FlatLds<float, false> fl[WG / 64];
   const int t = threadIdx.x % NT;
   const int g = __builtin_amdgcn_readfirstlane(threadIdx.x / NT);  // wave-uniform: keep row state scalar
+  FlatLds<float, false>& wl = fl[__builtin_amdgcn_readfirstlane(threadIdx.x / 64)];
   int* K = hk[g];
   const int64_t beg = *pbeg, end = *pend;
   if constexpr (NT == 64) {
@@ -1081,7 +1198,7 @@ __global__ __launch_bounds__(wg_of<NT>()) void k_symbolic_hash(
       wave_sync();
       HashSink<T, float, false, false> sk{K, nullptr};
       for_row_products_pre<64, G, 4, false, float>(t, rp.a0, rp.a1, rp.d, bstart, blen, (const float*)nullptr, Bidx,
-                                                   (const float*)nullptr, sk, &st0);
+                                                   (const float*)nullptr, wl, sk, &st0);
       // the next row's first gathers (past the last row: the current row again, unused)
       gather_step<G, 4, false, float>(st0, t, 0, (int)min((int64_t)64, rp.na1 - rp.na0), rp.nd, Bidx,
                                       (const float*)nullptr);
@@ -1109,7 +1226,7 @@ __global__ __launch_bounds__(wg_of<NT>()) void k_symbolic_hash(
     const int64_t a0 = Aptr[row], a1 = Aptr[row + 1];
     HashSink<T, float, false, false> sk{K, nullptr};
     for_row_products<NT, G, 4, false, float>(t, a0, a1, bstart, blen, (const float*)nullptr, Bidx,
-                                             (const float*)nullptr, sk);
+                                             (const float*)nullptr, wl, sk);
     const int cnt = Group<NT>::reduce(sk.created, OpAdd(), sc[g]);
     const int bad = Group<NT>::reduce(sk.bad, OpMax(), sc[g]);
     if (t == 0) {
@@ -1530,58 +1647,6 @@ __global__ __launch_bounds__(kHubSplitNT) void k_hub_split(
   }
 }
 
-// Element-parallel walk of one wave over the spans of up to 64 entries, one per lane (`len`
-// elements at `start`): extra(rank) stores what else the elements need of this lane's entry, at its
-// rank among the entries with elements, and body(at, j) takes U elements per lane, element u of
-// them at position at[u], of the entry of rank j[u] (at[u] < 0: none). The owner of a flattened
-// element is not searched: the entries set a bit where their elements begin (word 64-wide, bit
-// S - 1 for the entry that starts at S >= 1), and an element's owner is the number of bits before
-// it, one mbcnt on a mask that readlane makes wave-uniform (a bisection over 64 starts costs 6
-// dependent LDS reads per element). tb and wm: 64 entries of LDS of this wave's own.
-template <int U, typename X, typename F>
-__device__ __forceinline__ void walk_spans(int lane, int len, int64_t start, int64_t* tb, unsigned long long* wm,
-                                           X&& extra, F&& body) {
-  const uint64_t live = __builtin_amdgcn_ballot_w64(len > 0);
-  if (!live) return;
-  const int incl = wave_incl_scan_dpp(len);
-  const int S = incl - len;
-  const int T = __builtin_amdgcn_readlane(incl, 63);
-  if (len > 0) {
-    const int r = __builtin_amdgcn_mbcnt_hi((uint32_t)(live >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)live, 0));
-    tb[r] = start - S;
-    extra(r);
-  }
-  for (int g0 = 0; g0 < T; g0 += 4096) {  // wave-uniform: 64 words of 64 elements
-    wm[lane] = 0ull;
-    wave_sync();
-    const int b = S - 1 - g0;
-    if (len > 0 && S > 0 && b >= 0 && b < 4096) atomicOr(&wm[b >> 6], 1ull << (b & 63));
-    wave_sync();
-    const unsigned long long m = wm[lane];
-    const int pc = __popcll(m);
-    const int before = __popcll(__builtin_amdgcn_ballot_w64(len > 0 && S > 0 && b < 0));
-    const int ex = before + wave_incl_scan_dpp(pc) - pc;
-    const int words = min(64, (T - g0 + 63) >> 6);
-    for (int w = 0; w < words; w += U) {
-      int64_t at[U];
-      int j[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int wu = min(w + u, 63);
-        const uint64_t mw = (uint64_t)readlane64((int64_t)m, wu);
-        const int f = g0 + 64 * (w + u) + lane;
-        const bool ok = w + u < words && f < T;
-        const int o = __builtin_amdgcn_readlane(ex, wu) +
-                      __builtin_amdgcn_mbcnt_hi((uint32_t)(mw >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mw, 0));
-        j[u] = ok ? o : 0;
-        at[u] = ok ? tb[j[u]] + f : -1;
-      }
-      body(at, j);
-    }
-  }
-  wave_sync();  // the tables are rewritten by the wave's next entries
-}
-
 // A row whose windows of `wide` ranges would hold more than 1/kHubFine of all products each: it is
 // counted range by range.
 constexpr int kHubFine = 1024;
@@ -1612,8 +1677,7 @@ __global__ __launch_bounds__(NT) void k_hub_count(
   constexpr int RL = RT < 32 ? RT : 32;             // of them, lanes that add up before the LDS add
   static_assert(NT % 64 == 0 && (NWORD % NT == 0 || NT % NWORD == 0) && RT >= 1, "a thread's words lie in one range");
   __shared__ __align__(16) uint32_t bm[NWORD];
-  __shared__ int64_t tb[NT];
-  __shared__ unsigned long long wm[NT];
+  __shared__ SpanLds sl[NT / 64];
   __shared__ int rc[SW];
   const int t = threadIdx.x, lane = t & 63;
   const int64_t i = blockIdx.x / nwin;
@@ -1640,7 +1704,7 @@ __global__ __launch_bounds__(NT) void k_hub_count(
       len = bd[w1] - s0;
       start = r.b0 + s0;
     }
-    walk_spans<U>(lane, len, start, tb + (t & ~63), wm + (t & ~63), [](int) {},
+    walk_spans<U>(lane, len, start, sl[t >> 6], [](int) {},
                   [&](const int64_t (&at)[U], const int (&)[U]) {
                     int c[U];
 #pragma unroll
@@ -1656,7 +1720,7 @@ __global__ __launch_bounds__(NT) void k_hub_count(
   for (int e0 = 0; e0 < nL; e0 += NT) {  // short rows whole
     const int e = e0 + t;
     const HubRec r = e < nL ? recs[a1 - 1 - e] : HubRec{0, 0, 0};
-    walk_spans<U>(lane, r.s, r.b0, tb + (t & ~63), wm + (t & ~63), [](int) {},
+    walk_spans<U>(lane, r.s, r.b0, sl[t >> 6], [](int) {},
                   [&](const int64_t (&at)[U], const int (&)[U]) {
                     int c[U];
 #pragma unroll
@@ -1706,9 +1770,8 @@ __global__ __launch_bounds__(256) void k_hub_bucket(
     const int* __restrict__ err) {
   constexpr int NT = 256, U = 4;
   extern __shared__ unsigned long long lc[];  // nrng counts, then places
-  __shared__ int64_t tb[NT];
+  __shared__ SpanLds sl[NT / 64];
   __shared__ V tva[NT];
-  __shared__ unsigned long long wm[NT];
   if (WRITE && (*err & kErrCapacity)) return;  // the buckets (or C) are smaller than this structure needs
   const int64_t q = blockIdx.x;
   if (q >= coff[n]) return;  // the grid is a bound
@@ -1721,7 +1784,7 @@ __global__ __launch_bounds__(256) void k_hub_bucket(
   __syncthreads();
   for (int e0 = l0; e0 < l1; e0 += NT) {
     const HubRec r = e0 + t < l1 ? recs[a1 - 1 - (e0 + t)] : HubRec{0, 0, 0};
-    walk_spans<U>(lane, r.s, r.b0, tb + (t & ~63), wm + (t & ~63), [](int) {},
+    walk_spans<U>(lane, r.s, r.b0, sl[t >> 6], [](int) {},
                   [&](const int64_t (&at)[U], const int (&)[U]) {
                     int c[U];
 #pragma unroll
@@ -1745,7 +1808,7 @@ __global__ __launch_bounds__(256) void k_hub_bucket(
   for (int e0 = l0; e0 < l1; e0 += NT) {
     const HubRec r = e0 + t < l1 ? recs[a1 - 1 - (e0 + t)] : HubRec{0, 0, 0};
     const V va = e0 + t < l1 ? Aval[a0 + r.e] : V(0);
-    walk_spans<U>(lane, r.s, r.b0, tb + (t & ~63), wm + (t & ~63), [&](int k) { wva[k] = va; },
+    walk_spans<U>(lane, r.s, r.b0, sl[t >> 6], [&](int k) { wva[k] = va; },
                   [&](const int64_t (&at)[U], const int (&jj)[U]) {
                     int c[U];
                     V p[U];
@@ -1795,9 +1858,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   constexpr int PT = kHubRange / NT;  // columns per thread
   static_assert(NT % 64 == 0 && kHubRange % NT == 0 && PT * NW <= 128, "shape");
   __shared__ __align__(16) double dv[kHubRange];
-  __shared__ int64_t tb[NT];
+  __shared__ SpanLds sl[NW];
   __shared__ double tva[NT];
-  __shared__ unsigned long long wm[NT];
   __shared__ int wcnt[128];
   const int64_t item = blockIdx.x;
   const int64_t j = item / nrng;
@@ -1810,9 +1872,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   const int64_t c0 = (item - j * nrng) << kHubRangeShift;
   const int64_t w0 = c0 >> kBandShift;
   const int64_t w1 = min(w0 + kHubRangeBands, nb1 - 1);
-  int64_t* wtb = tb + (t & ~63);
   double* wva = tva + (t & ~63);
-  unsigned long long* wwm = wm + (t & ~63);
 #pragma unroll
   for (int q = 0; q < PT / 2; ++q) reinterpret_cast<double2*>(dv)[t + q * NT] = make_double2(-0.0, -0.0);
   __syncthreads();
@@ -1832,7 +1892,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       start = q.b0 + s0;
       va = (double)Aval[row.a0 + q.e];
     }
-    walk_spans<U>(lane, len, start, wtb, wwm, [&](int k) { wva[k] = va; },
+    walk_spans<U>(lane, len, start, sl[wv], [&](int k) { wva[k] = va; },
                   [&](const int64_t (&at)[U], const int (&jj)[U]) {
                     int c[U];
                     V b[U];
@@ -1858,7 +1918,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       const int e = e0 + wv + NW * lane;
       const HubRec q = e < row.nL ? recs[row.a1 - 1 - e] : HubRec{0, 0, 0};
       const double va = e < row.nL ? (double)Aval[row.a0 + q.e] : 0.0;
-      walk_spans<U>(lane, q.s, q.b0, wtb, wwm, [&](int k) { wva[k] = va; },
+      walk_spans<U>(lane, q.s, q.b0, sl[wv], [&](int k) { wva[k] = va; },
                     [&](const int64_t (&at)[U], const int (&jj)[U]) {
                       int c[U];
                       V b[U];
@@ -2107,8 +2167,10 @@ __device__ __forceinline__ void numeric_hash_body(
   __shared__ V hv[GPB][T];
   __shared__ int bc[GPB][WAVE ? 1 : NB + 1];
   __shared__ int sc[GPB][NT > 64 ? NT / 64 : 1];
+  __shared__ FlatLds<V, true> fl[WG / 64];
   const int t = threadIdx.x % NT;
   const int g = __builtin_amdgcn_readfirstlane(threadIdx.x / NT);  // wave-uniform
+  FlatLds<V, true>& wl = fl[__builtin_amdgcn_readfirstlane(threadIdx.x / 64)];
   int* K = hk[g];
   V* H = hv[g];
   const int64_t beg = *pbeg, end = *pend;
@@ -2189,7 +2251,7 @@ __device__ __forceinline__ void numeric_hash_body(
       clear_table<T, V>(t, K, H);
       wave_sync();
       HashSink<T, V, true> sk{K, H};
-      for_row_products_pre<64, G, 4, true, V>(t, rp.a0, rp.a1, rp.d, bstart, blen, Aval, Bidx, Bval, sk, &st0);
+      for_row_products_pre<64, G, 4, true, V>(t, rp.a0, rp.a1, rp.d, bstart, blen, Aval, Bidx, Bval, wl, sk, &st0);
       // the next row's first gathers (past the last row: the current row again, unused); they
       // are in flight while this row is ranked and stored
       gather_step<G, 4, true, V>(st0, t, 0, (int)min((int64_t)64, rp.na1 - rp.na0), rp.nd, Bidx, Bval);
@@ -2250,7 +2312,7 @@ __device__ __forceinline__ void numeric_hash_body(
       gsync<NT>();
       const int64_t a0 = Aptr[row], a1 = Aptr[row + 1];
       HashSink<T, V, true> sk{K, H};
-      for_row_products<NT, G, 4, true, V>(t, a0, a1, bstart, blen, Aval, Bidx, Bval, sk);
+      for_row_products<NT, G, 4, true, V>(t, a0, a1, bstart, blen, Aval, Bidx, Bval, wl, sk);
       gsync<NT>();
       const int cmin = Group<NT>::reduce(sk.cmin, OpMin(), sc[g]);
       const int cmax = Group<NT>::reduce(sk.cmax, OpMax(), sc[g]);

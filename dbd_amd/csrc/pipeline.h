@@ -32,14 +32,14 @@ struct Tables {
   CatTable sym_ct, num_ct;
   KernelShape sym_k[kMaxCats], num_k[kMaxCats];
   int id = 0;
-  int g_small = 16, g_big = 64;  // lanes per A entry in tables of <= 1024 / larger slot counts
+  int g_small = 16, g_big = 64;  // lanes per A entry in one-wave / workgroup tables
   double load = 0.5;             // hash-table load limit
   int top = 8192;                // slots of the largest numeric LDS table (symbolic: twice that)
   int64_t hub_min_cols = 0;  // numeric hub category used when ncols >= this
 };
 
 // Symbolic key min(P_i, ncols), numeric key nnz_i; hash tables sized so the load stays <= `load`
-// (one-wave symbolic tables at half of that); G lanes per A entry for small / large tables; the
+// (one-wave symbolic tables at half of that); G lanes per A entry for one-wave / workgroup tables; the
 // numeric tables stop at `top` slots (4096 or 8192), the symbolic ones at 2 * top. Rows past the
 // last table are long rows; the numeric table ends with the hub category, used when B has at
 // least hub_min_cols columns.

@@ -194,8 +194,9 @@ dbd_status dbd_batch_launch(dbd_ctx* ctx, int64_t* d_Cptr, int32_t* d_Cidx, void
 dbd_status dbd_autotune(dbd_ctx* ctx, int32_t* chosen);
 /* The knobs a candidate table is built from. Table 0 is the default table. */
 typedef struct dbd_table_desc {
-  int32_t g_small;      /* lanes per B row in hash tables of up to 1024 slots (16 or 64) */
-  int32_t g_big;        /* lanes per B row in larger tables (16 or 64) */
+  int32_t g_small;      /* lanes per B row in one-wave hash tables (16 or 64) */
+  int32_t g_big;        /* lanes per B row in workgroup tables: 16, or 64 (element-parallel: the
+                           entries' products flattened over the lanes) */
   double load;          /* hash-table load limit: a table of T slots takes rows of <= load*T keys */
   int32_t top;          /* slots of the largest numeric LDS table (4096 or 8192; symbolic 2x);
                            rows beyond it take the long-row windows */
