@@ -91,6 +91,13 @@ struct HostBuf {
   T* as() const { return (T*)p; }
 };
 
+// A part of a DevBuf.
+struct View {
+  void* p = nullptr;
+  template <typename T>
+  T* as() const { return (T*)p; }
+};
+
 }  // namespace
 
 // ---- category tables -------------------------------------------------------------------
@@ -128,6 +135,8 @@ Tables dbd::default_tables(int g_small, int g_big, double load, int top, int64_t
   t.num_ct.lim[n] = INT64_MAX;  // hub rows: the long rows hub_row picks
   t.num_k[n++] = {kHubShape, 1024, 0};
   t.num_ct.n = n;
+  for (int c = t.sym_ct.n; c < kMaxCats; ++c) t.sym_ct.lim[c] = INT64_MAX;
+  for (int c = t.num_ct.n; c < kMaxCats; ++c) t.num_ct.lim[c] = INT64_MAX;
   return t;
 }
 
@@ -311,7 +320,11 @@ struct dbd_ctx {
   bool table_explicit = false;  // dbd_set_table was called: opts.tune does not override it
   bool planned = false, symb = false;
   int64_t nr = 0, nb = 0, nwg = 0;
-  DevBuf P, Pptr, nnz, Cptr, rows_sym, rows_num, cnt, offs_sym, offs_num, tmp, cursor, blk, err, bdesc_s, bdesc_l;
+  // per-row and per-nonzero workspace, one allocation (ws), and the kernels' reports (pinned)
+  DevBuf ws, cursor;
+  View P, nnz, Cptr, rows_sym, rows_num, cnt, offs_sym, offs_num, tmp, err, bdesc_s, bdesc_l;
+  HostBuf report;
+  bool err_dirty = false;  // an error was reported: the device's error word is to be cleared
   // band index of B's long rows (for the long-row window kernels), built once per operand set
   DevBuf band_hist, band_flag, band_tmp, band_slot, band_row, band;
   bool band_ready = false;
@@ -322,7 +335,8 @@ struct dbd_ctx {
   HubWork hub;
   bool hub_split = false;  // the entry records (in `cursor`) are those of the current plan
   int64_t band_minlen = 0, band_rows = 0, band_nb1 = 0;
-  std::vector<int64_t> h_blk, h_blockP, h_blockC, h_offs_num, h_sym_tot;
+  std::vector<int64_t> h_blockP, h_blockC, h_sym_tot, h_num_tot;
+  std::vector<int64_t> h_offs_num;  // numeric bin offsets by tile, copied when a run has several chunks
   dbd_plan_info info{};
 
   // outputs
@@ -341,7 +355,6 @@ struct dbd_ctx {
   int64_t batch_cap = 0;  // entries of C the batch caller allocated (exact nnz at prepare)
   // the batch's hub rows: position in the numeric bins, count, bucket capacity (from prepare)
   int64_t bh_pos0 = 0, bh_n = 0, bh_nshort = 0;
-  DevBuf g_rng;
 };
 
 namespace {
@@ -358,14 +371,27 @@ dbd_status ensure_events(dbd_ctx* c) {
   return DBD_OK;
 }
 
-// `many`: the number of hub rows of many entries, which lies beside the error word.
-dbd_status check_err(dbd_ctx* c, const char* phase, int* many = nullptr) {
-  int e[2] = {0, 0};
-  HIPCHK(hipMemcpyAsync(e, c->err.p, sizeof(e), hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
-  if (many) *many = e[1];
-  if (e[0] != 0) return set_error(DBD_ERR_INTERNAL, "%s: device consistency check failed (flags 0x%x)", phase, e[0]);
+HostReport* report(dbd_ctx* c) { return c->report.as<HostReport>(); }
+
+// The error word and the number of hub rows of many entries beside it, as the last report has them.
+dbd_status reported_err(dbd_ctx* c, const char* phase, int* many = nullptr) {
+  const int e = report(c)->err[0];
+  if (many) *many = report(c)->err[1];
+  c->err_dirty = e != 0;
+  if (e != 0) return set_error(DBD_ERR_INTERNAL, "%s: device consistency check failed (flags 0x%x)", phase, e);
   return DBD_OK;
+}
+
+dbd_status check_err(dbd_ctx* c, const char* phase) {
+  launch_report_err(c->err.as<int>(), report(c), c->st);
+  HIPCHK(hipStreamSynchronize(c->st));
+  return reported_err(c, phase);
+}
+
+// The error word is 0 but after an error (plan clears it in any case).
+void clear_err(dbd_ctx* c) {
+  if (c->err_dirty) launch_fill_i32(c->err.as<int32_t>(), 1, 0, c->st);
+  c->err_dirty = false;
 }
 
 // Whether hub rows can take the range kernels: they read B's band index for long B rows and
@@ -573,48 +599,50 @@ dbd_status plan(dbd_ctx* c) {
   const int BR = c->o.block_rows;
   c->nb = nr == 0 ? 0 : (nr - 1) / BR + 1;
   hipStream_t s = c->st;
-  CHK(c->P.ensure(8 * (size_t)(nr + 1)));
-  CHK(c->Pptr.ensure(8 * (size_t)(nr + 1)));
-  CHK(c->nnz.ensure(8 * (size_t)(nr + 1)));
-  CHK(c->Cptr.ensure(8 * (size_t)(nr + 1)));
-  CHK(c->rows_sym.ensure(4 * (size_t)(nr + 1)));
-  CHK(c->rows_num.ensure(4 * (size_t)(nr + 1)));
   const size_t ncnt = (size_t)kMaxCats * (size_t)c->nwg + 1;
-  CHK(c->cnt.ensure(8 * ncnt));
-  CHK(c->offs_sym.ensure(8 * (ncnt + 1)));
-  CHK(c->offs_num.ensure(8 * (ncnt + 1)));
-  CHK(c->tmp.ensure(8 * (size_t)scan_tmp_elems((int64_t)ncnt + nr + 1)));
-  CHK(c->blk.ensure(8 * (size_t)(std::max(c->nb, (int64_t)kMaxCats) + 2)));
-  CHK(c->err.ensure(64));  // error word, then a sink the numeric kernels write degenerate rows to
-  CHK(c->bdesc_s.ensure(8 * (size_t)(c->A.nnz + 1)));
-  // the lengths, then the row analysis' tile table
-  CHK(c->bdesc_l.ensure(4 * (size_t)(c->A.nnz + 1 + row_tiles(c->A.nnz) + 1)));
+  // the descriptors' lengths, then the row analysis' tile table; the error word, then a sink the
+  // numeric kernels write degenerate rows to
+  const struct {
+    View* v;
+    size_t bytes;
+  } parts[] = {{&c->P, 8 * (size_t)(nr + 1)},        {&c->nnz, 8 * (size_t)(nr + 1)},
+               {&c->Cptr, 8 * (size_t)(nr + 1)},     {&c->rows_sym, 4 * (size_t)(nr + 1)},
+               {&c->rows_num, 4 * (size_t)(nr + 1)}, {&c->cnt, 8 * ncnt},
+               {&c->offs_sym, 8 * (ncnt + 1)},       {&c->offs_num, 8 * (ncnt + 1)},
+               {&c->tmp, 8 * (size_t)scan_tmp_elems((int64_t)ncnt)}, {&c->err, 64},
+               {&c->bdesc_s, 8 * (size_t)(c->A.nnz + 1)},
+               {&c->bdesc_l, 4 * (size_t)(c->A.nnz + 1 + row_tiles(c->A.nnz) + 1)}};
+  size_t total = 0;
+  for (auto& q : parts) total += (q.bytes + 255) & ~(size_t)255;
+  CHK(c->ws.ensure(total));
+  total = 0;
+  for (auto& q : parts) {
+    q.v->p = c->ws.as<char>() + total;
+    total += (q.bytes + 255) & ~(size_t)255;
+  }
+  CHK(c->report.ensure(sizeof(HostReport) + 8 * (size_t)(c->nb + 1)));
   c->A.bstart = c->bdesc_s.as<int64_t>();
   c->A.blen = c->bdesc_l.as<int32_t>();
   if (c->same) c->B = c->A;
   launch_row_products(c->A, c->B, c->P.as<int64_t>(), c->nnz.as<int64_t>(), (int64_t*)c->A.bstart,
                       (int32_t*)c->A.blen, c->bdesc_l.as<int32_t>() + c->A.nnz + 1, c->err.as<int>(), s);
-  launch_exclusive_scan(c->P.as<int64_t>(), c->Pptr.as<int64_t>(), nr, c->tmp.as<int64_t>(), s);
-  launch_gather_strided(c->Pptr.as<int64_t>(), nr, BR, c->nb, c->blk.as<int64_t>(), s);
-  c->h_blk.assign((size_t)c->nb + 1, 0);
-  HIPCHK(hipMemcpyAsync(c->h_blk.data(), c->blk.p, 8 * (size_t)(c->nb + 1), hipMemcpyDeviceToHost, s));
-
-  // symbolic bins
+  // symbolic bins, and the products by block
   const CatTable& ct = c->tb.sym_ct;
-  const int64_t n_off = (int64_t)ct.n * c->nwg;
-  launch_bin_count(c->P.as<int64_t>(), nr, c->B.ncols, ct, c->cnt.as<int64_t>(), s);
-  launch_exclusive_scan(c->cnt.as<int64_t>(), c->offs_sym.as<int64_t>(), n_off, c->tmp.as<int64_t>(), s);
-  launch_bin_scatter(c->P.as<int64_t>(), nr, c->B.ncols, ct, c->offs_sym.as<int64_t>(), c->rows_sym.as<int32_t>(), s);
-  DevBuf& g = c->g_rng;
-  CHK(g.ensure(8 * (kMaxCats + 2)));
-  launch_gather_strided(c->offs_sym.as<int64_t>(), n_off, c->nwg, ct.n, g.as<int64_t>(), s);
-  c->h_sym_tot.assign((size_t)ct.n + 1, 0);
-  HIPCHK(hipMemcpyAsync(c->h_sym_tot.data(), g.p, 8 * (size_t)(ct.n + 1), hipMemcpyDeviceToHost, s));
+  HostReport& rep = *report(c);
+  if (nr == 0) memset(&rep, 0, sizeof(rep));
+  BinOut o;
+  o.host = &rep;
+  o.err = c->err.as<int>();
+  o.bt = BR / 256;
+  launch_bin(c->P.as<int64_t>(), nr, c->B.ncols, ct, c->cnt.as<int64_t>(), c->offs_sym.as<int64_t>(),
+             c->tmp.as<int64_t>(), c->rows_sym.as<int32_t>(), o, s);
   HIPCHK(hipStreamSynchronize(s));
+  c->err_dirty = false;
+  c->h_sym_tot.assign(rep.tot, rep.tot + ct.n + 1);
 
   // block table + reference criteria
   c->h_blockP.assign((size_t)c->nb, 0);
-  for (int64_t b = 0; b < c->nb; ++b) c->h_blockP[(size_t)b] = c->h_blk[(size_t)b + 1] - c->h_blk[(size_t)b];
+  for (int64_t b = 0; b < c->nb; ++b) c->h_blockP[(size_t)b] = rep.blk[b + 1] - rep.blk[b];
   dbd_plan_info& in = c->info;
   memset(&in, 0, sizeof(in));
   block_criteria(c->h_blockP.data(), c->nb, BR, &in);
@@ -643,8 +671,9 @@ dbd_status plan(dbd_ctx* c) {
 // window-kernel workspace: 16 bytes per A nonzero (cursor state of long rows)
 dbd_status ensure_cursor(dbd_ctx* c) { return c->cursor.ensure(16 * (size_t)(c->A.nnz + 1)); }
 
-// Symbolic pass over all rows -> nnz_i -> Cptr (device, ctx-owned) -> numeric bins.
-dbd_status symbolic(dbd_ctx* c) {
+// Symbolic pass over all rows -> nnz_i -> Cptr (device, ctx-owned; also into d_Cptr if given) ->
+// numeric bins.
+dbd_status symbolic(dbd_ctx* c, int64_t* d_Cptr = nullptr) {
   if (!c->planned) return set_error(DBD_ERR_STATE, "symbolic before plan");
   hipStream_t s = c->st;
   const CatTable& ct = c->tb.sym_ct;
@@ -665,34 +694,51 @@ dbd_status symbolic(dbd_ctx* c) {
                     offs + (int64_t)(k + 1) * c->nwg, n, 0, c->A, c->B, c->nnz.as<int64_t>(),
                     c->cursor.as<int64_t>(), c->err.as<int>(), s, c->hub.slot);
   }
-  launch_exclusive_scan(c->nnz.as<int64_t>(), c->Cptr.as<int64_t>(), c->nr, c->tmp.as<int64_t>(), s);
-  const int BR = c->o.block_rows;
-  launch_gather_strided(c->Cptr.as<int64_t>(), c->nr, BR, c->nb, c->blk.as<int64_t>(), s);
-  std::vector<int64_t> hb((size_t)c->nb + 1, 0);
-  HIPCHK(hipMemcpyAsync(hb.data(), c->blk.p, 8 * (size_t)(c->nb + 1), hipMemcpyDeviceToHost, s));
-  // numeric bins by exact nnz_i
+  // numeric bins by exact nnz_i, C's row pointer, and nnz(C) by block
   const CatTable& nt = c->tb.num_ct;
-  const int64_t n_off = (int64_t)nt.n * c->nwg;
-  launch_bin_count(c->nnz.as<int64_t>(), c->nr, INT64_MAX, nt, c->cnt.as<int64_t>(), s, c->hub.slot,
-                   c->err.as<int>() + 1);
-  launch_exclusive_scan(c->cnt.as<int64_t>(), c->offs_num.as<int64_t>(), n_off, c->tmp.as<int64_t>(), s);
-  launch_bin_scatter(c->nnz.as<int64_t>(), c->nr, INT64_MAX, nt, c->offs_num.as<int64_t>(), c->rows_num.as<int32_t>(),
-                     s, c->hub.slot);
-  c->h_offs_num.assign((size_t)n_off + 1, 0);
-  HIPCHK(hipMemcpyAsync(c->h_offs_num.data(), c->offs_num.p, 8 * (size_t)(n_off + 1), hipMemcpyDeviceToHost, s));
+  HostReport& rep = *report(c);
+  if (c->nr == 0) memset(&rep, 0, sizeof(rep));
+  BinOut o;
+  o.ptr = c->Cptr.as<int64_t>();
+  o.ptr2 = d_Cptr;
+  o.host = &rep;
+  o.err = c->err.as<int>();
+  o.bt = c->o.block_rows / 256;
+  launch_bin(c->nnz.as<int64_t>(), c->nr, INT64_MAX, nt, c->cnt.as<int64_t>(), c->offs_num.as<int64_t>(),
+             c->tmp.as<int64_t>(), c->rows_num.as<int32_t>(), o, s, c->hub.slot, c->err.as<int>() + 1);
+  c->h_offs_num.clear();
+  HIPCHK(hipStreamSynchronize(s));
   int many = 0;
-  CHK(check_err(c, "symbolic", &many));  // synchronises the stream
+  CHK(reported_err(c, "symbolic", &many));
+  c->h_num_tot.assign(rep.tot, rep.tot + nt.n + 1);
   c->h_blockC.assign((size_t)c->nb, 0);
-  for (int64_t b = 0; b < c->nb; ++b) c->h_blockC[(size_t)b] = hb[(size_t)b + 1] - hb[(size_t)b];
-  c->info.nnz = c->nb > 0 ? hb[(size_t)c->nb] : 0;
-  for (int k = 0; k < nt.n; ++k)
-    c->info.num_rows[k] = c->h_offs_num[(size_t)(k + 1) * c->nwg] - c->h_offs_num[(size_t)k * c->nwg];
+  for (int64_t b = 0; b < c->nb; ++b) c->h_blockC[(size_t)b] = rep.blk[b + 1] - rep.blk[b];
+  c->info.nnz = rep.blk[c->nb];
+  for (int k = 0; k < nt.n; ++k) c->info.num_rows[k] = c->h_num_tot[(size_t)k + 1] - c->h_num_tot[(size_t)k];
   if (c->hub.n > 0) {  // the report's hub category: rows of more than kHubEntries entries
     const int64_t few = c->info.num_rows[nt.n - 1] - many;
     c->info.num_rows[nt.n - 1] -= few;
     c->info.num_rows[nt.n - 2] += few;
   }
   c->symb = true;
+  return DBD_OK;
+}
+
+// First row in the list of category k's part in tiles [w0, w1), and the number of its rows: from the
+// totals for all tiles, else from the offsets by tile, copied once per symbolic pass.
+dbd_status num_part(dbd_ctx* c, int k, int64_t w0, int64_t w1, int64_t* first, int64_t* n) {
+  if (w0 == 0 && w1 == c->nwg) {
+    *first = c->h_num_tot[(size_t)k];
+    *n = c->h_num_tot[(size_t)k + 1] - *first;
+    return DBD_OK;
+  }
+  if (c->h_offs_num.empty()) {
+    c->h_offs_num.resize((size_t)c->tb.num_ct.n * (size_t)c->nwg + 1);
+    HIPCHK(hipMemcpyAsync(c->h_offs_num.data(), c->offs_num.p, 8 * c->h_offs_num.size(), hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipStreamSynchronize(c->st));
+  }
+  *first = c->h_offs_num[(size_t)k * c->nwg + w0];
+  *n = c->h_offs_num[(size_t)k * c->nwg + w1] - *first;
   return DBD_OK;
 }
 
@@ -709,10 +755,11 @@ dbd_status numeric_blocks(dbd_ctx* c, int64_t b0, int64_t b1, const int64_t* Cpt
   const bool distinct = c->info.nnz >= 0 && c->info.nnz >= c->info.products - c->info.products / 10;
   for (int k = 1; k < nt.n; ++k) {
     const int64_t i0 = (int64_t)k * c->nwg + w0, i1 = (int64_t)k * c->nwg + w1;
-    const int64_t n = c->h_offs_num[(size_t)i1] - c->h_offs_num[(size_t)i0];
+    int64_t first = 0, n = 0;
+    CHK(num_part(c, k, w0, w1, &first, &n));
     if (n <= 0) continue;
     if (c->tb.num_k[k].T == kHubShape) {  // rows with hub slots: the range kernels apply
-      CHK(hub_numeric(c, c->h_offs_num[(size_t)i0], n, Cptr, cbase, Cidx, Cval));
+      CHK(hub_numeric(c, first, n, Cptr, cbase, Cidx, Cval));
       continue;
     }
     if (c->tb.num_k[k].T == 0 || c->tb.num_k[k].T == kHubShape) CHK(ensure_cursor(c));
@@ -759,9 +806,7 @@ dbd_status make_chunks(dbd_ctx* c, int64_t cap, std::vector<Chunk>& out, const s
 
 int64_t fixed_device_bytes(dbd_ctx* c) {
   int64_t s = c->a_bytes + (c->same ? 0 : c->b_bytes);
-  s += (int64_t)c->P.bytes + c->Pptr.bytes + c->nnz.bytes + c->Cptr.bytes + c->rows_sym.bytes + c->rows_num.bytes;
-  s += (int64_t)c->cnt.bytes + c->offs_sym.bytes + c->offs_num.bytes + c->tmp.bytes + c->cursor.bytes;
-  s += (int64_t)c->bdesc_s.bytes + c->bdesc_l.bytes;
+  s += (int64_t)c->ws.bytes + c->cursor.bytes;
   s += (int64_t)c->band_hist.bytes + c->band_flag.bytes + c->band_tmp.bytes + c->band_slot.bytes + c->band_row.bytes +
        c->band.bytes + c->hub_meta.bytes + c->hub_scnt.bytes + c->hub_rcnt.bytes + c->hub_tmp.bytes +
        c->hub_scol.bytes + c->hub_sval.bytes + c->hub_slot.bytes + c->hub_flag.bytes + c->hub_rng.bytes;
@@ -1143,8 +1188,7 @@ dbd_status dbd_destroy(dbd_ctx* c) {
   if (!c) return DBD_OK;
   (void)hipStreamSynchronize(c->st);  // a null st is the default stream
   if (c->cst) (void)hipStreamSynchronize(c->cst);
-  for (auto* b : {&c->P, &c->Pptr, &c->nnz, &c->Cptr, &c->rows_sym, &c->rows_num, &c->cnt, &c->offs_sym, &c->offs_num,
-                  &c->tmp, &c->cursor, &c->blk, &c->err, &c->g_rng, &c->bdesc_s, &c->bdesc_l, &c->band_hist,
+  for (auto* b : {&c->ws, &c->cursor, &c->band_hist,
                   &c->band_flag, &c->band_tmp, &c->band_slot, &c->band_row, &c->band, &c->hub_meta, &c->hub_scnt,
                   &c->hub_rcnt, &c->hub_tmp, &c->hub_scol, &c->hub_sval, &c->hub_slot, &c->hub_flag,
                   &c->hub_rng})
@@ -1162,6 +1206,7 @@ dbd_status dbd_destroy(dbd_ctx* c) {
   for (auto e : c->ev_slot) (void)hipEventDestroy(e);
   for (auto e : {c->ev_t0, c->ev_t1, c->ev_c0, c->ev_c1})
     if (e) (void)hipEventDestroy(e);
+  c->report.release();
   c->h_cptr.release();
   c->h_idx.release();
   c->h_val.release();
@@ -1221,8 +1266,11 @@ dbd_status dbd_set_operands(dbd_ctx* c, const dbd_csr* A, const dbd_csr* B) {
   } else {
     CHK(upload(c, B, c->B, c->upB, c->b_bytes));
   }
-  HIPCHK(hipStreamSynchronize(c->st));
-  c->h2d_s = (A->location == DBD_HOST || B->location == DBD_HOST) ? now_s() - t0 : 0.0;
+  c->h2d_s = 0.0;
+  if (A->location == DBD_HOST || B->location == DBD_HOST) {  // device views are only borrowed: nothing to wait for
+    HIPCHK(hipStreamSynchronize(c->st));
+    c->h2d_s = now_s() - t0;
+  }
   c->host_ops = A->location == DBD_HOST && B->location == DBD_HOST;
   c->hostA = *A;
   c->hostB = *B;
@@ -1319,9 +1367,7 @@ dbd_status dbd_symbolic(dbd_ctx* c, int64_t* d_Cptr, int64_t* nnz_out) {
   clear_error();
   if (!c) return set_error(DBD_ERR_INVALID, "null ctx");
   if (!c->planned) CHK(plan(c));
-  CHK(symbolic(c));
-  if (d_Cptr)
-    HIPCHK(hipMemcpyAsync(d_Cptr, c->Cptr.p, 8 * (size_t)(c->nr + 1), hipMemcpyDeviceToDevice, c->st));
+  CHK(symbolic(c, d_Cptr));
   if (nnz_out) *nnz_out = c->info.nnz;
   return DBD_OK;
 }
@@ -1330,7 +1376,7 @@ dbd_status dbd_numeric(dbd_ctx* c, const int64_t* d_Cptr, int32_t* d_Cidx, void*
   clear_error();
   if (!c || !d_Cptr || (c->info.nnz > 0 && (!d_Cidx || !d_Cval))) return set_error(DBD_ERR_INVALID, "null argument");
   if (!c->symb) return set_error(DBD_ERR_STATE, "dbd_numeric before dbd_symbolic");
-  launch_fill_i32(c->err.as<int32_t>(), 1, 0, c->st);
+  clear_err(c);
   CHK(numeric_blocks(c, 0, c->nb, d_Cptr, 0, d_Cidx, d_Cval));
   return check_err(c, "numeric");
 }
@@ -1341,7 +1387,7 @@ dbd_status dbd_backward(dbd_ctx* c, const int64_t* d_Cptr, const int32_t* d_Cidx
   if (!c || !d_Cptr || !d_Cidx || !d_dC) return set_error(DBD_ERR_INVALID, "null argument");
   if (!c->symb) return set_error(DBD_ERR_STATE, "dbd_backward needs the forward plan (run dbd_symbolic first)");
   hipStream_t s = c->st;
-  launch_fill_i32(c->err.as<int32_t>(), 1, 0, s);
+  clear_err(c);
   c->hub_split = false;  // the long rows' cursors take the records' place
   if (d_dA) launch_fill_bytes0(d_dA, (int64_t)c->vsz * c->A.nnz, s);
   const CatTable& nt = c->tb.num_ct;
@@ -1352,7 +1398,7 @@ dbd_status dbd_backward(dbd_ctx* c, const int64_t* d_Cptr, const int32_t* d_Cidx
     // its rows from the end (the hub rows, the heaviest, first)
     const bool with_hub = c->tb.num_k[k].T == 0 && k + 1 < nt.n && c->tb.num_k[k + 1].T == kHubShape;
     const int64_t i0 = (int64_t)k * c->nwg, i1 = (int64_t)(k + (with_hub ? 2 : 1)) * c->nwg;
-    const int64_t n = c->h_offs_num[(size_t)i1] - c->h_offs_num[(size_t)i0];
+    const int64_t n = c->h_num_tot[(size_t)(k + (with_hub ? 2 : 1))] - c->h_num_tot[(size_t)k];
     const KernelShape ks = c->tb.num_k[k];
     if (with_hub) ++k;
     if (n <= 0) continue;
@@ -1385,18 +1431,15 @@ void dbd::enqueue_pipeline(const Work& w, const Tables& tb, Mat A, const Mat& B,
   // the analysis' tile table lies in the cursors, which the row kernels only write later
   launch_row_products(A, B, w.P, w.nnz, w.bstart, w.blen, (int32_t*)w.cursor, w.err, s);
   const CatTable& ct = tb.sym_ct;
-  launch_bin_count(w.P, nr, B.ncols, ct, w.cnt, s);
-  launch_exclusive_scan(w.cnt, w.offs_sym, (int64_t)ct.n * w.nwg, w.tmp, s);
-  launch_bin_scatter(w.P, nr, B.ncols, ct, w.offs_sym, w.rows_sym, s);
+  launch_bin(w.P, nr, B.ncols, ct, w.cnt, w.offs_sym, w.tmp, w.rows_sym, BinOut{}, s);
   if (w.hub_sym_fn) w.hub_sym_fn(w.hub_arg, s);
   for (int k = 1; k < ct.n; ++k)
     launch_symbolic(tb.sym_k[k], w.rows_sym, w.offs_sym + (int64_t)k * w.nwg, w.offs_sym + (int64_t)(k + 1) * w.nwg, 0,
                     persistent_grid(num_cu, tb.sym_k[k]), A, B, w.nnz, w.cursor, w.err, s, w.hub_slot);
-  launch_exclusive_scan(w.nnz, d_Cptr, nr, w.tmp, s);
   const CatTable& nt = tb.num_ct;
-  launch_bin_count(w.nnz, nr, INT64_MAX, nt, w.cnt, s, w.hub_slot, w.err + 1);
-  launch_exclusive_scan(w.cnt, w.offs_num, (int64_t)nt.n * w.nwg, w.tmp, s);
-  launch_bin_scatter(w.nnz, nr, INT64_MAX, nt, w.offs_num, w.rows_num, s, w.hub_slot);
+  BinOut o;
+  o.ptr = d_Cptr;
+  launch_bin(w.nnz, nr, INT64_MAX, nt, w.cnt, w.offs_num, w.tmp, w.rows_num, o, s, w.hub_slot, w.err + 1);
   launch_capacity_guard(d_Cptr + nr, cap, w.offs_num, (int64_t)nt.n * w.nwg + 1, w.err, s);
   for (int k = 1; k < nt.n; ++k) {
     if (tb.num_k[k].T == kHubShape) continue;  // the range kernels below (empty without hub slots)
@@ -1458,7 +1501,7 @@ dbd_status dbd_batch_prepare(dbd_ctx* c, const dbd_csr* A_cat, const dbd_csr* B_
   c->bh_n = c->bh_pos0 = c->bh_nshort = 0;
   const CatTable& nt = c->tb.num_ct;
   if (c->hub.n > 0 && c->tb.num_k[nt.n - 1].T == kHubShape) {
-    const int64_t p0 = c->h_offs_num[(size_t)(nt.n - 1) * c->nwg], p1 = c->h_offs_num[(size_t)nt.n * c->nwg];
+    const int64_t p0 = c->h_num_tot[(size_t)nt.n - 1], p1 = c->h_num_tot[(size_t)nt.n];
     if (p1 > p0) {
       CHK(hub_reserve(c, p1 - p0));
       hub_head(c, p0, p1 - p0, c->st);

@@ -12,8 +12,8 @@ namespace dbd {
 
 constexpr int kMaxCats = 16;
 
-// Category thresholds: row key k -> smallest c with k <= lim[c] (c = 0 is "k == 0"),
-// else the last category (the long-row path).
+// Category thresholds: row key k -> the number of limits below it, i.e. the smallest c with k <=
+// lim[c] (c = 0 is "k == 0"). The limits of the last categories and of those past n are INT64_MAX.
 struct CatTable {
   int64_t lim[kMaxCats];
   int32_t n;  // number of categories including 0 and the long category
@@ -76,9 +76,6 @@ void launch_fill_bytes0(void* p, int64_t nbytes, hipStream_t s);
 // Exclusive scan of n int64 (in may equal out); out[n] = total. tmp needs scan_tmp_elems(n).
 int64_t scan_tmp_elems(int64_t n);
 void launch_exclusive_scan(const int64_t* in, int64_t* out, int64_t n, int64_t* tmp, hipStream_t s);
-// out[b] = ptr[min(b*stride, n)] for b in [0, nb]
-void launch_gather_strided(const int64_t* ptr, int64_t n, int64_t stride, int64_t nb, int64_t* out, hipStream_t s);
-
 // Inside a captured pipeline: if *total > cap, set the capacity bit (16) in *err and zero
 // offs[0 .. n), which empties every bin range that the following row kernels read.
 constexpr int kErrCapacityBit = 16;
@@ -108,15 +105,30 @@ void launch_band_index(const int32_t* slot_row, int64_t nslots, const int64_t* B
 int64_t row_tiles(int64_t nnz);
 void launch_row_products(const Mat& A, const Mat& B, int64_t* P, int64_t* nnz, int64_t* bstart, int32_t* blen,
                          int32_t* tile_row, int* err, hipStream_t s);
-// Stable counting sort of rows [0, n) by category of min(key[i], cap).
-// counts/offs have ncat * nwg (+1) int64 where nwg = bin_tiles(n).
-int64_t bin_tiles(int64_t n);
+// Host memory (pinned) that the kernels report to; read it after synchronising the stream.
+struct HostReport {
+  int64_t tot[kMaxCats + 1];  // first row of every category in the list, the last: all rows
+  int32_t err[2];             // error word; hub rows of many entries
+  int64_t blk[1];             // per block the keys' sum before it; behind the last block the total
+};
+// Where a binning writes besides the list: the keys' exclusive prefix (n + 1 entries, twice if asked
+// for) and a report with blocks of `bt` tiles. All optional (host null: no report).
+struct BinOut {
+  int64_t *ptr = nullptr, *ptr2 = nullptr;
+  HostReport* host = nullptr;
+  const int* err = nullptr;
+  int64_t bt = 1;
+};
+// Stable counting sort of rows [0, n) by category of min(key[i], cap) into rows; offs (cat-major by
+// tile of bin_tiles(n), then the number of rows plus the keys' prefix by tile) has (ct.n + 1) *
+// bin_tiles(n) + 1 entries, counts (scratch) (ct.n + 1) * bin_tiles(n).
 // With hub_slot, rows of the category before the last (the long one by key) that have a hub slot
 // (>= 0) go to the last category (the hub category); *many counts those marked kHubMany.
-void launch_bin_count(const int64_t* key, int64_t n, int64_t cap, const CatTable& ct, int64_t* counts,
-                      hipStream_t s, const int32_t* hub_slot = nullptr, int* many = nullptr);
-void launch_bin_scatter(const int64_t* key, int64_t n, int64_t cap, const CatTable& ct, const int64_t* offs,
-                        int32_t* rows, hipStream_t s, const int32_t* hub_slot = nullptr);
+int64_t bin_tiles(int64_t n);
+void launch_bin(const int64_t* key, int64_t n, int64_t cap, const CatTable& ct, int64_t* counts, int64_t* offs,
+                int64_t* tmp, int32_t* rows, const BinOut& o, hipStream_t s, const int32_t* hub_slot = nullptr,
+                int* many = nullptr);
+void launch_report_err(const int* err, HostReport* host, hipStream_t s);
 
 // ---- symbolic / numeric / backward per category ----
 // grid == 0 -> exact grid from nrows_hint; else a persistent grid of that many workgroups.

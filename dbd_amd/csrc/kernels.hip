@@ -58,59 +58,6 @@ __device__ __forceinline__ void gsync() {
     __syncthreads();
 }
 
-template <int NT>
-struct Group {
-  static constexpr int W = NT < 64 ? NT : 64;
-  static constexpr int NW = NT > 64 ? NT / 64 : 1;
-
-  template <typename T, typename Op>
-  __device__ static T reduce(T v, Op op, T* sc) {
-#pragma unroll
-    for (int o = W / 2; o > 0; o >>= 1) v = op(v, __shfl_xor(v, o, W));
-    if constexpr (NT > 64) {
-      const int t = threadIdx.x % NT;
-      if ((t & 63) == 0) sc[t >> 6] = v;
-      __syncthreads();
-      v = sc[0];
-#pragma unroll
-      for (int i = 1; i < NW; ++i) v = op(v, sc[i]);
-      __syncthreads();
-    }
-    return v;
-  }
-
-  // Exclusive prefix of v over the group; total returned through `total`.
-  template <typename T>
-  __device__ static T exscan(T v, T& total, T* sc) {
-    const int t = threadIdx.x % NT;
-    const int lane = t % W;
-    T x = v;
-#pragma unroll
-    for (int o = 1; o < W; o <<= 1) {
-      T y = __shfl_up(x, o, W);
-      if (lane >= o) x += y;
-    }
-    if constexpr (NT <= 64) {
-      total = __shfl(x, W - 1, W);
-      return x - v;
-    } else {
-      const int wid = t >> 6;
-      if (lane == 63) sc[wid] = x;
-      __syncthreads();
-      T pre = 0, tot = 0;
-#pragma unroll
-      for (int i = 0; i < NW; ++i) {
-        T s = sc[i];
-        if (i < wid) pre += s;
-        tot += s;
-      }
-      __syncthreads();
-      total = tot;
-      return pre + x - v;
-    }
-  }
-};
-
 struct OpMin {
   template <typename T>
   __device__ T operator()(T a, T b) const { return a < b ? a : b; }
@@ -127,32 +74,100 @@ struct OpAdd {
   __device__ T operator()(T a, T b) const { return a + b; }
 };
 
-// Whole-wave reduction of an int without LDS: DPP within rows of 16 lanes (quad swaps, half
+// Lane move within the wave by DPP control word, of a 4- or 8-byte value; lanes without a source
+// keep `old`.
+template <int CTRL, int ROWS = 0xF, int BANKS = 0xF, typename T>
+__device__ __forceinline__ T dpp_mov(T old, T x) {
+  if constexpr (sizeof(T) == 4) {
+    return (T)__builtin_amdgcn_update_dpp((int)old, (int)x, CTRL, ROWS, BANKS, false);
+  } else {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)(uint64_t)old, (int)(uint32_t)(uint64_t)x,
+                                                              CTRL, ROWS, BANKS, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)((uint64_t)old >> 32),
+                                                              (int)(uint32_t)((uint64_t)x >> 32), CTRL, ROWS, BANKS, false);
+    return (T)(((uint64_t)hi << 32) | lo);
+  }
+}
+
+template <typename T>
+__device__ __forceinline__ T read_lane(T x, int lane) {
+  if constexpr (sizeof(T) == 4)
+    return (T)__builtin_amdgcn_readlane((int)x, lane);
+  else
+    return (T)readlane64((int64_t)x, lane);
+}
+
+// Whole-wave reduction of an integer without LDS: DPP within rows of 16 lanes (quad swaps, half
 // mirror, mirror), then the four row results through readlane. All 64 lanes must be active.
-template <typename Op>
-__device__ __forceinline__ int wave_reduce_dpp(int x, Op op) {
-  x = op(x, __builtin_amdgcn_update_dpp(x, x, 0xB1, 0xF, 0xF, false));   // quad_perm [1,0,3,2]
-  x = op(x, __builtin_amdgcn_update_dpp(x, x, 0x4E, 0xF, 0xF, false));   // quad_perm [2,3,0,1]
-  x = op(x, __builtin_amdgcn_update_dpp(x, x, 0x141, 0xF, 0xF, false));  // row_half_mirror
-  x = op(x, __builtin_amdgcn_update_dpp(x, x, 0x140, 0xF, 0xF, false));  // row_mirror
-  const int r0 = __builtin_amdgcn_readlane(x, 0), r1 = __builtin_amdgcn_readlane(x, 16);
-  const int r2 = __builtin_amdgcn_readlane(x, 32), r3 = __builtin_amdgcn_readlane(x, 48);
-  return op(op(r0, r1), op(r2, r3));
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_reduce_dpp(T x, Op op) {
+  x = op(x, dpp_mov<0xB1>(x, x));   // quad_perm [1,0,3,2]
+  x = op(x, dpp_mov<0x4E>(x, x));   // quad_perm [2,3,0,1]
+  x = op(x, dpp_mov<0x141>(x, x));  // row_half_mirror
+  x = op(x, dpp_mov<0x140>(x, x));  // row_mirror
+  return op(op(read_lane(x, 0), read_lane(x, 16)), op(read_lane(x, 32), read_lane(x, 48)));
 }
 
 // Inclusive prefix sum over the wave with DPP: shifts of 1-3, 4 and 8 lanes inside each row of
 // 16 lanes, then the row totals through the row broadcasts of lanes 15 and 31. All 64 lanes
 // must be active.
-__device__ __forceinline__ int wave_incl_scan_dpp(int x) {
-  int s = x + __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
-  s += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);         // row_shr:2
-  s += __builtin_amdgcn_update_dpp(0, x, 0x113, 0xF, 0xF, false);         // row_shr:3
-  s += __builtin_amdgcn_update_dpp(0, s, 0x114, 0xF, 0xE, false);         // row_shr:4, lanes 4-15
-  s += __builtin_amdgcn_update_dpp(0, s, 0x118, 0xF, 0xC, false);         // row_shr:8, lanes 8-15
-  s += __builtin_amdgcn_update_dpp(0, s, 0x142, 0xA, 0xF, false);         // row_bcast:15 -> rows 1, 3
-  s += __builtin_amdgcn_update_dpp(0, s, 0x143, 0xC, 0xF, false);         // row_bcast:31 -> rows 2, 3
+template <typename T>
+__device__ __forceinline__ T wave_incl_scan_dpp(T x) {
+  T s = x + dpp_mov<0x111>(T(0), x);              // row_shr:1
+  s += dpp_mov<0x112>(T(0), x);                   // row_shr:2
+  s += dpp_mov<0x113>(T(0), x);                   // row_shr:3
+  s += dpp_mov<0x114, 0xF, 0xE>(T(0), s);         // row_shr:4, lanes 4-15
+  s += dpp_mov<0x118, 0xF, 0xC>(T(0), s);         // row_shr:8, lanes 8-15
+  s += dpp_mov<0x142, 0xA, 0xF>(T(0), s);         // row_bcast:15 -> rows 1, 3
+  s += dpp_mov<0x143, 0xC, 0xF>(T(0), s);         // row_bcast:31 -> rows 2, 3
   return s;
 }
+
+template <int NT>
+struct Group {
+  static_assert(NT >= 64, "whole waves");
+  static constexpr int NW = NT / 64;
+
+  template <typename T, typename Op>
+  __device__ static T reduce(T v, Op op, T* sc) {
+    v = wave_reduce_dpp(v, op);
+    if constexpr (NT > 64) {
+      const int t = threadIdx.x % NT;
+      if ((t & 63) == 0) sc[t >> 6] = v;
+      __syncthreads();
+      v = sc[0];
+#pragma unroll
+      for (int i = 1; i < NW; ++i) v = op(v, sc[i]);
+      __syncthreads();
+    }
+    return v;
+  }
+
+  // Exclusive prefix of v over the group; total returned through `total`.
+  template <typename T>
+  __device__ static T exscan(T v, T& total, T* sc) {
+    const int t = threadIdx.x % NT;
+    const T x = wave_incl_scan_dpp(v);
+    if constexpr (NT <= 64) {
+      total = read_lane(x, 63);
+      return x - v;
+    } else {
+      const int lane = t & 63, wid = t >> 6;
+      if (lane == 63) sc[wid] = x;
+      __syncthreads();
+      T pre = 0, tot = 0;
+#pragma unroll
+      for (int i = 0; i < NW; ++i) {
+        T s = sc[i];
+        if (i < wid) pre += s;
+        tot += s;
+      }
+      __syncthreads();
+      total = tot;
+      return pre + x - v;
+    }
+  }
+};
 
 // Mask of the G lanes (within this wave) that share this lane's subgroup.
 template <int G>
@@ -826,28 +841,44 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_apply(const int64_t* in, 
   if (blockIdx.x == nb - 1 && threadIdx.x == 0) out[n] = part[nb];
 }
 
+// One workgroup, 16 items a thread at a time: one launch instead of three up to kScanOne items, where a
+// launch costs more than the idle CUs (16,384 items: 5 us against 3 x 4 us and two gaps).
+constexpr int64_t kScanOne = 32768;
+__global__ __launch_bounds__(1024) void k_scan_one(const int64_t* in, int64_t* out, int64_t n) {
+  __shared__ int64_t sc[16];
+  int64_t carry = 0;
+  for (int64_t b = 0; b < n; b += 1024 * kScanItems) {  // uniform
+    const int64_t base = b + (int64_t)threadIdx.x * kScanItems;
+    int64_t loc[kScanItems], sum = 0, tot;
+#pragma unroll
+    for (int i = 0; i < kScanItems; ++i) {
+      loc[i] = base + i < n ? in[base + i] : 0;
+      sum += loc[i];
+    }
+    int64_t pre = carry + Group<1024>::exscan(sum, tot, sc);
+#pragma unroll
+    for (int i = 0; i < kScanItems; ++i) {
+      if (base + i < n) out[base + i] = pre;
+      pre += loc[i];
+    }
+    carry += tot;
+  }
+  if (threadIdx.x == 0) out[n] = carry;
+}
+
 void launch_exclusive_scan(const int64_t* in, int64_t* out, int64_t n, int64_t* tmp, hipStream_t s) {
   if (n <= 0) {
     launch_fill_i64(out, 1, 0, s);
+    return;
+  }
+  if (n <= kScanOne) {
+    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, s, in, out, n);
     return;
   }
   const int64_t nb = (n + kScanTile - 1) / kScanTile;
   hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(kScanThreads), 0, s, in, n, tmp);
   hipLaunchKernelGGL(k_scan_partials, dim3(1), dim3(1024), 0, s, tmp, nb);
   hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(kScanThreads), 0, s, in, out, n, tmp, nb);
-}
-
-__global__ void k_gather_strided(const int64_t* __restrict__ ptr, int64_t n, int64_t stride, int64_t nb,
-                                 int64_t* __restrict__ out) {
-  for (int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; b <= nb; b += (int64_t)gridDim.x * blockDim.x) {
-    int64_t r = b * stride;
-    if (r > n) r = n;
-    out[b] = ptr[r];
-  }
-}
-
-void launch_gather_strided(const int64_t* ptr, int64_t n, int64_t stride, int64_t nb, int64_t* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_gather_strided, dim3(fill_grid(nb + 1)), dim3(256), 0, s, ptr, n, stride, nb, out);
 }
 
 // Output capacity check inside a captured pipeline: when the exact output size (*total) exceeds
@@ -1078,11 +1109,12 @@ void launch_band_index(const int32_t* slot_row, int64_t nslots, const int64_t* B
 constexpr int kBinTile = 256;
 int64_t bin_tiles(int64_t n) { return (n + kBinTile - 1) / kBinTile; }
 
+// The limits past the last category are INT64_MAX, so no branch and no load depends on the key.
 __device__ __forceinline__ int category_of(int64_t k, const CatTable& ct) {
-  if (k <= 0) return 0;
-  for (int c = 1; c < ct.n - 1; ++c)
-    if (k <= ct.lim[c]) return c;
-  return ct.n - 1;
+  int c = 0;
+#pragma unroll
+  for (int x = 0; x < kMaxCats; ++x) c += k > ct.lim[x];
+  return c;
 }
 
 // Category of row i: by key. Numeric tables end with the long category (limit INT64_MAX, so no
@@ -1096,37 +1128,51 @@ __device__ __forceinline__ int row_category(int64_t k, const CatTable& ct, const
   return c;
 }
 
+// The tiles' category counts (cat-major) and, behind them, the tiles' sums of the keys: one scan turns
+// them into the bins' offsets and the prefix of the keys.
 __global__ __launch_bounds__(kBinTile) void k_bin_count(const int64_t* __restrict__ key, int64_t n, int64_t cap,
                                                         CatTable ct, int64_t* __restrict__ counts, int64_t nwg,
                                                         const int32_t* __restrict__ hub_slot,
                                                         int* __restrict__ many) {
   __shared__ int hist[kMaxCats];
+  __shared__ int64_t sc[kBinTile / 64];
   if (threadIdx.x < kMaxCats) hist[threadIdx.x] = 0;
   __syncthreads();
   const int64_t i = (int64_t)blockIdx.x * kBinTile + threadIdx.x;
+  const int64_t k = i < n ? key[i] : 0;
   if (i < n) {
-    int64_t k = key[i];
-    if (k > cap) k = cap;
-    const int c = row_category(k, ct, hub_slot, i);
+    const int c = row_category(min(k, cap), ct, hub_slot, i);
     atomicAdd(&hist[c], 1);
     if (hub_slot && c == ct.n - 1 && (hub_slot[i] & kHubMany)) atomicAdd(many, 1);
   }
-  __syncthreads();
+  const int64_t sum = Group<kBinTile>::reduce(k, OpAdd(), sc);  // also: the counts are complete
   if ((int)threadIdx.x < ct.n) counts[(int64_t)threadIdx.x * nwg + blockIdx.x] = hist[threadIdx.x];
+  if (threadIdx.x == 0) counts[(int64_t)ct.n * nwg + blockIdx.x] = sum;
+}
+
+// What the host reads after a binning, in pinned memory: categories' offsets, error word (with the
+// count beside it), and the keys' sums up to the start of each block of `bt` tiles (the last one: all).
+__device__ __forceinline__ void bin_report(const BinOut& o, int64_t tile, int64_t nwg, int ncat, const int64_t* offs,
+                                           int64_t key_sum, int64_t key_all) {
+  if (!o.host) return;
+  const int t = threadIdx.x;
+  if (tile == 0) {
+    if (t <= ncat) o.host->tot[t] = offs[(int64_t)t * nwg];
+    if (t < 2) o.host->err[t] = o.err[t];
+    if (t == 0) o.host->blk[(nwg + o.bt - 1) / o.bt] = key_all;
+  }
+  if (t == 0 && tile % o.bt == 0) o.host->blk[tile / o.bt] = key_sum;
 }
 
 __global__ __launch_bounds__(kBinTile) void k_bin_scatter(const int64_t* __restrict__ key, int64_t n, int64_t cap,
                                                           CatTable ct, const int64_t* __restrict__ offs, int64_t nwg,
                                                           int32_t* __restrict__ rows,
-                                                          const int32_t* __restrict__ hub_slot) {
+                                                          const int32_t* __restrict__ hub_slot, BinOut o) {
   __shared__ int wc[kBinTile / 64][kMaxCats];
+  __shared__ int64_t sc[kBinTile / 64];
   const int64_t i = (int64_t)blockIdx.x * kBinTile + threadIdx.x;
-  int c = -1;
-  if (i < n) {
-    int64_t k = key[i];
-    if (k > cap) k = cap;
-    c = row_category(k, ct, hub_slot, i);
-  }
+  const int64_t k = i < n ? key[i] : 0;
+  const int c = i < n ? row_category(min(k, cap), ct, hub_slot, i) : -1;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   int rank = 0;
@@ -1140,21 +1186,129 @@ __global__ __launch_bounds__(kBinTile) void k_bin_scatter(const int64_t* __restr
     for (int w = 0; w < wid; ++w) rank += wc[w][c];
     rows[offs[(int64_t)c * nwg + blockIdx.x] + rank] = (int32_t)i;
   }
+  const int64_t* kp = offs + (int64_t)ct.n * nwg;  // keys' prefix by tile, behind the number of rows
+  const int64_t before = kp[blockIdx.x] - kp[0];
+  if (o.ptr) {
+    int64_t tot;
+    const int64_t at = before + Group<kBinTile>::exscan(k, tot, sc);
+    if (i < n) {
+      o.ptr[i] = at;
+      if (o.ptr2) o.ptr2[i] = at;
+      if (i == n - 1) {
+        o.ptr[n] = at + k;
+        if (o.ptr2) o.ptr2[n] = at + k;
+      }
+    }
+  }
+  bin_report(o, blockIdx.x, nwg, ct.n, offs, before, kp[nwg] - kp[0]);
 }
 
-void launch_bin_count(const int64_t* key, int64_t n, int64_t cap, const CatTable& ct, int64_t* counts,
-                      hipStream_t s, const int32_t* hub_slot, int* many) {
+// Both binning kernels and the scan between them in one launch of one workgroup, for up to 64 tiles:
+// chunk of 64 rows q * 16 + wave is lane-parallel in its wave, the counts of all chunks and the
+// keys' sums are scanned in LDS.
+constexpr int kBinOneTiles = 64;
+__global__ __launch_bounds__(1024) void k_bin_one(const int64_t* __restrict__ key, int64_t n, int64_t cap, CatTable ct,
+                                                  int64_t* __restrict__ offs, int64_t nwg, int32_t* __restrict__ rows,
+                                                  const int32_t* __restrict__ hub_slot, int* __restrict__ many, BinOut o) {
+  constexpr int CH = kBinOneTiles * kBinTile / 64;  // chunks of 64 rows
+  constexpr int Q = CH / 16;                        // per wave
+  __shared__ int cc[kMaxCats * CH];                 // rows by (category, chunk), then their places
+  __shared__ int64_t ks[CH];                        // keys by chunk, then their prefix
+  __shared__ int64_t sc[16];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int nch = (int)((n + 63) / 64);
+  int64_t k[Q];
+  int c[Q], rank[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int64_t i = (int64_t)(q * 16 + wv) * 64 + lane;
+    k[q] = i < n ? key[i] : 0;
+  }
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int ch = q * 16 + wv;
+    const int64_t i = (int64_t)ch * 64 + lane;
+    if (ch >= nch) continue;  // wave-uniform
+    c[q] = i < n ? row_category(min(k[q], cap), ct, hub_slot, i) : -1;
+    rank[q] = 0;
+    int cnt = 0;  // lane x: rows of category x
+    for (int x = 0; x < ct.n; ++x) {
+      const uint64_t b = __builtin_amdgcn_ballot_w64(c[q] == x);
+      if (c[q] == x) rank[q] = __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0));
+      cnt = lane == x ? (int)__popcll(b) : cnt;
+    }
+    if (lane < ct.n) cc[lane * nch + ch] = cnt;
+    if (hub_slot && c[q] == ct.n - 1 && (hub_slot[i] & kHubMany)) atomicAdd(many, 1);
+    int64_t tot;
+    const int64_t ex = Group<64>::exscan(k[q], tot, sc);
+    if (lane == 0) ks[ch] = tot;
+    k[q] = ex;  // within the chunk, from here on
+  }
+  __syncthreads();
+  int64_t carry = 0, tot;
+  for (int b = 0; b < ct.n * nch; b += 1024) {  // uniform
+    const int v = b + t < ct.n * nch ? cc[b + t] : 0;
+    const int64_t ex = carry + Group<1024>::exscan((int64_t)v, tot, sc);
+    if (b + t < ct.n * nch) cc[b + t] = (int)ex;
+    carry += tot;
+  }
+  const int64_t kv = t < nch ? ks[t] : 0;
+  const int64_t kex = Group<1024>::exscan(kv, tot, sc);
+  if (t < nch) ks[t] = kex;
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int ch = q * 16 + wv;
+    const int64_t i = (int64_t)ch * 64 + lane;
+    if (i >= n) continue;
+    rows[cc[c[q] * nch + ch] + rank[q]] = (int32_t)i;
+    if (o.ptr) {
+      const int64_t at = ks[ch] + k[q];
+      o.ptr[i] = at;
+      if (o.ptr2) o.ptr2[i] = at;
+    }
+  }
+  if (o.ptr && t == 0) {
+    o.ptr[n] = tot;
+    if (o.ptr2) o.ptr2[n] = tot;
+  }
+  // the offsets as the launches by tile leave them
+  for (int x = t; x < ct.n * (int)nwg; x += 1024) offs[x] = cc[(x / (int)nwg) * nch + 4 * (x % (int)nwg)];
+  for (int x = t; x <= (int)nwg; x += 1024) offs[(int64_t)ct.n * nwg + x] = n + (x < (int)nwg ? ks[4 * x] : tot);
+  if (!o.host) return;
+  if (t < ct.n) o.host->tot[t] = cc[t * nch];
+  if (t == ct.n) o.host->tot[t] = n;
+  if (t < 2) o.host->err[t] = o.err[t];
+  const int nb = (int)((nwg + o.bt - 1) / o.bt);
+  for (int b = t; b <= nb; b += 1024) o.host->blk[b] = b < nb ? ks[4 * b * o.bt] : tot;
+}
+
+void launch_bin(const int64_t* key, int64_t n, int64_t cap, const CatTable& ct, int64_t* counts, int64_t* offs,
+                int64_t* tmp, int32_t* rows, const BinOut& o, hipStream_t s, const int32_t* hub_slot, int* many) {
   const int64_t nwg = bin_tiles(n);
-  if (nwg == 0) return;
+  if (nwg == 0) {
+    launch_fill_i64(offs, 1, 0, s);
+    if (o.ptr) launch_fill_i64(o.ptr, 1, 0, s);
+    if (o.ptr2) launch_fill_i64(o.ptr2, 1, 0, s);
+    return;
+  }
+  if (nwg <= kBinOneTiles) {
+    hipLaunchKernelGGL(k_bin_one, dim3(1), dim3(1024), 0, s, key, n, cap, ct, offs, nwg, rows, hub_slot, many, o);
+    return;
+  }
   hipLaunchKernelGGL(k_bin_count, dim3((unsigned)nwg), dim3(kBinTile), 0, s, key, n, cap, ct, counts, nwg, hub_slot,
                      many);
-}
-void launch_bin_scatter(const int64_t* key, int64_t n, int64_t cap, const CatTable& ct, const int64_t* offs,
-                        int32_t* rows, hipStream_t s, const int32_t* hub_slot) {
-  const int64_t nwg = bin_tiles(n);
-  if (nwg == 0) return;
+  launch_exclusive_scan(counts, offs, (ct.n + 1) * nwg, tmp, s);
   hipLaunchKernelGGL(k_bin_scatter, dim3((unsigned)nwg), dim3(kBinTile), 0, s, key, n, cap, ct, offs, nwg, rows,
-                     hub_slot);
+                     hub_slot, o);
+}
+
+// The error word and the count beside it to the host's copy.
+__global__ void k_report_err(const int* __restrict__ err, HostReport* host) {
+  if (threadIdx.x < 2) host->err[threadIdx.x] = err[threadIdx.x];
+}
+void launch_report_err(const int* err, HostReport* host, hipStream_t s) {
+  hipLaunchKernelGGL(k_report_err, dim3(1), dim3(64), 0, s, err, host);
 }
 
 // ------------------------------------------------------------------------------------

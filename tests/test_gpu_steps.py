@@ -94,3 +94,35 @@ def test_hub_sums_of_special_values(gpu_ok, ncols, dtype):
             C = ctx.result()
         assert np.array_equal(C.ptr, Cptr) and np.array_equal(C.idx, Cidx), what
         assert np.array_equal(C.val, Cval.astype(dtype), equal_nan=True), what
+
+
+# binning: one launch up to 64 tiles of 256 rows, by tile beyond; the scan in one launch up to 32768
+# counters, in three beyond; block tables over both
+@pytest.mark.parametrize("block_rows", [256, 4096])
+@pytest.mark.parametrize("nrows", [1, 63, 64, 65, 255, 257, 16383, 16384, 16385, 16640, 700_001])
+def test_bins_and_block_tables(gpu_ok, nrows, block_rows):
+    rng = np.random.default_rng(nrows)
+    B = from_lengths(rng.integers(0, 70, 300), 5000, 16)
+    lens = np.minimum(rng.geometric(0.3, nrows) - 1, 40) if nrows > 1 else [7]
+    ptr = np.concatenate([[0], np.cumsum(lens)])
+    idx = np.concatenate([np.sort(rng.permutation(300)[:n]) for n in range(41)])  # a row of n entries: the n-th list
+    at = np.concatenate([[0], np.cumsum(np.arange(41))])
+    idx = idx[np.repeat(at[np.asarray(lens)] - ptr[:-1], lens) + np.arange(ptr[-1])]
+    A = dbd_amd.CSR(ptr, idx.astype(np.int32), rng.standard_normal(int(ptr[-1])), (nrows, 300))
+    P = oracle.row_products(A.ptr, A.idx, B.ptr)
+    ref = reference(A, B)
+    with dbd_amd.Context(block_rows=block_rows) as ctx:
+        ctx.set_operands(A, B)
+        info = ctx.plan()
+        bptr, bprod, binfo = dbd_amd.plan_blocks(P, block_rows)
+        gptr, gprod = ctx.blocks(info["num_blocks"])
+        assert np.array_equal(gptr, bptr) and np.array_equal(gprod, bprod)
+        assert all(info[k] == binfo[k] for k in ("products", "criteria", "max_block_products", "blocks_any"))
+        ctx.run("compute")
+        compare(ctx.result(), ref, np.float64, f"{nrows} rows")
+        assert sum(ctx.plan_info()["num_rows"]) == nrows
+    if nrows > 60000:  # several chunks: the offsets by tile
+        with dbd_amd.Context(block_rows=block_rows, chunks_hint=5) as ctx:
+            ctx.set_operands(A, B)
+            assert ctx.run("d2h")["chunks"] > 1
+            compare(ctx.result(), ref, np.float64, "chunks")
