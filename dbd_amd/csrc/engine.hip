@@ -1434,7 +1434,7 @@ void dbd::enqueue_pipeline(const Work& w, const Tables& tb, Mat A, const Mat& B,
   launch_bin(w.P, nr, B.ncols, ct, w.cnt, w.offs_sym, w.tmp, w.rows_sym, BinOut{}, s);
   if (w.hub_sym_fn) w.hub_sym_fn(w.hub_arg, s);
   for (int k = 1; k < ct.n; ++k)
-    launch_symbolic(tb.sym_k[k], w.rows_sym, w.offs_sym + (int64_t)k * w.nwg, w.offs_sym + (int64_t)(k + 1) * w.nwg, 0,
+    launch_symbolic(tb.sym_k[k], w.rows_sym, w.offs_sym + (int64_t)k * w.nwg, w.offs_sym + (int64_t)(k + 1) * w.nwg, nr,
                     persistent_grid(num_cu, tb.sym_k[k]), A, B, w.nnz, w.cursor, w.err, s, w.hub_slot);
   const CatTable& nt = tb.num_ct;
   BinOut o;
@@ -1444,7 +1444,7 @@ void dbd::enqueue_pipeline(const Work& w, const Tables& tb, Mat A, const Mat& B,
   for (int k = 1; k < nt.n; ++k) {
     if (tb.num_k[k].T == kHubShape) continue;  // the range kernels below (empty without hub slots)
     launch_numeric(dtype, tb.num_k[k], w.rows_num, w.offs_num + (int64_t)k * w.nwg, w.offs_num + (int64_t)(k + 1) * w.nwg,
-                   0, persistent_grid(num_cu, tb.num_k[k]), A, B, d_Cptr, 0, d_Cidx, d_Cval, w.cursor, w.err, s, false);
+                   nr, persistent_grid(num_cu, tb.num_k[k]), A, B, d_Cptr, 0, d_Cidx, d_Cval, w.cursor, w.err, s, false);
   }
   if (w.hub_slot && w.hub_fn) w.hub_fn(w.hub_arg, d_Cptr, d_Cidx, d_Cval, s);
 }

@@ -131,7 +131,8 @@ void launch_bin(const int64_t* key, int64_t n, int64_t cap, const CatTable& ct, 
 void launch_report_err(const int* err, HostReport* host, hipStream_t s);
 
 // ---- symbolic / numeric / backward per category ----
-// grid == 0 -> exact grid from nrows_hint; else a persistent grid of that many workgroups.
+// grid == 0 -> exact grid from nrows_hint, the number of rows; else a persistent grid of that many
+// workgroups, nrows_hint a bound on the rows.
 int symbolic_groups_per_wg(const KernelShape& k);
 // With hub_slot, the long-row kernel leaves out the rows that have a slot (>= 0): launch_hub_count's.
 void launch_symbolic(const KernelShape& k, const int32_t* rows, const int64_t* pbeg, const int64_t* pend,

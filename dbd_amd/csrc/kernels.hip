@@ -1391,6 +1391,262 @@ __global__ __launch_bounds__(wg_of<NT>()) __attribute__((amdgpu_waves_per_eu(NT 
   }
 }
 
+// ------------------------------------------------------------------------------------
+// several short rows per wave
+// ------------------------------------------------------------------------------------
+// A wave per row leaves most lanes idle on rows of a few products, and pays the table clears, the
+// ranking and every wait once per row. Rows of up to 256 table slots share a wave instead: 512 / T
+// rows, T / 8 lanes and T slots each, eight slots a lane. The rows' A entries (a lane each) are
+// flattened together (walk_spans), so one gather covers all of the wave's rows; inserts go to the
+// row's own part of the table; the ranking (as wave_rank_keys) runs in all rows at once, its scans
+// within the row's lanes. Bound by the chain row id - row pointers - descriptors - gathers, which
+// 20 waves a CU and up to 8 rows a wave hide. Where: kMultiRows.
+constexpr int kMultiSlots = 512;
+
+// Reduction and inclusive prefix sum within groups of L = 8, 16 or 32 lanes.
+template <int L, typename Op>
+__device__ __forceinline__ int lanes_reduce(int x, Op op) {
+  x = op(x, dpp_mov<0xB1>(x, x));
+  x = op(x, dpp_mov<0x4E>(x, x));
+  x = op(x, dpp_mov<0x141>(x, x));
+  if constexpr (L >= 16) x = op(x, dpp_mov<0x140>(x, x));
+  if constexpr (L >= 32) x = op(x, __shfl_xor(x, 16));
+  return x;
+}
+template <int L>
+__device__ __forceinline__ int lanes_incl_scan(int x, int l) {
+  int y = dpp_mov<0x111>(0, x);
+  x += l >= 1 ? y : 0;
+  y = dpp_mov<0x112>(0, x);
+  x += l >= 2 ? y : 0;
+  y = dpp_mov<0x114>(0, x);
+  x += l >= 4 ? y : 0;
+  if constexpr (L >= 16) {
+    y = dpp_mov<0x118>(0, x);
+    x += (l & 15) >= 8 ? y : 0;
+  }
+  if constexpr (L >= 32) x += dpp_mov<0x142, 0xA, 0xF>(0, x);
+  return x;
+}
+
+// LDS of one wave: the rows' tables, and per rank of walk_spans A's value and the row's table.
+template <typename V, bool WITHV>
+struct MultiLds {
+  __align__(16) int K[kMultiSlots];
+  __align__(16) double H[WITHV ? kMultiSlots : 2];
+  SpanLds sp;
+  V va[WITHV ? 64 : 1];
+  int tab[64];
+};
+
+// Inserts the products of the wave's rows: lane l holds entries e, e + L, .. < a1 of its row, whose
+// table starts at K[tab]. Returns a non-zero value in some lane if a table is full.
+template <int T, bool WITHV, typename V>
+__device__ __forceinline__ int multi_insert(int lane, int64_t e, int64_t a1, int tab, MultiLds<V, WITHV>& m,
+                                            const int64_t* __restrict__ bstart, const int32_t* __restrict__ blen,
+                                            const V* __restrict__ Aval, const int32_t* __restrict__ Bidx,
+                                            const V* __restrict__ Bval) {
+  constexpr int L = T / 8, U = 4;
+  int bad = 0;
+  while (__builtin_amdgcn_ballot_w64(e < a1)) {  // wave-uniform
+    int len = 0;
+    int64_t start = 0;
+    V va = V(0);
+    if (e < a1) {
+      len = blen[e];
+      start = bstart[e];
+      if (WITHV) va = Aval[e];
+    }
+    walk_spans<U>(lane, len, start, m.sp,
+                  [&](int r) {
+                    if (WITHV) m.va[r] = va;
+                    m.tab[r] = tab;
+                  },
+                  [&](const int64_t (&at)[U], const int (&j)[U]) {
+                    int c[U], old[U];
+                    V b[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                      const int64_t p = at[u] < 0 ? 0 : at[u];
+                      c[u] = Bidx[p];
+                      b[u] = WITHV ? Bval[p] : V(0);
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                      old[u] = at[u] < 0 ? 0 : atomicCAS(&m.K[m.tab[j[u]] + hslot<T>(c[u])], kEmpty, c[u]);
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                      if (at[u] < 0) continue;
+                      const int tb = m.tab[j[u]];
+                      uint32_t h = hslot<T>(c[u]);
+                      int o = old[u], probe = 0;
+                      while (o != kEmpty && o != c[u] && probe < T) {
+                        h = (h + 1) & (T - 1);
+                        o = atomicCAS(&m.K[tb + h], kEmpty, c[u]);
+                        ++probe;
+                      }
+                      if (probe == T) bad = 1;
+                      else if (WITHV) lds_add(&m.H[tb + h], (double)m.va[WITHV ? j[u] : 0] * (double)b[u]);
+                    }
+                  });
+    e += L;
+  }
+  return bad;
+}
+
+template <int T>
+__global__ __launch_bounds__(256) void k_symbolic_multi(
+    const int32_t* __restrict__ rows, const int64_t* __restrict__ pbeg, const int64_t* __restrict__ pend,
+    const int64_t* __restrict__ Aptr, const int64_t* __restrict__ bstart, const int32_t* __restrict__ blen,
+    const int32_t* __restrict__ Bidx, int64_t* __restrict__ nnz, int* __restrict__ err) {
+  constexpr int R = kMultiSlots / T, L = 64 / R;
+  __shared__ MultiLds<float, false> lds[4];
+  const int lane = threadIdx.x & 63, g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  MultiLds<float, false>& m = lds[g];
+  const int rl = lane / L, l = lane % L;
+  const int64_t beg = *pbeg, end = *pend;
+  int bad = 0;
+  for (int64_t s0 = beg + (xcd_block() * 4 + g) * R; s0 < end; s0 += (int64_t)gridDim.x * 4 * R) {  // wave-uniform
+    const bool have = s0 + rl < end;
+    const int row = rows[have ? s0 + rl : s0];
+    const int64_t a0 = Aptr[row], a1 = have ? Aptr[row + 1] : a0;
+    int4* K4 = reinterpret_cast<int4*>(m.K);
+    K4[lane] = K4[lane + 64] = make_int4(kEmpty, kEmpty, kEmpty, kEmpty);
+    wave_sync();
+    bad |= multi_insert<T, false, float>(lane, a0 + l, a1, rl * T, m, bstart, blen, nullptr, Bidx, nullptr);
+    wave_sync();
+    const int4 x = K4[2 * lane], y = K4[2 * lane + 1];  // this lane's eight slots of its row's table
+    int cnt = (x.x != kEmpty) + (x.y != kEmpty) + (x.z != kEmpty) + (x.w != kEmpty) + (y.x != kEmpty) +
+              (y.y != kEmpty) + (y.z != kEmpty) + (y.w != kEmpty);
+    cnt = lanes_reduce<L>(cnt, OpAdd());
+    if (have && l == 0) nnz[row] = cnt;
+    wave_sync();
+  }
+  if (__builtin_amdgcn_ballot_w64(bad) && lane == 0) atomicOr(err, kErrTableFull);
+}
+
+template <typename V, int T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_numeric_multi(
+    const int32_t* __restrict__ rows, const int64_t* __restrict__ pbeg, const int64_t* __restrict__ pend,
+    const int64_t* __restrict__ Aptr, const int64_t* __restrict__ bstart, const int32_t* __restrict__ blen,
+    const V* __restrict__ Aval, const int32_t* __restrict__ Bidx, const V* __restrict__ Bval,
+    const int64_t* __restrict__ Cptr, int64_t cbase, int32_t* __restrict__ Cidx, V* __restrict__ Cval,
+    int* __restrict__ err) {
+  constexpr int R = kMultiSlots / T, L = 64 / R;
+  constexpr int NB = T / 2 - 1;  // buckets of a row; the counter behind them ends up as the total
+  __shared__ MultiLds<V, true> lds[4];
+  const int lane = threadIdx.x & 63, g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  MultiLds<V, true>& m = lds[g];
+  const int rl = lane / L, l = lane % L;
+  int* K = m.K + rl * T;        // this row's table, then its bucket counters, then its ranked keys
+  int* perm = K + T / 2;        // keys by bucket, then the ranked keys' slots
+  double* H = m.H + rl * T;
+  const int64_t beg = *pbeg, end = *pend;
+  int flags = 0;
+  for (int64_t s0 = beg + (xcd_block() * 4 + g) * R; s0 < end; s0 += (int64_t)gridDim.x * 4 * R) {  // wave-uniform
+    const bool have = s0 + rl < end;
+    const int row = rows[have ? s0 + rl : s0];
+    const int64_t a0 = Aptr[row], a1 = have ? Aptr[row + 1] : a0;
+    const int64_t c0 = Cptr[row] - cbase;
+    const int nexp = have ? (int)(Cptr[row + 1] - Cptr[row]) : 0;  // at most T / 2
+    int4* K4 = reinterpret_cast<int4*>(m.K);
+    K4[lane] = K4[lane + 64] = make_int4(kEmpty, kEmpty, kEmpty, kEmpty);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) reinterpret_cast<int4*>(m.H)[lane + 64 * q] = make_int4(0, 0, 0, 0);
+    wave_sync();
+    if (multi_insert<T, true, V>(lane, a0 + l, a1, rl * T, m, bstart, blen, Aval, Bidx, Bval)) flags |= kErrTableFull;
+    wave_sync();
+    int kk[8], bi[8];
+    {
+      const int4 x = K4[2 * lane], y = K4[2 * lane + 1];
+      kk[0] = x.x, kk[1] = x.y, kk[2] = x.z, kk[3] = x.w, kk[4] = y.x, kk[5] = y.y, kk[6] = y.z, kk[7] = y.w;
+    }
+    int cmin = INT_MAX, cmax = -1;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      cmin = kk[q] != kEmpty ? min(cmin, kk[q]) : cmin;
+      cmax = max(cmax, kk[q]);
+    }
+    cmin = lanes_reduce<L>(cmin, OpMin());
+    cmax = lanes_reduce<L>(cmax, OpMax());
+    wave_sync();
+    // ---- bucket counts and their prefix ----
+    reinterpret_cast<int4*>(K)[l] = make_int4(0, 0, 0, 0);
+    const uint32_t range = (uint32_t)(cmax - cmin) + 1u;
+    const bool direct = range <= (uint32_t)NB;
+    const uint32_t mul = direct ? 0u : (uint32_t)((float)NB * 4294967296.0f / (float)range * 0.99999f);
+    wave_sync();
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      bi[q] = 0;
+      if (kk[q] != kEmpty) {
+        const uint32_t x = (uint32_t)(kk[q] - cmin);
+        const int b = direct ? (int)x : (int)__umulhi(x, mul);
+        bi[q] = b | (atomicAdd(&K[b], 1) << 16);
+      }
+    }
+    wave_sync();
+    {
+      const int4 x = reinterpret_cast<int4*>(K)[l];
+      const int sum = x.x + x.y + x.z + x.w;
+      const int p = lanes_incl_scan<L>(sum, l) - sum;
+      wave_sync();
+      reinterpret_cast<int4*>(K)[l] = make_int4(p, p + x.x, p + x.x + x.y, p + x.x + x.y + x.z);
+    }
+    wave_sync();
+    // ---- keys by bucket, ranks within the buckets ----
+    const int n = K[NB];
+    int sl[8];  // start | length << 16
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      sl[q] = 0;
+      if (kk[q] != kEmpty) {
+        const int b = bi[q] & 0xFFFF;
+        const int b0 = K[b], b1 = min(K[b + 1], T / 2);
+        sl[q] = b0 | (max(b1 - b0, 0) << 16);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (kk[q] != kEmpty) {
+        const int pos = (sl[q] & 0xFFFF) + (bi[q] >> 16);
+        if (pos < T / 2) perm[pos] = kk[q];
+      }
+    wave_sync();
+    int rk[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) rk[q] = kk[q] != kEmpty ? (sl[q] & 0xFFFF) : T;
+    for (int j = 0;; ++j) {
+      bool more = false;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int len = sl[q] >> 16;
+        if (len > 1 && j < len) rk[q] += (perm[(sl[q] & 0xFFFF) + j] < kk[q]);
+        more |= (len > 1 && j + 1 < len);
+      }
+      if (!__builtin_amdgcn_ballot_w64(more)) break;
+    }
+    wave_sync();
+    // ---- key at its rank, slot beside it; stores ----
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (rk[q] < T / 2) {
+        K[rk[q]] = kk[q];
+        perm[rk[q]] = 8 * l + q;
+      }
+    wave_sync();
+    flags |= (n != nexp) ? kErrCountMismatch : 0;
+    const int nw = min(n, nexp);
+    for (int k = l; k < nw; k += L) {
+      Cidx[c0 + k] = K[k];
+      Cval[c0 + k] = (V)H[perm[k]];
+    }
+    wave_sync();
+  }
+  flags = wave_reduce_dpp(flags, OpOr());
+  if (lane == 0 && flags) atomicOr(err, flags);
+}
+
 // Per-row records of the banded long-row windows, 16 bytes each (the workspace holds 16 bytes per
 // A nonzero): an entry with a banded B row (start of its B row, its slot, its index in the row),
 // and one without (position from its B row's start, index in the row, next column, entries left).
@@ -3655,6 +3911,13 @@ static int grid_for(int64_t nrows, int gpb, int grid, const void* f = nullptr, i
   return (int)g;
 }
 
+// Rows of a category from which several share a wave: up to there every row can have a wave of its own
+// at once (256 CUs, 20 waves each), whose chain is shorter (1,000 rows of 62: 8 us against 14). From
+// there on, per launch: 1,200,000 rows of up to 32 columns 0.70 -> 0.26 ms, batch members' rows of up
+// to 64 / 128 columns 52 -> 36 / 67 -> 50 us. Rows of distinct products past 32 columns keep the
+// register path of k_numeric_wave_fast (20,000 rows of up to 64 columns: 26 us against 40).
+constexpr int64_t kMultiRows = 8192;
+
 constexpr int kLongNT = 256;
 constexpr int kSymLongW = 131072;  // bits per symbolic window (16 KB bitmap)
 #ifndef DBD_NUM_LONG_BW
@@ -3692,6 +3955,17 @@ void launch_symbolic(const KernelShape& k, const int32_t* rows, const int64_t* p
                        A.bstart, A.blen, B.idx, nnz, cursor, err, hub_slot, A.idx, B.hslot, B.band, B.nb1);
     return;
   }
+#define M(T_)                                                                                                    \
+  if (k.T == T_ && k.NT == 64 && k.G == 16 && nrows_hint > kMultiRows) {                                       \
+    const dim3 gr(grid_for(nrows_hint, 4 * (kMultiSlots / T_), grid, (const void*)k_symbolic_multi<T_>, 256)); \
+    hipLaunchKernelGGL((k_symbolic_multi<T_>), gr, dim3(256), 0, s, rows, pbeg, pend, A.ptr, A.bstart, A.blen, \
+                       B.idx, nnz, err);                                                                        \
+    return;                                                                                                     \
+  }
+  M(64)
+  M(128)
+  M(256)
+#undef M
 #define X(T_, NT_, G_)                                                                                         \
   if (k.T == T_ && k.NT == NT_ && k.G == G_) {                                                               \
     const dim3 gr(grid_for(nrows_hint, gpb, grid, (const void*)k_symbolic_hash<T_, NT_, G_>, wg_of<NT_>())); \
@@ -3724,6 +3998,17 @@ static void launch_numeric_t(const KernelShape& k, const int32_t* rows, const in
                        B.hslot, B.band, B.nb1);
     return;
   }
+#define M(T_)                                                                                                    \
+  if (k.T == T_ && k.NT == 64 && k.G == 16 && nrows_hint > kMultiRows && (T_ == 64 || !distinct)) {            \
+    const dim3 gr(grid_for(nrows_hint, 4 * (kMultiSlots / T_), grid, (const void*)k_numeric_multi<V, T_>, 256)); \
+    hipLaunchKernelGGL((k_numeric_multi<V, T_>), gr, dim3(256), 0, s, rows, pbeg, pend, A.ptr, A.bstart, A.blen, \
+                       Av, B.idx, Bv, Cptr, cbase, Cidx, Cval, err);                                            \
+    return;                                                                                                     \
+  }
+  M(64)
+  M(128)
+  M(256)
+#undef M
 #define X(T_, NT_, G_)                                                                                           \
   if (k.T == T_ && k.NT == NT_ && k.G == G_) {                                                                 \
     if constexpr (NT_ == 64) {                                                                                 \

@@ -126,3 +126,19 @@ def test_bins_and_block_tables(gpu_ok, nrows, block_rows):
             ctx.set_operands(A, B)
             assert ctx.run("d2h")["chunks"] > 1
             compare(ctx.result(), ref, np.float64, "chunks")
+
+
+# several rows per wave (more than 8192 rows of a category): groups cut off at the end of a bin, rows
+# with more entries than their lanes, with one long B row, and full tables; one-wave rows below that
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("nrows", [8100, 8193, 30011])
+def test_several_rows_per_wave(gpu_ok, nrows, dtype):
+    rng = np.random.default_rng(nrows)
+    blen = rng.permutation([0] * 20 + [1] * 300 + [2, 3, 5, 8, 13, 16, 31, 32, 33, 63, 64, 65, 127, 128] * 20)
+    for ncols, per_row in ((700, 6), (40, 40), (3_000_000, 12)):  # duplicates; full tables of 32 columns; distinct
+        B = from_lengths(np.minimum(blen, ncols), ncols, 17, dtype)
+        lens = rng.integers(0, per_row, nrows)
+        idx = np.concatenate([np.sort(rng.choice(B.shape[0], n, replace=False)) for n in lens])
+        A = dbd_amd.CSR(np.concatenate([[0], np.cumsum(lens)]), idx.astype(np.int32),
+                        rng.standard_normal(idx.size).astype(dtype), (nrows, B.shape[0]))
+        check_product(A, B, what=f"{ncols} columns")
