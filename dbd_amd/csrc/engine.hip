@@ -321,7 +321,7 @@ struct dbd_ctx {
   bool planned = false, symb = false;
   int64_t nr = 0, nb = 0, nwg = 0;
   // per-row and per-nonzero workspace, one allocation (ws), and the kernels' reports (pinned)
-  DevBuf ws, cursor;
+  DevBuf ws, cursor, db_part;
   View P, nnz, Cptr, rows_sym, rows_num, cnt, offs_sym, offs_num, tmp, err, bdesc_s, bdesc_l;
   HostBuf report;
   bool err_dirty = false;  // an error was reported: the device's error word is to be cleared
@@ -1188,7 +1188,7 @@ dbd_status dbd_destroy(dbd_ctx* c) {
   if (!c) return DBD_OK;
   (void)hipStreamSynchronize(c->st);  // a null st is the default stream
   if (c->cst) (void)hipStreamSynchronize(c->cst);
-  for (auto* b : {&c->ws, &c->cursor, &c->band_hist,
+  for (auto* b : {&c->ws, &c->cursor, &c->db_part, &c->band_hist,
                   &c->band_flag, &c->band_tmp, &c->band_slot, &c->band_row, &c->band, &c->hub_meta, &c->hub_scnt,
                   &c->hub_rcnt, &c->hub_tmp, &c->hub_scol, &c->hub_sval, &c->hub_slot, &c->hub_flag,
                   &c->hub_rng})
@@ -1388,24 +1388,55 @@ dbd_status dbd_backward(dbd_ctx* c, const int64_t* d_Cptr, const int32_t* d_Cidx
   if (!c->symb) return set_error(DBD_ERR_STATE, "dbd_backward needs the forward plan (run dbd_symbolic first)");
   hipStream_t s = c->st;
   clear_err(c);
-  c->hub_split = false;  // the long rows' cursors take the records' place
   if (d_dA) launch_fill_bytes0(d_dA, (int64_t)c->vsz * c->A.nnz, s);
   const CatTable& nt = c->tb.num_ct;
   const int64_t* offs = c->offs_num.as<int64_t>();
+  const int64_t n_hub = c->hub.n > 0 ? c->h_num_tot[(size_t)nt.n] - c->h_num_tot[(size_t)nt.n - 1] : 0;
+  // many FP32 products per value of B: summed in parts (into dB itself if there is no room for them)
+  void* db = d_dB;
+  int64_t db_stride = 0;
+  if (const size_t bytes = d_dB ? db_part_bytes(c->o.dtype, c->info.products, c->B.nnz) : 0) {
+    if (c->db_part.ensure(bytes) == DBD_OK) {
+      db = c->db_part.p;
+      db_stride = c->B.nnz;
+      launch_fill_bytes0(db, (int64_t)bytes, s);
+    }
+    clear_error();
+  }
+  const bool in_ranges = n_hub > 0 && hub_backward_ranges(c->o.dtype, c->B.ncols) > 0;
   for (int k = 1; k < nt.n; ++k) {
-    // long and hub rows both take the window backward kernel, which keeps a cursor per A entry;
-    // the two categories lie next to each other in the bins and share one launch, which takes
+    const KernelShape ks = c->tb.num_k[k];
+    if (ks.T == kHubShape && in_ranges) {
+      const int64_t items = n_hub * hub_ranges(c->B.ncols);
+      CHK(hub_reserve(c, n_hub));
+      if (!c->hub_split) {
+        hub_split(c, s);
+        c->hub_split = true;
+      }
+      int64_t* rcnt = c->hub_rcnt.as<int64_t>();
+      launch_hub_gather_counts(c->hub, c->rows_num.as<int32_t>() + c->h_num_tot[(size_t)k], n_hub, c->A, c->B, d_Cptr, 0,
+                               rcnt, s);
+      launch_exclusive_scan(rcnt, rcnt + items + 1, items, c->hub.tmp, s);
+      launch_hub_backward(c->o.dtype, c->hub, n_hub, c->A, c->B, rcnt + items + 1, d_Cidx, d_dC, d_dA, db,
+                          db_stride, c->err.as<int>(), s);
+      continue;
+    }
+    // long and other hub rows both take the window backward kernel, which keeps a cursor per A
+    // entry; the two categories lie next to each other in the bins and share one launch, which takes
     // its rows from the end (the hub rows, the heaviest, first)
-    const bool with_hub = c->tb.num_k[k].T == 0 && k + 1 < nt.n && c->tb.num_k[k + 1].T == kHubShape;
+    const bool with_hub = ks.T == 0 && k + 1 < nt.n && c->tb.num_k[k + 1].T == kHubShape && !in_ranges;
     const int64_t i0 = (int64_t)k * c->nwg, i1 = (int64_t)(k + (with_hub ? 2 : 1)) * c->nwg;
     const int64_t n = c->h_num_tot[(size_t)(k + (with_hub ? 2 : 1))] - c->h_num_tot[(size_t)k];
-    const KernelShape ks = c->tb.num_k[k];
-    if (with_hub) ++k;
+    if (with_hub) {
+      ++k;
+      if (n_hub > 0) c->hub_split = false;  // the hub rows' cursors take their records' place
+    }
     if (n <= 0) continue;
     if (ks.T == 0 || ks.T == kHubShape) CHK(ensure_cursor(c));
     launch_backward(c->o.dtype, ks, c->rows_num.as<int32_t>(), offs + i0, offs + i1, n, 0, c->A, c->B, d_Cptr,
-                    d_Cidx, d_dC, d_dA, d_dB, c->cursor.as<int64_t>(), c->err.as<int>(), s);
+                    d_Cidx, d_dC, d_dA, db, db_stride, c->cursor.as<int64_t>(), c->err.as<int>(), s);
   }
+  if (db_stride > 0) launch_db_sum(db, c->B.nnz, d_dB, s);
   return check_err(c, "backward");
 }
 

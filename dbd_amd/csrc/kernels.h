@@ -196,9 +196,19 @@ void launch_hub_range(int dtype, const HubWork& h, int64_t nh, const Mat& A, con
                       const int32_t* scol, const void* sval, const int64_t* roff, int32_t* Cidx, void* Cval, int* err,
                       hipStream_t s);
 
+// Gradients of the hub rows (their columns per range gathered and scanned as for range, with the
+// caller's Cptr and cbase 0); dA is 0 beforehand. hub_backward_ranges: 0 if B is too wide for it.
+int hub_backward_ranges(int dtype, int64_t ncols);
+void launch_hub_backward(int dtype, const HubWork& h, int64_t n, const Mat& A, const Mat& B, const int64_t* roff,
+                         const int32_t* Cidx, const void* dC, void* dA, void* dB, int64_t db_stride, int* err, hipStream_t s);
+
+// dB's products go to dB + (part) * db_stride: 0 for dB itself, nnz(B) for a workspace of
+// db_part_bytes (0: none is wanted) cleared beforehand, which launch_db_sum adds to dB.
+size_t db_part_bytes(int dtype, int64_t products, int64_t nnzB);
+void launch_db_sum(const void* part, int64_t n, void* dB, hipStream_t s);
 void launch_backward(int dtype, const KernelShape& k, const int32_t* rows, const int64_t* pbeg,
                      const int64_t* pend, int64_t nrows_hint, int grid, const Mat& A, const Mat& B,
-                     const int64_t* Cptr, const int32_t* Cidx, const void* dC, void* dA, void* dB, int64_t* cursor,
+                     const int64_t* Cptr, const int32_t* Cidx, const void* dC, void* dA, void* dB, int64_t db_stride, int64_t* cursor,
                      int* err, hipStream_t s);
 // Is this (T, NT, G) compiled? (the autotuner only proposes compiled shapes)
 bool shape_available(int phase, const KernelShape& k);  // phase 0 symbolic, 1 numeric, 2 backward

@@ -89,6 +89,11 @@ __device__ __forceinline__ T dpp_mov(T old, T x) {
   }
 }
 
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double old, double x) {
+  return __longlong_as_double(dpp_mov<CTRL>(__double_as_longlong(old), __double_as_longlong(x)));
+}
+
 template <typename T>
 __device__ __forceinline__ T read_lane(T x, int lane) {
   if constexpr (sizeof(T) == 4)
@@ -378,7 +383,7 @@ __device__ __forceinline__ void walk_spans(int lane, int len, int64_t start, Spa
         const bool ok = w + u < words && f < T;
         const int o = __builtin_amdgcn_readlane(ex, wu) +
                       __builtin_amdgcn_mbcnt_hi((uint32_t)(mw >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mw, 0));
-        j[u] = ok ? o : 0;
+        j[u] = w + u < words ? o : 0;  // past the last element: its owner again
         at[u] = ok ? l.tb[j[u]] + f : -1;
       }
       body(at, j);
@@ -3652,77 +3657,115 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3))) void k_
 // ------------------------------------------------------------------------------------
 // backward: dA_ik = sum_j dC_ij B_kj ; dB_kj += A_ik dC_ij  (pattern of C from forward)
 // ------------------------------------------------------------------------------------
-// One step of the backward walk: U entries per subgroup (as in gather_step); every product
-// looks its column up in the row's dC table, dA_ik is reduced over the subgroup and
-// A_ik * dC_ij is added into dB.
-template <int T, int G, int U, typename V, int S>
-__device__ __forceinline__ void bwd_step(int lane, int e0, int cnt, int64_t base, const ADesc<V>& d, const int* K,
-                                         const V* H, const int32_t* __restrict__ Bidx, const V* __restrict__ Bval,
-                                         V* __restrict__ dA, V* __restrict__ dB, int& bad) {
-  const int sg = lane / G, lg = lane % G;
-  Step<U, V> st;
-  gather_step<G, U, true, V, S>(st, lane, e0, cnt, d, Bidx, Bval);
-  V acc[U];
-  static_for<U>([&](auto uc) {
-    constexpr int u = decltype(uc)::value;
-    const int e = step_entry<G, S>(e0, u, sg);
-    const int er = min(e0 + u, 63);
-    const int lv = ebcast<G, 4 * S + (u & 3)>(d.len, er);
-    const int pl = e < cnt ? lv : 0;
-    const int64_t pb = ebcast64<G, 4 * S + (u & 3)>(d.b0, er);
-    const V pva = ebcastv<G, 4 * S + (u & 3)>(d.va, er);
-    acc[u] = V(0);
-    if (lg < pl) {
-      const int s = hash_find<T>(K, st.c[u]);
-      if (s < 0) {
-        bad = 1;  // product column absent from C's row: C does not belong to these operands
-      } else {
-        const V gv = H[s];
-        acc[u] = gv * st.bv[u];
-        if (dB) atomicAdd(&dB[pb + lg], pva * gv);
-      }
-    }
-    for (int q = G + lg; q < pl; q += G) {
-      const int64_t p = pb + q;
-      const int s = hash_find<T>(K, Bidx[p]);
-      if (s < 0) {
-        bad = 1;
-        continue;
-      }
-      const V gv = H[s];
-      acc[u] += gv * Bval[p];
-      if (dB) atomicAdd(&dB[p], pva * gv);
-    }
-  });
+// FP32 sums of dB over many products: every add rounds at the size of the sum so far, and thousands
+// of rows meet in the values of a graph's hub rows (R-MAT 16: 400 products a value on average, a
+// relative error of 1.1e-6 to 1.6e-6 with the order of the rows). From kDbPartsFrom products per
+// value on, workgroup b adds into part b % kDbParts of a workspace instead, and the parts are added
+// up in FP64: 2.1e-7 at the same speed. The parts go by XCD as the workgroups do.
+constexpr int kDbParts = 8;
+constexpr int64_t kDbPartsFrom = 32;
+__global__ void k_db_sum(const float* __restrict__ part, int64_t n, float* __restrict__ dB) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    double x = 0.0;
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-#pragma unroll
-    for (int o = G / 2; o > 0; o >>= 1) acc[u] += __shfl_xor(acc[u], o, G);
-    const int e = step_entry<G, S>(e0, u, sg);
-    if (dA && lg == 0 && e < cnt) dA[base + e] = acc[u];
+    for (int q = 0; q < kDbParts; ++q) x += (double)part[q * n + i];
+    dB[i] = (float)((double)dB[i] + x);
   }
 }
+size_t db_part_bytes(int dtype, int64_t products, int64_t nnzB) {
+  return dtype == 0 && nnzB > 0 && products / nnzB >= kDbPartsFrom ? (size_t)kDbParts * 4 * (size_t)nnzB : 0;
+}
+void launch_db_sum(const void* part, int64_t n, void* dB, hipStream_t s) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_db_sum, dim3(fill_grid(n)), dim3(256), 0, s, (const float*)part, n, (float*)dB);
+}
 
-// Per C row: dC_i goes into an LDS table keyed by column; then every A entry of the row walks
-// its B row (descriptor chunks, U gathers in flight per subgroup as in the forward kernels),
-// looks each product column up, reduces dA_ik over its subgroup and adds A_ik * dC_ij into dB.
-template <typename V, int T, int NT, int G>
+// LDS of one wave: the spans' tables, and per rank A's value and the sum of dA's products.
+template <typename V>
+struct BwdLds {
+  SpanLds sp;
+  V va[64];
+  double acc[64];
+};
+
+// The products of one entry per lane (entry ka, `len` elements of its B row from `start` on, A's value
+// va), element-parallel: find(c, g) looks the column up (1: g = dC_ij, 0: not this window's, -1: not in
+// C's row), A_ik * dC_ij is added into dB and dC_ij * B_kj into the entry's sum, which goes to dA
+// atomically (other waves and windows hold the rest of it; dA is 0 beforehand).
+template <int U, typename V, typename F>
+__device__ __forceinline__ void walk_bwd(int lane, int len, int64_t start, int64_t ka, V va, BwdLds<V>& l,
+                                         const int32_t* __restrict__ Bidx, const V* __restrict__ Bval,
+                                         V* __restrict__ dA, V* __restrict__ dB, int& bad, F&& find, int w0 = 0,
+                                         int wstep = U) {
+  int mine = -1;
+  l.acc[lane] = 0.0;
+  walk_spans<U>(lane, len, start, l.sp,
+                [&](int r) {
+                  l.va[r] = va;
+                  mine = r;
+                },
+                [&](const int64_t (&at)[U], const int (&j)[U]) {
+                  int c[U];
+                  V b[U];
+#pragma unroll
+                  for (int u = 0; u < U; ++u) {
+                    const int64_t p = at[u] < 0 ? 0 : at[u];
+                    c[u] = Bidx[p];
+                    b[u] = Bval[p];
+                  }
+#pragma unroll
+                  for (int u = 0; u < U; ++u) {
+                    V g = V(0);
+                    const int ok = at[u] < 0 ? 0 : find(c[u], g);
+                    if (ok < 0) bad = 1;
+                    if (dB && ok > 0) atomicAdd(&dB[at[u]], l.va[j[u]] * g);
+                    // lanes of one entry add into one sum, and LDS takes such adds lane after lane: a
+                    // row of 16 lanes that is all one entry's (owners do not decrease along the lanes)
+                    // adds up by DPP first
+                    double x = ok > 0 ? (double)g * (double)b[u] : 0.0;
+                    if (dpp_mov<0x150>(0, j[u]) == dpp_mov<0x15F>(0, j[u])) {  // row-uniform
+                      x += dpp_mov<0xB1>(x, x);
+                      x += dpp_mov<0x4E>(x, x);
+                      x += dpp_mov<0x141>(x, x);
+                      x += dpp_mov<0x140>(x, x);
+                      if ((lane & 15) == 0) lds_add(&l.acc[j[u]], x);
+                    } else if (ok > 0) {
+                      lds_add(&l.acc[j[u]], x);
+                    }
+                  }
+                },
+                w0, wstep);
+  wave_sync();
+  if (dA && mine >= 0) atomicAdd(&dA[ka], (V)l.acc[mine]);
+  wave_sync();  // the sums are rewritten by the wave's next entries
+}
+
+// Per C row: dC_i goes into an LDS table keyed by column; then the products of the row's entries are
+// walked as in the forward kernels (rows of up to 64 entries by all waves together) and looked up.
+// Bound by the atomics into dB: 266 G/s on neighbouring entries on this GPU (170 G/s in runs of 16).
+// Walked 16 lanes per B row with 64 entries a wave, rows of 2049-4096 columns at R-MAT 16 took
+// 1.98 ms, 0.49 now (an LDS add per product alone: 0.55).
+template <typename V, int T, int NT>
 __global__ __launch_bounds__(wg_of<NT>()) void k_backward_hash(
     const int32_t* __restrict__ rows, const int64_t* __restrict__ pbeg, const int64_t* __restrict__ pend,
     const int64_t* __restrict__ Aptr, const int64_t* __restrict__ bstart, const int32_t* __restrict__ blen,
     const V* __restrict__ Aval, const int32_t* __restrict__ Bidx, const V* __restrict__ Bval,
     const int64_t* __restrict__ Cptr, const int32_t* __restrict__ Cidx, const V* __restrict__ dC,
-    V* __restrict__ dA, V* __restrict__ dB, int* __restrict__ err) {
+    V* __restrict__ dA, V* __restrict__ dB, int64_t db_stride, int* __restrict__ err) {
   constexpr int WG = wg_of<NT>();
   constexpr int GPB = WG / NT;
+  constexpr int NW = NT / 64;
   constexpr int U = 4;
-  static_assert(NT % 64 == 0 && NT % G == 0 && T % NT == 0, "shape");
+  static_assert(NT % 64 == 0 && T % NT == 0, "shape");
   __shared__ int hk[GPB][T];
   __shared__ V hv[GPB][T];
+  __shared__ BwdLds<V> bl[WG / 64];
   __shared__ int sc[GPB][NT > 64 ? NT / 64 : 1];
+  if (dB) dB += (blockIdx.x % kDbParts) * db_stride;
   const int t = threadIdx.x % NT;
   const int g = __builtin_amdgcn_readfirstlane(threadIdx.x / NT);
   const int lane = t & 63, wv = t >> 6;
+  BwdLds<V>& l = bl[__builtin_amdgcn_readfirstlane(threadIdx.x / 64)];
   int* K = hk[g];
   V* H = hv[g];
   const int64_t beg = *pbeg, end = *pend;
@@ -3747,22 +3790,98 @@ __global__ __launch_bounds__(wg_of<NT>()) void k_backward_hash(
     }
     gsync<NT>();
     const int64_t a0 = Aptr[row], a1 = Aptr[row + 1];
-    for (int64_t base = a0 + 64 * wv; base < a1; base += NT) {  // wave-uniform
-      const int cnt = (int)min((int64_t)64, a1 - base);
-      const ADesc<V> d = load_desc<G, true, V>(base, a1, lane, bstart, blen, Aval);
-      if constexpr (G == 16) {  // compile-time steps (DPP broadcast lanes are immediates)
-        if (0 < cnt) bwd_step<T, G, U, V, 0>(lane, 0, cnt, base, d, K, H, Bidx, Bval, dA, dB, bad);
-        if (16 < cnt) bwd_step<T, G, U, V, 1>(lane, 16, cnt, base, d, K, H, Bidx, Bval, dA, dB, bad);
-        if (32 < cnt) bwd_step<T, G, U, V, 2>(lane, 32, cnt, base, d, K, H, Bidx, Bval, dA, dB, bad);
-        if (48 < cnt) bwd_step<T, G, U, V, 3>(lane, 48, cnt, base, d, K, H, Bidx, Bval, dA, dB, bad);
-      } else {
-        for (int e0 = 0; e0 < cnt; e0 += U) bwd_step<T, G, U, V, 0>(lane, e0, cnt, base, d, K, H, Bidx, Bval, dA, dB, bad);
-      }
+    const bool shared = NW > 1 && a1 - a0 <= 64;  // uniform
+    for (int64_t base = a0; base < a1; base += NT) {
+      const int64_t ka = base + (shared ? lane : wv + NW * lane);
+      const bool have = ka < a1;
+      walk_bwd<U>(lane, have ? blen[ka] : 0, have ? bstart[ka] : 0, ka, have ? Aval[ka] : V(0), l, Bidx, Bval, dA, dB, bad,
+                  [&](int c, V& gv) {
+                    const int s = hash_find<T>(K, c);
+                    if (s < 0) return -1;  // C does not belong to these operands
+                    gv = H[s];
+                    return 1;
+                  },
+                  shared ? wv * U : 0, shared ? NW * U : U);
     }
     bad = Group<NT>::reduce(bad, OpMax(), sc[g]);
     if (t == 0 && bad) atomicOr(err, kErrMissingKey);
     gsync<NT>();
   }
+}
+
+// Hub rows in column windows of SR ranges, a workgroup per (row, window): the window's part of C's
+// row (found by the symbolic pass's range counts) lies densely in LDS, and the entries are read as in
+// k_hub_range; the short ones whole in every window, so few windows are wanted (hub_backward_ranges).
+// The 5,900 heaviest rows at R-MAT 16, FP32: 2.96 ms (4.73 with an LDS add per product, whose lanes
+// mostly share an entry; 2.6 of it without any), of which the atomics into dB take 1 ms.
+__device__ __forceinline__ float absent(float) { return __int_as_float(0x7fc0dead); }
+__device__ __forceinline__ double absent(double) { return __longlong_as_double(0x7ff8dead00000000ll); }
+__device__ __forceinline__ bool is_absent(float x) { return __float_as_int(x) == 0x7fc0dead; }
+__device__ __forceinline__ bool is_absent(double x) { return __double_as_longlong(x) == 0x7ff8dead00000000ll; }
+
+template <typename V, int NT, int SR>
+__global__ __launch_bounds__(NT) void k_hub_backward(
+    const HubRow* __restrict__ info, int nrng, int nwin, const V* __restrict__ Aval, const int32_t* __restrict__ Bidx,
+    const V* __restrict__ Bval, const int32_t* __restrict__ band, int64_t nb1, const HubRec* __restrict__ recs,
+    const int64_t* __restrict__ roff, const int32_t* __restrict__ Cidx, const V* __restrict__ dC, V* __restrict__ dA,
+    V* __restrict__ dB, int64_t db_stride, int* __restrict__ err) {
+  constexpr int W = SR * kHubRange;
+  constexpr int NW = NT / 64;
+  constexpr int U = 4;
+  static_assert(W % NT == 0, "shape");
+  __shared__ V dv[W];
+  __shared__ BwdLds<V> bl[NW];
+  if (dB) dB += (blockIdx.x % kDbParts) * db_stride;
+  const int64_t j = blockIdx.x / nwin;
+  const int w = (int)(blockIdx.x - j * nwin);
+  const int64_t* ro = roff + j * nrng;
+  const int64_t o0 = ro[w * SR] - ro[0], o1 = ro[min(w * SR + SR, nrng)] - ro[0];
+  const HubRow row = info[j];
+  if (o1 == o0) return;  // no column, so no product
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int64_t c0 = (int64_t)w * W;
+  int bad = 0;
+#pragma unroll 4
+  for (int q = t; q < W; q += NT) dv[q] = absent(V(0));
+  __syncthreads();
+  for (int64_t m = o0 + t; m < o1; m += NT) {
+    const int64_t o = Cidx[row.out + m] - c0;
+    if (o >= 0 && o < W) dv[o] = dC[row.out + m];
+    else bad = 1;
+  }
+  __syncthreads();
+  const int64_t w0 = c0 >> kBandShift, w1 = min((c0 + W) >> kBandShift, nb1 - 1);
+  for (int e0 = 0; e0 < row.nH; e0 += NT) {  // uniform
+    const int e = e0 + wv + NW * lane;
+    int len = 0;
+    int64_t start = 0, ka = 0;
+    V va = V(0);
+    if (e < row.nH) {
+      const HubRec q = recs[row.a0 + e];
+      const int32_t* bd = band + (int64_t)q.s * nb1;
+      const int s0 = bd[w0];
+      len = bd[w1] - s0;
+      start = q.b0 + s0;
+      ka = row.a0 + q.e;
+      va = Aval[ka];
+    }
+    walk_bwd<U>(lane, len, start, ka, va, bl[wv], Bidx, Bval, dA, dB, bad, [&](int c, V& g) {
+      g = dv[c - c0];
+      return is_absent(g) ? -1 : 1;
+    });
+  }
+  for (int e0 = 0; e0 < row.nL; e0 += NT) {  // uniform
+    const int e = e0 + wv + NW * lane;
+    const HubRec q = e < row.nL ? recs[row.a1 - 1 - e] : HubRec{0, 0, 0};
+    const int64_t ka = row.a0 + q.e;
+    walk_bwd<U>(lane, q.s, q.b0, ka, e < row.nL ? Aval[ka] : V(0), bl[wv], Bidx, Bval, dA, dB, bad, [&](int c, V& g) {
+      const int64_t o = c - c0;
+      if (o < 0 || o >= W) return 0;
+      g = dv[o];
+      return is_absent(g) ? -1 : 1;
+    });
+  }
+  if (__builtin_amdgcn_ballot_w64(bad) && lane == 0) atomicOr(err, kErrMissingKey);
 }
 
 // Long rows: dC's row values are scattered into a dense LDS window (the C row is sorted, so
@@ -3773,10 +3892,11 @@ __global__ __launch_bounds__(NT) void k_backward_long(
     const int64_t* __restrict__ Aptr, const int32_t* __restrict__ Aidx, const V* __restrict__ Aval,
     const int64_t* __restrict__ Bptr, const int32_t* __restrict__ Bidx, const V* __restrict__ Bval,
     const int64_t* __restrict__ Cptr, const int32_t* __restrict__ Cidx, const V* __restrict__ dC,
-    V* __restrict__ dA, V* __restrict__ dB, int64_t* __restrict__ cursor, int* __restrict__ err) {
+    V* __restrict__ dA, V* __restrict__ dB, int64_t db_stride, int64_t* __restrict__ cursor, int* __restrict__ err) {
   __shared__ V dv[W];
   __shared__ int sc[NT / 64];
   __shared__ long long scl[NT / 64];
+  if (dB) dB += (blockIdx.x % kDbParts) * db_stride;
   const int t = threadIdx.x;
   const int64_t beg = *pbeg, end = *pend;
   // rows from the end of the range: callers put the heaviest rows last
@@ -3785,7 +3905,7 @@ __global__ __launch_bounds__(NT) void k_backward_long(
     const int64_t a0 = Aptr[row], a1 = Aptr[row + 1];
     const int64_t c0 = Cptr[row], c1 = Cptr[row + 1];
     for (int64_t ka = a0 + t; ka < a1; ka += NT) {
-      cursor[ka] = Bptr[Aidx[ka]];
+      cursor[2 * ka] = Bptr[Aidx[ka]];
       if (dA) dA[ka] = V(0);
     }
     int64_t cc = c0;
@@ -3809,7 +3929,7 @@ __global__ __launch_bounds__(NT) void k_backward_long(
       for (int64_t ka = a0 + t / G; ka < a1; ka += NT / G) {
         const int k = Aidx[ka];
         const V va = Aval[ka];
-        int64_t p = cursor[ka];
+        int64_t p = cursor[2 * ka];
         const int64_t b1 = Bptr[k + 1];
         V acc = V(0);
         // one step of G, then (a long B row) UL steps at a time with their loads issued together
@@ -3847,7 +3967,7 @@ __global__ __launch_bounds__(NT) void k_backward_long(
 #pragma unroll
         for (int o = G / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, G);
         if ((t % G) == 0) {
-          cursor[ka] = p;
+          cursor[2 * ka] = p;
           if (dA) dA[ka] += acc;
         }
       }
@@ -3860,7 +3980,7 @@ __global__ __launch_bounds__(NT) void k_backward_long(
     }
     // every B entry reached must have been covered by a window
     for (int64_t ka = a0 + t; ka < a1; ka += NT)
-      if (cursor[ka] != Bptr[Aidx[ka] + 1]) bad = 1;
+      if (cursor[2 * ka] != Bptr[Aidx[ka] + 1]) bad = 1;
     bad = Group<NT>::reduce(bad, OpMax(), sc);
     if (t == 0 && bad) atomicOr(err, kErrMissingKey);
     __syncthreads();
@@ -4250,7 +4370,7 @@ void launch_hub_range(int dtype, const HubWork& h, int64_t nh, const Mat& A, con
 template <typename V>
 static void launch_backward_t(const KernelShape& k, const int32_t* rows, const int64_t* pbeg, const int64_t* pend,
                               int64_t nrows_hint, int grid, const Mat& A, const Mat& B, const int64_t* Cptr,
-                              const int32_t* Cidx, const V* dC, V* dA, V* dB, int64_t* cursor, int* err,
+                              const int32_t* Cidx, const V* dC, V* dA, V* dB, int64_t db_stride, int64_t* cursor, int* err,
                               hipStream_t s) {
   const int gpb = symbolic_groups_per_wg(k);
   const V* Av = (const V*)A.val;
@@ -4259,31 +4379,79 @@ static void launch_backward_t(const KernelShape& k, const int32_t* rows, const i
     const dim3 gr(grid_for(nrows_hint, gpb, grid));
     constexpr int W = sizeof(V) == 8 ? kBwdLongW64 : kBwdLongW32;
     hipLaunchKernelGGL((k_backward_long<V, kLongNT, W, kLongG>), gr, dim3(kLongNT), 0, s, rows, pbeg, pend, A.ptr,
-                       A.idx, Av, B.ptr, B.idx, Bv, Cptr, Cidx, dC, dA, dB, cursor, err);
+                       A.idx, Av, B.ptr, B.idx, Bv, Cptr, Cidx, dC, dA, dB, db_stride, cursor, err);
     return;
   }
-#define X(T_, NT_, G_)                                                                                             \
-  if (k.T == T_ && k.NT == NT_ && k.G == G_) {                                                                   \
-    const dim3 gr(grid_for(nrows_hint, gpb, grid, (const void*)k_backward_hash<V, T_, NT_, G_>, wg_of<NT_>())); \
-    hipLaunchKernelGGL((k_backward_hash<V, T_, NT_, G_>), gr, dim3(wg_of<NT_>()), 0, s, rows, pbeg, pend, A.ptr, \
-                       A.bstart, A.blen, Av, B.idx, Bv, Cptr, Cidx, dC, dA, dB, err);                            \
-    return;                                                                                                       \
+#define X(T_, NT_)                                                                                              \
+  if (k.T == T_ && k.NT == NT_) {                                                                               \
+    const dim3 gr(grid_for(nrows_hint, gpb, grid, (const void*)k_backward_hash<V, T_, NT_>, wg_of<NT_>()));     \
+    hipLaunchKernelGGL((k_backward_hash<V, T_, NT_>), gr, dim3(wg_of<NT_>()), 0, s, rows, pbeg, pend, A.ptr,    \
+                       A.bstart, A.blen, Av, B.idx, Bv, Cptr, Cidx, dC, dA, dB, db_stride, err);                           \
+    return;                                                                                                     \
   }
-  DBD_SHAPES(X, 16)
-  DBD_SHAPES(X, 64)
+  X(64, 64)
+  X(128, 64)
+  X(256, 64)
+  X(512, 64)
+  X(1024, 128)
+  X(2048, 256)
+  X(4096, 512)
+  X(8192, 1024)
 #undef X
 }
 
 void launch_backward(int dtype, const KernelShape& k, const int32_t* rows, const int64_t* pbeg, const int64_t* pend,
                      int64_t nrows_hint, int grid, const Mat& A, const Mat& B, const int64_t* Cptr,
-                     const int32_t* Cidx, const void* dC, void* dA, void* dB, int64_t* cursor, int* err,
+                     const int32_t* Cidx, const void* dC, void* dA, void* dB, int64_t db_stride, int64_t* cursor, int* err,
                      hipStream_t s) {
   if (dtype == 1)
     launch_backward_t<double>(k, rows, pbeg, pend, nrows_hint, grid, A, B, Cptr, Cidx, (const double*)dC,
-                              (double*)dA, (double*)dB, cursor, err, s);
+                              (double*)dA, (double*)dB, db_stride, cursor, err, s);
   else
     launch_backward_t<float>(k, rows, pbeg, pend, nrows_hint, grid, A, B, Cptr, Cidx, (const float*)dC,
-                             (float*)dA, (float*)dB, cursor, err, s);
+                             (float*)dA, (float*)dB, db_stride, cursor, err, s);
+}
+
+// Ranges per window of the hub rows' backward kernel for B of this width, 0: the window kernel takes
+// them. Up to kHubWhole ranges one (FP64: two workgroups per CU); beyond, all of a CU's LDS, as long
+// as no more than 16 windows read the short entries (R-MAT 18: 8 windows FP32, 16 FP64).
+int hub_backward_ranges(int dtype, int64_t ncols) {
+  const int nrng = hub_ranges(ncols), big = dtype == 1 ? 2 : 4;
+  return nrng <= kHubWhole ? 1 : (nrng + big - 1) / big <= 16 ? big : 0;
+}
+
+template <typename V, int NT, int SR>
+static void launch_hub_backward_t(const HubWork& h, int64_t n, const Mat& A, const Mat& B, const int64_t* roff,
+                                  const int32_t* Cidx, const V* dC, V* dA, V* dB, int64_t db_stride, int* err,
+                                  hipStream_t s) {
+  const int nrng = hub_ranges(B.ncols), nwin = (nrng + SR - 1) / SR;
+  row_groups(n, nwin, NT, [&](int64_t j0, int64_t nj) {
+    hipLaunchKernelGGL((k_hub_backward<V, NT, SR>), dim3((unsigned)(nj * nwin)), dim3(NT), 0, s, (const HubRow*)h.info + j0,
+                       nrng, nwin, (const V*)A.val, B.idx, (const V*)B.val, B.band, B.nb1, (const HubRec*)h.recs,
+                       roff + j0 * nrng, Cidx, dC, dA, dB, db_stride, err);
+  });
+}
+
+void launch_hub_backward(int dtype, const HubWork& h, int64_t n, const Mat& A, const Mat& B, const int64_t* roff,
+                         const int32_t* Cidx, const void* dC, void* dA, void* dB, int64_t db_stride, int* err,
+                         hipStream_t s) {
+  if (n <= 0) return;
+  const bool one = hub_backward_ranges(dtype, B.ncols) == 1;
+  if (dtype == 1) {
+    if (one)
+      launch_hub_backward_t<double, 512, 1>(h, n, A, B, roff, Cidx, (const double*)dC, (double*)dA, (double*)dB, db_stride,
+                                             err, s);
+    else
+      launch_hub_backward_t<double, 1024, 2>(h, n, A, B, roff, Cidx, (const double*)dC, (double*)dA, (double*)dB, db_stride,
+                                             err, s);
+  } else {
+    if (one)
+      launch_hub_backward_t<float, 512, 1>(h, n, A, B, roff, Cidx, (const float*)dC, (float*)dA, (float*)dB, db_stride, err,
+                                            s);
+    else
+      launch_hub_backward_t<float, 1024, 4>(h, n, A, B, roff, Cidx, (const float*)dC, (float*)dA, (float*)dB, db_stride, err,
+                                            s);
+  }
 }
 
 bool shape_available(int phase, const KernelShape& k) {

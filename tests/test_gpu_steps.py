@@ -142,3 +142,51 @@ def test_several_rows_per_wave(gpu_ok, nrows, dtype):
         A = dbd_amd.CSR(np.concatenate([[0], np.cumsum(lens)]), idx.astype(np.int32),
                         rng.standard_normal(idx.size).astype(dtype), (nrows, B.shape[0]))
         check_product(A, B, what=f"{ncols} columns")
+
+
+# backward of hub rows: in windows of one range (up to 8 ranges), of several (up to 16 windows), and by
+# the window kernel beyond; the forward pass again afterwards (it shares workspace with the latter)
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("ncols", [8193, 65536, 65537, 200_000, 262_145, 600_000])
+def test_backward_hub_rows(gpu_ok, ncols, dtype):
+    import torch
+    from test_gpu_backward import check_grads, run_backward
+    rng = np.random.default_rng(ncols)
+    B = from_lengths(rng.permutation(np.concatenate([rng.integers(0, 64, 1500), rng.integers(64, 700, 400)])), ncols, 18,
+                     dtype)
+    A = from_lengths([1, 1800, 64, 65, 300, 0, 1025, 30], B.shape[0], 19, dtype)
+    check_grads(A, B, *run_backward(A, B))
+    ref = reference(A, B)
+    dA, dB = dbd_amd.DeviceCSR.from_host(A), dbd_amd.DeviceCSR.from_host(B)
+    with dbd_amd.Context(dtype=dtype, stream=torch.cuda.current_stream()) as ctx:
+        ctx.set_operands(dA, dB)
+        ctx.plan()
+        p = torch.empty(A.shape[0] + 1, dtype=torch.int64, device="cuda")
+        n = ctx.symbolic(p)
+        i, v = torch.empty(n, dtype=torch.int32, device="cuda"), torch.empty(n, dtype=dA.val.dtype, device="cuda")
+        ctx.numeric(p, i, v)
+        ctx.backward(p, i, v, torch.empty_like(dA.val), torch.zeros_like(dB.val))
+        i.fill_(-1), v.fill_(0)
+        ctx.numeric(p, i, v)
+        compare(dbd_amd.CSR(p.cpu().numpy(), i.cpu().numpy(), v.cpu().numpy(), (A.shape[0], ncols)), ref, dtype)
+
+
+def test_backward_sums_in_parts_add_to_db(gpu_ok):
+    """Many FP32 products per value of B are summed in parts; dB is added to, as without them, and each
+    value is as near the FP64 gradient as a sum of few parts."""
+    import torch
+    A, B = dbd_amd.gen_rmat(12, 48, seed=20, dtype=np.float32), dbd_amd.gen_er(4096, 600, 5, seed=21, dtype=np.float32)
+    dA, dB = dbd_amd.DeviceCSR.from_host(A), dbd_amd.DeviceCSR.from_host(B)
+    with dbd_amd.Context(dtype="f32", stream=torch.cuda.current_stream()) as ctx:
+        ctx.set_operands(dA, dB)
+        assert ctx.plan()["products"] >= 32 * B.nnz  # the parts are in use
+        p = torch.empty(A.shape[0] + 1, dtype=torch.int64, device="cuda")
+        n = ctx.symbolic(p)
+        i, v = torch.empty(n, dtype=torch.int32, device="cuda"), torch.empty(n, device="cuda")
+        ctx.numeric(p, i, v)
+        gB = torch.full_like(dB.val, 3.0)
+        ctx.backward(p, i, v, None, gB)
+    _, db, miss = oracle.backward(A, B, p.cpu().numpy(), i.cpu().numpy(), v.double().cpu().numpy())
+    assert miss == 0
+    scale = np.abs(db) + 3.0
+    assert np.all(np.abs(gB.cpu().numpy() - 3.0 - db) <= 1e-5 * scale)
