@@ -583,10 +583,12 @@ void attach_band(dbd_ctx* c) {
     c->B.hslot = c->band_slot.as<int32_t>();
     c->B.band = c->band.as<int32_t>();
     c->B.nb1 = c->band_nb1;
+    c->B.band_min = c->band_minlen;
   } else {
     c->B.hslot = nullptr;
     c->B.band = nullptr;
     c->B.nb1 = 0;
+    c->B.band_min = 0;
   }
 }
 

@@ -33,6 +33,7 @@ struct Mat {
   const int32_t* hslot = nullptr;
   const int32_t* band = nullptr;
   int64_t nb1 = 0;
+  int64_t band_min = 0;  // smallest length of a banded row
 };
 
 // One category's kernel shape, chosen by the planner/autotuner.
@@ -87,6 +88,7 @@ void launch_capacity_guard(const int64_t* total, int64_t cap, int64_t* offs, int
 constexpr int kBandShift = 12;
 constexpr int kBandPad = 32;
 int64_t band_count(int64_t ncols);
+constexpr int64_t kRankShort = 64;  // k_numeric_rank takes long rows if the index has all B rows from here on
 // hist[j] (32 int64) = number of B rows with at least 2^j entries.
 void launch_len_hist(const int64_t* Bptr, int64_t nrows, int64_t* hist, hipStream_t s);
 // slot[k] = index of B row k among the rows of at least minlen entries (-1 for the others),

@@ -190,3 +190,29 @@ def test_backward_sums_in_parts_add_to_db(gpu_ok):
     assert miss == 0
     scale = np.abs(db) + 3.0
     assert np.all(np.abs(gB.cpu().numpy() - 3.0 - db) <= 1e-5 * scale)
+
+
+# rows of 1024 columns and more without a hash table: at the edges of the width of a window of values
+# (4096 columns), of a window of ranks (65536) and of four windows of values; rows of up to 64 entries
+# (shared by the waves), up to 512 (one per lane) and more; short, banded and mixed B rows; products of
+# zeros, whose sums must not pass for absent columns
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("ncols, base, width", [
+    (4096, 0, 4096), (4097, 0, 4097), (8192, 2048, 4096), (16384, 0, 16384), (16385, 1, 16384), (65536, 0, 65536),
+    (65537, 0, 65537), (65537, 1, 65536), (200000, 70001, 4095), (200000, 70001, 4097), (200000, 131071, 65537),
+    (400000, 0, 400000)])
+def test_rank_windows(gpu_ok, dtype, ncols, base, width):
+    rng = np.random.default_rng(ncols + width)
+    lens = np.concatenate([rng.integers(0, 64, 1500), rng.integers(64, 300, 1400), rng.integers(2500, 3000, 100)])
+    B = from_lengths(lens, width, 21, dtype)
+    B.idx += base
+    B.val[rng.random(len(B.val)) < 0.05] = -0.0
+    B = dbd_amd.CSR(B.ptr, B.idx, B.val, (len(lens), ncols))
+    groups = [np.arange(1500), np.arange(3000), np.arange(2900, 3000)]  # short, mixed, long B rows
+    rows = []
+    for nA, k in [(1, 2), (2, 2), (4, 2), (12, 1), (30, 1), (63, 1), (64, 0), (64, 1), (65, 0), (65, 1), (150, 0), (200, 0),
+                  (511, 0), (512, 0), (513, 0), (700, 0), (1024, 0)]:
+        rows.append(np.sort(rng.choice(groups[k], nA, replace=False)))
+    A = dbd_amd.CSR(np.concatenate([[0], np.cumsum([len(r) for r in rows])]), np.concatenate(rows).astype(np.int32),
+                    rng.standard_normal(sum(map(len, rows))).astype(dtype), (len(rows), len(lens)))
+    check_product(A, B)
