@@ -102,8 +102,9 @@ struct View {
 
 // ---- category tables -------------------------------------------------------------------
 // Default table. Symbolic key: min(P_i, ncols) (a bound on nnz_i); numeric key: nnz_i.
-// Hash tables are sized so the load stays <= `load`; the one-wave symbolic tables (keys only,
-// 4 bytes a slot, up to 1024 slots) to half of that, which shortens their probe sequences.
+// Hash tables are sized so the load stays <= `load`; the symbolic ones (keys only, 4 bytes a slot) of
+// up to 512 slots to half of that, which shortens their probe sequences. Threads a row of the symbolic
+// tables: symbolic_shape.
 Tables dbd::default_tables(int g_small, int g_big, double load, int top, int64_t hub_min_cols) {
   Tables t;
   t.g_small = g_small;
@@ -113,12 +114,13 @@ Tables dbd::default_tables(int g_small, int g_big, double load, int top, int64_t
   t.hub_min_cols = hub_min_cols;
   const int Ts[] = {64, 128, 256, 512, 1024, 2048, 4096, 8192, 16384};
   const int NTs[] = {64, 64, 64, 64, 128, 256, 512, 1024, 1024};
+  const int SNTs[] = {64, 64, 64, 64, 64, 64, 256, 512, 1024};
   int n = 0;
   t.sym_ct.lim[n] = 0;
   t.sym_k[n++] = {0, 0, 0};
   for (int i = 0; i < 9 && Ts[i] <= 2 * top; ++i) {
-    t.sym_ct.lim[n] = (int64_t)(Ts[i] * (Ts[i] <= 1024 ? load * 0.5 : load));
-    t.sym_k[n++] = {Ts[i], Ts[i] <= 1024 ? 64 : NTs[i], Ts[i] <= 1024 ? g_small : g_big};
+    t.sym_ct.lim[n] = (int64_t)(Ts[i] * (Ts[i] < 1024 ? load * 0.5 : load));
+    t.sym_k[n++] = {Ts[i], SNTs[i], SNTs[i] == 64 ? g_small : g_big};
   }
   t.sym_ct.lim[n] = INT64_MAX;
   t.sym_k[n++] = {0, 1024, 16};  // long rows

@@ -4452,9 +4452,23 @@ int symbolic_groups_per_wg(const KernelShape& k) {
   return k.NT <= 64 ? 256 / k.NT : 1;
 }
 
-void launch_symbolic(const KernelShape& k, const int32_t* rows, const int64_t* pbeg, const int64_t* pend,
+// Threads per row of the symbolic tables from 1024 slots on. Many rows: one wave up to 2048 slots, 256
+// and 512 threads for 4096 and 8192 (waiting on the barriers and clearing the table are most of what a
+// row costs, and more rows share a CU). Few rows, which leave CUs idle: the widest workgroups, whose
+// chains are shorter. Per launch, wide -> narrow: 300,007 rows of 297 products 569 -> 326 us, 99,000
+// rows of 1024-2048 332 -> 254 us, 3,200 of 2048-4096 31 -> 20 us; a few hundred to 2000 rows of each
+// of a web graph 24 -> 65 us in all.
+constexpr int64_t kFewWaveRows = 8192, kFewGroupRows = 1024;
+static KernelShape symbolic_shape(KernelShape k, int64_t nrows) {
+  if (k.NT == 64 && nrows <= kFewWaveRows && (k.T == 1024 || k.T == 2048)) return {k.T, k.T / 8, 64};
+  if (k.NT == k.T / 16 && nrows <= kFewGroupRows && (k.T == 4096 || k.T == 8192)) return {k.T, k.T / 8, k.G};
+  return k;
+}
+
+void launch_symbolic(const KernelShape& table_shape, const int32_t* rows, const int64_t* pbeg, const int64_t* pend,
                      int64_t nrows_hint, int grid, const Mat& A, const Mat& B, int64_t* nnz, int64_t* cursor,
                      int* err, hipStream_t s, const int32_t* hub_slot) {
+  const KernelShape k = symbolic_shape(table_shape, nrows_hint);
   const int gpb = symbolic_groups_per_wg(k);
   if (k.T == 0) {
     const dim3 gr(grid_for(nrows_hint, gpb, grid));
@@ -4486,6 +4500,12 @@ void launch_symbolic(const KernelShape& k, const int32_t* rows, const int64_t* p
   X(16384, 1024, 64)
   X(1024, 64, 16)
   X(1024, 64, 64)
+  X(2048, 64, 16)
+  X(2048, 64, 64)
+  X(4096, 256, 16)
+  X(4096, 256, 64)
+  X(8192, 512, 16)
+  X(8192, 512, 64)
 #undef X
 }
 
@@ -4871,7 +4891,8 @@ bool shape_available(int phase, const KernelShape& k) {
                     (T == 512 && NT == 64) || (T == 1024 && NT == 128) || (T == 2048 && NT == 256) ||
                     (T == 4096 && NT == 512) || (T == 8192 && NT == 1024);
   if (base) return true;
-  return phase == 0 && ((T == 16384 && NT == 1024) || (T == 1024 && NT == 64));
+  return phase == 0 && ((T == 16384 && NT == 1024) || (T == 8192 && NT == 512) || (T == 4096 && NT == 256) ||
+                        (T == 2048 && NT == 64) || (T == 1024 && NT == 64));
 }
 
 }  // namespace dbd

@@ -216,3 +216,26 @@ def test_rank_windows(gpu_ok, dtype, ncols, base, width):
     A = dbd_amd.CSR(np.concatenate([[0], np.cumsum([len(r) for r in rows])]), np.concatenate(rows).astype(np.int32),
                     rng.standard_normal(sum(map(len, rows))).astype(dtype), (len(rows), len(lens)))
     check_product(A, B)
+
+
+# symbolic tables of 1024 slots and more, which take one wave, 256 or 512 threads a row where rows are many:
+# counts of rows on both sides of that, products at the tables' limits
+@pytest.mark.parametrize("few", [True, False])
+def test_symbolic_tables_by_row_count(gpu_ok, few):
+    rng = np.random.default_rng(23)
+    limits, counts = (256, 512, 1024, 2048, 4096), (40, 40, 40, 40) if few else (8193, 8193, 1025, 1025)
+    edge = [m + d for m in limits for d in (-1, 0, 1)]
+    B = from_lengths(rng.permutation(edge + list(rng.integers(1, 4096, 200))), 9001, 24)
+    order = np.argsort(np.diff(B.ptr), kind="stable")
+    lens = np.diff(B.ptr)[order]
+    rows = []
+    for (lo, hi), n in zip(zip(limits, limits[1:]), counts):
+        one = order[(lens >= lo - 1) & (lens <= hi + 1)]  # one entry a row
+        rows += [np.array([b]) for b in one]
+        small = order[lens <= hi // 2]
+        for _ in range(n):  # one or two entries, up to hi products
+            r = rng.choice(one, 1) if len(small) < 3 or rng.random() < 0.5 else rng.choice(small, 2, replace=False)
+            rows.append(np.sort(r))
+    A = dbd_amd.CSR(np.concatenate([[0], np.cumsum([len(r) for r in rows])]), np.concatenate(rows).astype(np.int32),
+                    rng.standard_normal(sum(map(len, rows))), (len(rows), B.shape[0]))
+    check_product(A, B)
