@@ -345,16 +345,18 @@ __device__ __forceinline__ void clear_table(int t, int* K, V* H) {
 // dependent LDS reads per element). l: LDS of this wave's own. With w0 and wstep several waves that
 // hold the same entries share the elements, U words at a time.
 constexpr int kSpanWords = 32;
-struct SpanLds {
-  int64_t tb[64];
+template <typename I>
+struct SpanLdsT {  // I: holds positions in B
+  I tb[64];
   unsigned long long wm[kSpanWords];
 };
+using SpanLds = SpanLdsT<int64_t>;
 struct SpanKeep {  // for a second walk over the same spans: span_words(lane, *this, 0, ..) if T fits kSpanWords
   int T = 0, ex = 0;
   unsigned long long m = 0ull;
 };
-template <int U, typename F>
-__device__ __forceinline__ void span_words(int lane, const SpanKeep& k, int g0, const SpanLds& l, F&& body, int w0,
+template <int U, typename I, typename F>
+__device__ __forceinline__ void span_words(int lane, const SpanKeep& k, int g0, const SpanLdsT<I>& l, F&& body, int w0,
                                            int wstep) {
   const int words = min(kSpanWords, (k.T - g0 + 63) >> 6);
   for (int w = w0; w < words; w += wstep) {
@@ -369,13 +371,13 @@ __device__ __forceinline__ void span_words(int lane, const SpanKeep& k, int g0, 
       const int o = __builtin_amdgcn_readlane(k.ex, wu) +
                     __builtin_amdgcn_mbcnt_hi((uint32_t)(mw >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mw, 0));
       j[u] = w + u < words ? o : 0;  // past the last element: its owner again
-      at[u] = ok ? l.tb[j[u]] + f : -1;
+      at[u] = ok ? l.tb[j[u]] + (I)f : -1;
     }
     body(at, j);
   }
 }
-template <int U, typename X, typename F>
-__device__ __forceinline__ SpanKeep walk_spans(int lane, int len, int64_t start, SpanLds& l, X&& extra, F&& body,
+template <int U, typename I, typename X, typename F>
+__device__ __forceinline__ SpanKeep walk_spans(int lane, int len, int64_t start, SpanLdsT<I>& l, X&& extra, F&& body,
                                                int w0 = 0, int wstep = U) {
   SpanKeep k;
   const uint64_t live = __builtin_amdgcn_ballot_w64(len > 0);
@@ -385,7 +387,7 @@ __device__ __forceinline__ SpanKeep walk_spans(int lane, int len, int64_t start,
   k.T = __builtin_amdgcn_readlane(incl, 63);
   if (len > 0) {
     const int r = __builtin_amdgcn_mbcnt_hi((uint32_t)(live >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)live, 0));
-    l.tb[r] = start - S;
+    l.tb[r] = (I)(start - S);
     extra(r);
   }
   for (int g0 = 0; g0 < k.T; g0 += 64 * kSpanWords) {  // wave-uniform
@@ -2269,13 +2271,15 @@ static_assert(sizeof(HubRow) == 32, "one load");
 // buckets, the short rows are read here.
 //
 // Bound by the latency of an item's chain (row, records, band ends, gathers, stores), so two
-// workgroups share a CU (77 KB of LDS each) and nothing else is kept in LDS: a column is present
+// workgroups share a CU (80 KB of LDS each), with all of its 32 waves as long as positions in B fit 32
+// bits (the walks' tables; with 64 bits half the waves: R-MAT 16 1.80 ms against 1.61, samples of R-MAT
+// 20 rows 4.42 against 3.97), and nothing else is kept in LDS: a column is present
 // when its sum is no longer -0.0, the initial value, which no sum reaches (products of -0.0 are
 // made +0.0 first), so there is no bitmap to OR (127 clocks a wave for 64 neighbouring columns) and
 // a thread emits the sums it reads. The sums are FP64 for FP32 operands too: ds_add_f32 takes 194
 // clocks a wave, ds_add_f64 9 to 21 (and the rounding is better).
-template <typename V, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_hub_range(
+template <typename V, int NT, typename I>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT / 128))) void k_hub_range(
     const HubRow* __restrict__ info, int nrng, const V* __restrict__ Aval, const int32_t* __restrict__ Bidx,
     const V* __restrict__ Bval, const int32_t* __restrict__ band, int64_t nb1, const HubRec* __restrict__ recs,
     const int64_t* __restrict__ soff, const int32_t* __restrict__ scol, const V* __restrict__ sval,
@@ -2285,9 +2289,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   constexpr int PT = kHubRange / NT;  // columns per thread
   static_assert(NT % 64 == 0 && kHubRange % NT == 0 && PT * NW <= 128, "shape");
   __shared__ __align__(16) double dv[kHubRange];
-  __shared__ SpanLds sl[NW];
+  __shared__ SpanLdsT<I> sl[NW];
   __shared__ double tva[NT];
-  __shared__ int wcnt[128];
+  int* wcnt = reinterpret_cast<int*>(tva);  // 128, once the walks are done
   const int64_t item = blockIdx.x;
   const int64_t j = item / nrng;
   const int64_t r0 = roff[item], nexp = roff[item + 1] - r0, rfirst = roff[j * nrng];
@@ -4775,14 +4779,17 @@ template <typename V>
 static void launch_hub_range_t(const HubWork& h, int64_t nh, const Mat& A, const Mat& B, const int64_t* soff,
                                const int32_t* scol, const V* sval, const int64_t* roff, int32_t* Cidx, V* Cval, int* err,
                                hipStream_t s) {
-  constexpr int NT = 512;
   const int nrng = hub_ranges(B.ncols);
-  row_groups(nh, nrng, NT, [&](int64_t j0, int64_t nj) {
-    const int64_t i0 = j0 * nrng;
-    hipLaunchKernelGGL((k_hub_range<V, NT>), dim3((unsigned)(nj * nrng)), dim3(NT), 0, s, (const HubRow*)h.info + j0,
-                       nrng, (const V*)A.val, B.idx, (const V*)B.val, B.band, B.nb1, (const HubRec*)h.recs,
-                       soff ? soff + i0 : nullptr, scol, sval, roff + i0, Cidx, Cval, err);
-  });
+  auto run = [&](auto* kernel, int NT) {
+    row_groups(nh, nrng, NT, [&](int64_t j0, int64_t nj) {
+      const int64_t i0 = j0 * nrng;
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(nj * nrng)), dim3(NT), 0, s, (const HubRow*)h.info + j0, nrng,
+                         (const V*)A.val, B.idx, (const V*)B.val, B.band, B.nb1, (const HubRec*)h.recs,
+                         soff ? soff + i0 : nullptr, scol, sval, roff + i0, Cidx, Cval, err);
+    });
+  };
+  if (B.nnz <= INT32_MAX) run(k_hub_range<V, 1024, int32_t>, 1024);
+  else run(k_hub_range<V, 512, int64_t>, 512);
 }
 
 void launch_hub_range(int dtype, const HubWork& h, int64_t nh, const Mat& A, const Mat& B, const int64_t* soff,
