@@ -4200,6 +4200,92 @@ __global__ __launch_bounds__(wg_of<NT>()) void k_backward_hash(
   }
 }
 
+// Rows of thousands of columns of a B of at most BW columns: C's row as a bitmap with its prefix, which
+// turns a product's column into its rank, and the row's part of dC by rank, VC values at a time (the
+// products are walked once for each). Bound by the atomics into dB, behind the chain bitmap - prefix -
+// value of a lookup: two workgroups of 8 waves share a CU (79 KB of LDS). At R-MAT 16, FP32, the 3,900
+// rows of more than 4096 columns that are no hub rows 1.64 (k_backward_long) -> 0.49 ms, those of
+// 1025-4096 0.60 (k_backward_hash) -> 0.4 ms. any_order: C's row may list its columns in any order, as in
+// the tables (the windows of k_backward_long take them in order only).
+template <typename V, int NT, int VC, int BW>
+__global__ __launch_bounds__(NT) void k_backward_rank(
+    const int32_t* __restrict__ rows, const int64_t* __restrict__ pbeg, const int64_t* __restrict__ pend,
+    const int64_t* __restrict__ Aptr, const int64_t* __restrict__ bstart, const int32_t* __restrict__ blen,
+    const V* __restrict__ Aval, const int32_t* __restrict__ Bidx, const V* __restrict__ Bval,
+    const int64_t* __restrict__ Cptr, const int32_t* __restrict__ Cidx, const V* __restrict__ dC,
+    V* __restrict__ dA, V* __restrict__ dB, int64_t db_stride, int* __restrict__ err, bool any_order) {
+  constexpr int NW = NT / 64, U = 4, NWORD = BW / 64;
+  static_assert(NWORD == 2 * NT, "two words a thread");
+  __shared__ V val[VC];
+  __shared__ unsigned long long bm[NWORD];
+  __shared__ uint16_t pre[NT];
+  __shared__ BwdLds<V> bl[NW];
+  __shared__ int sc[NW];
+  if (dB) dB += (blockIdx.x % kDbParts) * db_stride;
+  uint32_t* bm32 = reinterpret_cast<uint32_t*>(bm);
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int64_t beg = *pbeg, end = *pend;
+  int bad = 0;
+  for (int64_t slot = beg + blockIdx.x; slot < end; slot += gridDim.x) {
+    const int row = rows[slot];
+    const int64_t a0 = Aptr[row], a1 = Aptr[row + 1], c0 = Cptr[row];
+    const int n = (int)min(Cptr[row + 1] - c0, (int64_t)BW);
+    bm[2 * t] = bm[2 * t + 1] = 0ull;
+    __syncthreads();
+    int falls = 0;
+    for (int m = t; m < n; m += NT) {
+      const uint32_t c = (uint32_t)Cidx[c0 + m];
+      if (c < (uint32_t)BW) atomicOr(&bm32[c >> 5], 1u << (c & 31));
+      else bad = 1;
+      if (any_order && m > 0) falls |= (uint32_t)Cidx[c0 + m - 1] >= c;
+    }
+    const bool rises = !__syncthreads_or(falls);  // the columns, so an entry's place is its rank
+    int total;
+    const int mine = __popcll(bm[2 * t]) + __popcll(bm[2 * t + 1]);
+    pre[t] = (uint16_t)Group<NT>::exscan(mine, total, sc);  // below 65536: of all columns one lies behind
+    if (total != n) bad = 1;
+    __syncthreads();
+    // rank of a column, -1 if C's row does not have it
+    auto rank = [&](int col) -> int {
+      const uint32_t c = (uint32_t)col;
+      if (c >= (uint32_t)BW) return -1;
+      const int w = c >> 6;
+      const unsigned long long x = bm[w], y = w & 1 ? bm[w - 1] : 0ull;
+      if (!(x >> (c & 63) & 1ull)) return -1;
+      return (int)pre[w >> 1] + __popcll(y) + __popcll(x & ((1ull << (c & 63)) - 1ull));
+    };
+    const bool shared = a1 - a0 <= 64;  // uniform
+    for (int m0 = 0; m0 < n; m0 += VC) {  // uniform
+      const int nv = min(VC, n - m0);
+      if (rises) {
+        for (int m = t; m < nv; m += NT) val[m] = dC[c0 + m0 + m];
+      } else {
+        for (int m = t; m < n; m += NT) {
+          const uint32_t r = (uint32_t)(rank(Cidx[c0 + m]) - m0);
+          if (r < (uint32_t)nv) val[r] = dC[c0 + m];
+        }
+      }
+      __syncthreads();
+      for (int64_t base = a0; base < a1; base += NT) {
+        const int64_t ka = base + (shared ? lane : wv + NW * lane);
+        const bool have = ka < a1;
+        walk_bwd<U>(lane, have ? blen[ka] : 0, have ? bstart[ka] : 0, ka, have ? Aval[ka] : V(0), bl[wv], Bidx, Bval, dA, dB,
+                    bad,
+                    [&](int c, V& g) {
+                      const int r = rank(c);
+                      if (r < 0) return -1;
+                      if ((uint32_t)(r - m0) >= (uint32_t)nv) return 0;
+                      g = val[r - m0];
+                      return 1;
+                    },
+                    shared ? wv * U : 0, shared ? NW * U : U);
+      }
+      __syncthreads();
+    }
+  }
+  if (__builtin_amdgcn_ballot_w64(bad) && lane == 0) atomicOr(err, kErrMissingKey);
+}
+
 // Hub rows in column windows of SR ranges, a workgroup per (row, window): the window's part of C's
 // row (found by the symbolic pass's range counts) lies densely in LDS, and the entries are read as in
 // k_hub_range; the short ones whole in every window, so few windows are wanted (hub_backward_ranges).
@@ -4810,6 +4896,12 @@ static void launch_backward_t(const KernelShape& k, const int32_t* rows, const i
   const int gpb = symbolic_groups_per_wg(k);
   const V* Av = (const V*)A.val;
   const V* Bv = (const V*)B.val;
+  if ((k.T == 0 || k.T >= kRankSlots) && B.ncols <= kRankBW) {  // figures: k_backward_rank
+    constexpr int VC = 57344 / sizeof(V);
+    hipLaunchKernelGGL((k_backward_rank<V, kRankNT, VC, kRankBW>), dim3(grid_for(nrows_hint, 1, grid)), dim3(kRankNT), 0, s,
+                       rows, pbeg, pend, A.ptr, A.bstart, A.blen, Av, B.idx, Bv, Cptr, Cidx, dC, dA, dB, db_stride, err, k.T != 0);
+    return;
+  }
   if (k.T == 0 || k.T == kHubShape) {  // long and hub rows: windows over the C row
     const dim3 gr(grid_for(nrows_hint, gpb, grid));
     constexpr int W = sizeof(V) == 8 ? kBwdLongW64 : kBwdLongW32;

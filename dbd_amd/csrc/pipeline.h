@@ -39,7 +39,7 @@ struct Tables {
 };
 
 // Symbolic key min(P_i, ncols), numeric key nnz_i; hash tables sized so the load stays <= `load`
-// (one-wave symbolic tables at half of that); G lanes per A entry for one-wave / workgroup tables; the
+// (symbolic tables of up to 512 slots at half of that); G lanes per A entry for one-wave / workgroup tables; the
 // numeric tables stop at `top` slots (4096 or 8192), the symbolic ones at 2 * top. Rows past the
 // last table are long rows; the numeric table ends with the hub category, used when B has at
 // least hub_min_cols columns.

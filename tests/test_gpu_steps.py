@@ -239,3 +239,38 @@ def test_symbolic_tables_by_row_count(gpu_ok, few):
     A = dbd_amd.CSR(np.concatenate([[0], np.cumsum([len(r) for r in rows])]), np.concatenate(rows).astype(np.int32),
                     rng.standard_normal(sum(map(len, rows))), (len(rows), B.shape[0]))
     check_product(A, B)
+
+
+# backward of long rows over up to 65536 columns: C's row by rank, 14336 FP32 or 7168 FP64 values at a time
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("ncols", [65535, 65536, 65537])
+def test_backward_ranked_rows(gpu_ok, ncols, dtype):
+    from test_gpu_backward import check_grads, run_backward
+    rng = np.random.default_rng(ncols)
+    edge = [4096, 4097, 7167, 7168, 7169, 14335, 14336, 14337, 16000]
+    B = from_lengths(np.concatenate([edge, rng.integers(0, 200, 400)]), ncols, 25, dtype)
+    B.idx[B.ptr[8]], B.idx[B.ptr[9] - 1] = 0, ncols - 1  # a row from the first column to the last
+    rows = [np.array([e]) for e in range(9)] + [np.array([0, 2]), np.array([1, 3, 20])]
+    rows += [np.sort(rng.choice(np.arange(9, 409), n, replace=False)) for n in (64, 65, 100)]
+    A = dbd_amd.CSR(np.concatenate([[0], np.cumsum([len(r) for r in rows])]), np.concatenate(rows).astype(np.int32),
+                    rng.standard_normal(sum(map(len, rows))).astype(dtype), (len(rows), B.shape[0]))
+    check_grads(A, B, *run_backward(A, B))
+    # the entries of C's rows in another order, as the hash tables take them
+    import torch
+    dA, dB = dbd_amd.DeviceCSR.from_host(A), dbd_amd.DeviceCSR.from_host(B)
+    with dbd_amd.Context(dtype=dtype, stream=torch.cuda.current_stream()) as ctx:
+        ctx.set_operands(dA, dB)
+        ctx.plan()
+        p = torch.empty(A.shape[0] + 1, dtype=torch.int64, device="cuda")
+        n = ctx.symbolic(p)
+        i, v = torch.empty(n, dtype=torch.int32, device="cuda"), torch.empty(n, dtype=dA.val.dtype, device="cuda")
+        ctx.numeric(p, i, v)
+        h = p.cpu().numpy()
+        hub = h[1:] - h[:-1] > 4096  # hub and wide long rows: in order only
+        order = np.concatenate([np.arange(a, b) if w else np.arange(a, b)[::-1] for a, b, w in zip(h, h[1:], hub)])
+        if ncols > 65536:
+            order = np.arange(n)
+        order = torch.from_numpy(order).cuda()
+        gA, gB = torch.empty_like(dA.val), torch.zeros_like(dB.val)
+        ctx.backward(p, i[order], v[order], gA, gB)
+        check_grads(A, B, h, i.cpu().numpy(), v.cpu().numpy(), gA.cpu().numpy(), gB.cpu().numpy())
