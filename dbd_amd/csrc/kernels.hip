@@ -4495,13 +4495,16 @@ static int resident_blocks(const void* f, int block) {
   return n;
 }
 
-// Grid of a row kernel: `grid` if given (persistent launches), else one group per row. The
+// Grid of a row kernel: for persistent launches (`grid` given) as many workgroups as are resident at
+// once where the kernel is named (two per CU, whatever the shape, left most of a CU idle: a batch of 32
+// 5.69 ms, 5.03 so), else `grid`; otherwise one group per row. The
 // one-wave-per-row kernels (gpb > 1) walk many rows per wave, their row pipeline amortising
 // over them: their grid is capped at what is resident at once, so no second, partly filled
 // round of workgroups follows the first (all workgroups get equal row counts).
 static int grid_for(int64_t nrows, int gpb, int grid, const void* f = nullptr, int block = 256) {
-  if (grid > 0) return grid;
   int64_t g = (nrows + gpb - 1) / gpb;
+  if (grid > 0)
+    return f ? (int)std::max<int64_t>(std::min<int64_t>(g, (int64_t)device_cus() * resident_blocks(f, block)), 1) : grid;
   if (gpb > 1 && f) g = std::min<int64_t>(g, (int64_t)device_cus() * resident_blocks(f, block));
   if (g > 1048576) g = 1048576;
   if (g < 1) g = 1;
@@ -4619,13 +4622,13 @@ static void launch_numeric_t(const KernelShape& k, const int32_t* rows, const in
   const V* Bv = (const V*)B.val;
   const bool is_long = k.T == 0 || k.T == kHubShape;
   if ((is_long || k.T >= kRankSlots) && rank_rows(B)) {
-    const dim3 gr(grid_for(nrows_hint, 1, grid));
-    if (B.band && (is_long || B.ncols > kRankBW))
-      hipLaunchKernelGGL((k_numeric_rank<V, kRankNT, kRankVC, kRankBW, true>), gr, dim3(kRankNT), 0, s, rows, pbeg, pend,
-                         A.ptr, A.bstart, A.blen, Av, B.idx, Bv, Cptr, cbase, Cidx, Cval, err, A.idx, B.hslot, B.band, B.nb1);
-    else
-      hipLaunchKernelGGL((k_numeric_rank<V, kRankNT, kRankVC, kRankBW, false>), gr, dim3(kRankNT), 0, s, rows, pbeg, pend,
-                         A.ptr, A.bstart, A.blen, Av, B.idx, Bv, Cptr, cbase, Cidx, Cval, err, A.idx, B.hslot, B.band, B.nb1);
+    auto run = [&](auto* kernel) {
+      const dim3 gr(grid_for(nrows_hint, 1, grid, (const void*)kernel, kRankNT));
+      hipLaunchKernelGGL(kernel, gr, dim3(kRankNT), 0, s, rows, pbeg, pend, A.ptr, A.bstart, A.blen, Av, B.idx, Bv, Cptr,
+                         cbase, Cidx, Cval, err, A.idx, B.hslot, B.band, B.nb1);
+    };
+    if (B.band && (is_long || B.ncols > kRankBW)) run(k_numeric_rank<V, kRankNT, kRankVC, kRankBW, true>);
+    else run(k_numeric_rank<V, kRankNT, kRankVC, kRankBW, false>);
     return;
   }
   if (is_long) {  // hub rows reach here only when the range kernels cannot run
@@ -4660,7 +4663,7 @@ static void launch_numeric_t(const KernelShape& k, const int32_t* rows, const in
                            A.bstart, A.blen, Av, B.idx, Bv, Cptr, cbase, Cidx, Cval, err);                    \
       }                                                                                                        \
     } else {                                                                                                    \
-      const dim3 gr(grid_for(nrows_hint, gpb, grid));                                                          \
+      const dim3 gr(grid_for(nrows_hint, gpb, grid, (const void*)k_numeric_block<V, T_, NT_, G_>, NT_));       \
       hipLaunchKernelGGL((k_numeric_block<V, T_, NT_, G_>), gr, dim3(NT_), 0, s, rows, pbeg, pend, A.ptr,      \
                          A.bstart, A.blen, Av, B.idx, Bv, Cptr, cbase, Cidx, Cval, err);                      \
     }                                                                                                           \
